@@ -2101,16 +2101,22 @@ __device__ inline double ps_exp(double v) { return exp(v); }
 // terms: PT_COUL | PT_DISP | PT_REP select the pair terms evaluated (all three
 // in one pass, or the charge-independent dispersion and repulsion before the
 // EEQ solve and the Coulomb term after it, into separate partials).
+//
+// split: the 64 steps of a tile are dealt in equal runs to split wavefronts
+// (blocks t * split .. t * split + split - 1), each with partials of its own.
+// A step is a chain of erf, exp, square roots and divisions, about 1.5 us when
+// one wavefront has its SIMD to itself, so a launch of few tiles is bound by
+// that chain and not by throughput (ps_split).
 constexpr int PT_COUL = 1, PT_DISP = 2, PT_REP = 4, PT_ALL = 7;
 template <typename T, int NE>
 __global__ __launch_bounds__(PS_B) void k_pairs_sym(PairArgs a, double* __restrict__ part,
-                                                    const int4* __restrict__ tiles, int terms) {
+                                                    const int4* __restrict__ tiles, int terms, int split) {
     __shared__ double cx[PS_B], cy[PS_B], cz[PS_B];
     __shared__ T cq[PS_B], cal[PS_B], czt[PS_B], csz[PS_B], can[PS_B], crz[PS_B];
     __shared__ T cgw[7][PS_B], cdgw[7][PS_B];
     __shared__ int czem[PS_B];        // Z | element << 8 | metal << 16
     __shared__ double acc[PART_K][PS_B];  // column-side sums of this tile, in FP64 on both paths
-    const int t = blockIdx.x, l = threadIdx.x;
+    const int t = blockIdx.x / split, sub = blockIdx.x % split, l = threadIdx.x;
     // the tile's molecule (atoms a0 .. a0 + n - 1) and its row and column blocks
     int a0 = 0, n = a.n, R, C;
     if (tiles) {
@@ -2166,7 +2172,10 @@ __global__ __launch_bounds__(PS_B) void k_pairs_sym(PairArgs a, double* __restri
     }
     const int jmax = min(PS_B, n - C * PS_B);  // columns present in this tile
     const bool diag = R == C;
-    const int s0 = diag ? 1 : 0, s1 = diag ? (l < 32 ? 32 : 31) : PS_B - 1;
+    // this wavefront's run of the steps 1 .. 32 (diagonal tile) or 0 .. 63
+    const int run = (diag ? PS_B / 2 : PS_B) / split;
+    const int s0 = (diag ? 1 : 0) + sub * run;
+    const int s1 = min(s0 + run - 1, diag ? (l < 32 ? 32 : 31) : PS_B - 1);
     double gx = 0, gy = 0, gz = 0, dcn = 0, ec = 0, ed = 0, er = 0;
     for (int s = s0; s <= s1; ++s) {
         __atomic_signal_fence(__ATOMIC_SEQ_CST);  // keep the LDS updates of consecutive steps in order
@@ -2282,13 +2291,25 @@ __global__ __launch_bounds__(PS_B) void k_pairs_sym(PairArgs a, double* __restri
         if (rep) acc[6][jj] += (double)her;
     }
     __syncthreads();
-    double* pr = part + (size_t)t * 2 * PART_K * PS_B;
+    double* pr = part + (size_t)blockIdx.x * 2 * PART_K * PS_B;
     const double iv[PART_K] = {gx, gy, gz, dcn, ec, ed, er};
 #pragma unroll
     for (int k = 0; k < PART_K; ++k) {
         pr[k * PS_B + l] = iv[k];
         pr[(PART_K + k) * PS_B + l] = acc[k][l];
     }
+}
+
+// Wavefronts per tile: doubled until the launch has 2048 of them (two per
+// SIMD of the chip), at most 8.  Measured, pair kernel and evaluation: 122
+// atoms (3 tiles) 96 -> 14 us and 531 -> 450 us; 216 H2O (66 tiles) 406 -> 326
+// us per dynamics step, 334 us with at most 16 and 360 with 32 (the partial
+// sets cost the reduction more than the shorter chain gains); 512 H2O mixed
+// (300 tiles) 370 -> 331 us, 353 us with 4096 wavefronts.
+static int ps_split(int ntiles) {
+    int split = 1;
+    while (split < 8 && ntiles * split < 2048) split *= 2;
+    return split;
 }
 
 // Per atom a = A 64 + l: the row-side partials of tiles (A, C), C = 0 .. A,
@@ -2303,7 +2324,8 @@ __global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const d
                                                           const double* __restrict__ part2,
                                                           double* __restrict__ g, double* __restrict__ dEdcn,
                                                           double* __restrict__ e_coul, double* __restrict__ e_disp,
-                                                          double* __restrict__ e_rep, const int4* __restrict__ blocks) {
+                                                          double* __restrict__ e_rep, const int4* __restrict__ blocks,
+                                                          int split) {
     __shared__ double qs[4][PART_K][PS_B];
     int A = blockIdx.x, a0 = 0, base = 0;
     if (blocks) {
@@ -2315,13 +2337,15 @@ __global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const d
         nb = (n + PS_B - 1) / PS_B;
     }
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int ntile = nb + 1;  // A + 1 row-side tiles and nb - A column-side tiles
+    const int nset = (nb + 1) * split;  // A + 1 row-side tiles and nb - A column-side tiles, split sets each
     double s[PART_K] = {0, 0, 0, 0, 0, 0, 0};
-    for (int u = w; u < ntile; u += 4) {
+#pragma unroll 2
+    for (int v = w; v < nset; v += 4) {
+        const int u = v / split, sub = v % split;
         const bool rowside = u <= A;
         const int Rr = u - 1;  // column side: tile (R, A), R = u - 1 = A .. nb - 1
         const int t = base + (rowside ? A * (A + 1) / 2 + u : Rr * (Rr + 1) / 2 + A);
-        const size_t o = ((size_t)t * 2 + (rowside ? 0 : 1)) * PART_K * PS_B + l;
+        const size_t o = (((size_t)t * split + sub) * 2 + (rowside ? 0 : 1)) * PART_K * PS_B + l;
         const double* p = part + o;
 #pragma unroll
         for (int k = 0; k < PART_K; ++k) s[k] += p[k * PS_B];
@@ -5352,6 +5376,7 @@ struct DeviceEngine {
     int nslots = 0;
     int pair_cj = 0, pair_nchunk = 0;   // j-chunk size and count of the pair kernel
     int ps_nb = 0;                      // 64-atom blocks of the symmetric pair kernel (single molecules)
+    int ps_split = 1;                   // wavefronts per tile
     int ps_ntiles = 0, ps_nblocks = 0;  // its tiles and 64-atom blocks (0 tiles: batches on the row kernel)
     const int4* ps_tiles = nullptr;     // batches: tiles {a0, n, R, C} of every molecule
     const int4* ps_blocks = nullptr;    // batches: blocks {a0, n, A, first tile of the molecule}
@@ -6257,7 +6282,6 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             E->ps_ntiles = E->ps_nb * (E->ps_nb + 1) / 2;
             E->ps_nblocks = E->ps_nb;
             E->tbox = E->alloc<double>(6 * (size_t)cdiv(n, 256));
-            E->ps_part = E->alloc<double>((size_t)E->ps_ntiles * 2 * PART_K * PS_B);
         } else if (opt.batch_pairs == 0) {
             // batches: the same tiles per molecule, listed {a0, n, R, C}, and the
             // molecules' 64-atom blocks {a0, n, A, first tile} for the reduction
@@ -6273,10 +6297,13 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             E->ps_nblocks = (int)bl.size();
             E->ps_tiles = E->upload(tl);
             E->ps_blocks = E->upload(bl);
-            E->ps_part = E->alloc<double>((size_t)E->ps_ntiles * 2 * PART_K * PS_B);
+        }
+        if (E->ps_ntiles > 0) {
+            E->ps_split = ps_split(E->ps_ntiles);
+            E->ps_part = E->alloc<double>((size_t)E->ps_ntiles * E->ps_split * 2 * PART_K * PS_B);
         }
         E->pair_split = opt.pair_split != 0 && E->ps_ntiles > 0;
-        if (E->pair_split) E->ps_part2 = E->alloc<double>((size_t)E->ps_ntiles * 2 * PART_K * PS_B);
+        if (E->pair_split) E->ps_part2 = E->alloc<double>((size_t)E->ps_ntiles * E->ps_split * 2 * PART_K * PS_B);
         E->e_bond = E->alloc<double>(std::max(E->nbond, 1));
         E->e_ang = E->alloc<double>(std::max(E->nangle, 1));
         E->e_tor = E->alloc<double>(std::max(E->ntors, 1));
@@ -6569,22 +6596,22 @@ static void queue_batch_factor(DeviceEngine* E, hipStream_t s) {
 
 // k_pairs_sym over the engine's tiles for the selected pair terms
 static void queue_pairs_sym(DeviceEngine* E, hipStream_t s, const PairArgs& pa, double* part, int terms) {
-    const dim3 grid(E->ps_ntiles);
+    const dim3 grid(E->ps_ntiles * E->ps_split);
     if (!E->mixed) {
         switch (E->nelem) {
-            case 1: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 1>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            case 2: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 2>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            case 3: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 3>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            case 4: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 4>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            default: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 0>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
+            case 1: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 1>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            case 2: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 2>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            case 3: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 3>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            case 4: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 4>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            default: LAUNCH(KC_PAIRS, (k_pairs_sym<double, 0>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
         }
     } else {
         switch (E->nelem) {
-            case 1: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 1>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            case 2: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 2>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            case 3: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 3>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            case 4: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 4>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
-            default: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 0>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms); break;
+            case 1: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 1>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            case 2: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 2>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            case 3: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 3>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            case 4: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 4>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
+            default: LAUNCH(KC_PAIRS, (k_pairs_sym<float, 0>), grid, dim3(PS_B), s, pa, part, E->ps_tiles, terms, E->ps_split); break;
         }
     }
 }
@@ -6797,7 +6824,7 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
         queue_pairs_sym(E, s, pa, E->ps_part, E->pair_split ? PT_COUL : PT_ALL);
         LAUNCH(KC_PAIRS_AUX, k_pairs_sym_reduce, dim3(E->ps_nblocks), dim3(256), s, n, E->ps_nb, E->ps_part,
                E->pair_split ? (const double*)E->ps_part2 : nullptr,
-               E->gpair, E->dEdcn, E->e_coul, E->e_disp, E->e_rep, E->ps_blocks);
+               E->gpair, E->dEdcn, E->e_coul, E->e_disp, E->e_rep, E->ps_blocks, E->ps_split);
     } else {
         const dim3 grid(cdiv(n, TILE), E->pair_nchunk);
         if (!E->mixed) {

@@ -1,0 +1,76 @@
+"""Energy, gradient and charges at the edges of the kernels' tiles and of the
+rules that choose between their forms, against the CPU oracle.
+
+Atom counts around multiples of the 64-atom pair tiles and of the 64-variable
+EEQ blocks, from the smallest molecules to sizes past the largest split
+launch.  FP64: the oracle's arithmetic in another order, so energies agree to
+1e-9 Eh and gradients and charges to 1e-9 (the repository's parity bound);
+mixed: 1e-6 Eh per atom and 1e-5 Eh/Bohr RMS.
+"""
+import numpy as np
+import pytest
+
+from conftest import BOHR, gpu_available
+from curcuma_amd import GFNFFBatch, GFNFFMethod, Mol
+from curcuma_amd.workloads import alkane, alkane_bundle, glycine_peptide, water_cluster
+
+pytestmark = pytest.mark.gpu
+
+if not gpu_available():
+    pytest.skip("no HIP device", allow_module_level=True)
+
+
+def molecule(kind, size):
+    if kind == "alkane":
+        return alkane(size, sigma=0.02, seed=size)
+    if kind == "peptide":
+        return glycine_peptide(size, sigma=0.02, seed=size)
+    if kind == "bundle":
+        return alkane_bundle(size, 80, seed=size)
+    return water_cluster(size, seed=size)
+
+
+def check(m, Z, xyz, ref, precision):
+    g = m.getGradient()
+    if precision == "fp64":
+        assert abs(m._energy - ref["E"]) < 1e-9 * max(1, len(Z) / 100)
+        assert np.abs(g - ref["grad"]).max() < 1e-9
+        assert np.abs(m.getCharges() - ref["q"]).max() < 1e-9
+    else:
+        assert abs(m._energy - ref["E"]) / len(Z) < 1e-6
+        assert np.sqrt(((g - ref["grad"]) ** 2).mean()) < 1e-5
+
+
+# atoms: water 3 n, alkane 3 n + 2, peptide 7 n + 3, bundle 242 n; one to 66 pair tiles, reduced sizes 2 to 1400
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind,size", [("water", 1), ("alkane", 1), ("water", 21), ("alkane", 20), ("alkane", 21),
+                                       ("alkane", 42), ("alkane", 43), ("peptide", 9), ("peptide", 18), ("peptide", 27),
+                                       ("alkane", 85), ("water", 96), ("water", 97), ("peptide", 41), ("bundle", 3)])
+def test_single_molecule_sizes(kind, size, precision, oracle):
+    Z, xyz = molecule(kind, size)
+    m = GFNFFMethod(precision=precision)
+    assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
+    m.calculateEnergy(True)
+    assert not m.hasError(), m.getErrorMessage()
+    check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_small_batch_sizes(precision, oracle):
+    """Molecules of 5 to 386 atoms, one and several fragments, in one batch whose pair tiles are split."""
+    mols = [molecule(*k) for k in (("alkane", 1), ("alkane", 21), ("water", 2), ("peptide", 9), ("alkane", 42),
+                                   ("peptide", 27), ("water", 43), ("alkane", 128))]
+    off = np.cumsum([0] + [len(z) for z, _ in mols])
+    Z, xyz = np.concatenate([z for z, _ in mols]), np.vstack([x for _, x in mols])
+    b = GFNFFBatch(precision=precision)
+    assert b.setBatch(off, Z, xyz), b.getErrorMessage()
+    b.calculateEnergy(True)
+    assert not b.hasError(), b.getErrorMessage()
+    e, g, q = b.getEnergies(), b.getGradient(), b.getCharges()
+    for k, (z, x) in enumerate(mols):
+        m = GFNFFMethod()
+        assert m.setMolecule(Mol(z, x))
+        ref = oracle.eval(m.params_view(), x * (1.0 / BOHR))
+        m._energy, m._grad = e[k], g[off[k]:off[k + 1]]
+        m.getCharges = lambda: q[off[k]:off[k + 1]]
+        check(m, z, x, ref, precision)
