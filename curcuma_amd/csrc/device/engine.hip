@@ -1107,21 +1107,8 @@ __global__ __launch_bounds__(256) void k_trsv_bwd_sweep(int np, const T* __restr
 // once from HBM (row-major, both triangles stored), which replaces the
 // latency-bound chain of the blocked factorisation.
 // ---------------------------------------------------------------------------
-// Block-Jacobi preconditioner: inverse factors of the 64 x 64 diagonal blocks
-// of R (one workgroup per block; R is left intact).
-// block-Jacobi factors: L^-1 of every diagonal block of the packed matrix
-// (block I at Rp + (I (I + 1) / 2 + I) 64^2)
-__global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ Rp, double* __restrict__ Lj,
-                                                       int* __restrict__ flags) {
-    __shared__ double sL[NB][NB + 1];
-    __shared__ double col[2][NB];
-    __shared__ double rdiag[NB];
-    const size_t I = blockIdx.x;
-    chol_diag_block<double>(NB, 0, Rp + (I * (I + 1) / 2 + I) * NB * NB, Lj + I * NB * NB, flags, sL, col, rdiag,
-                            false);
-}
-
-constexpr int PCG_THREADS = 256;
+constexpr int PCG_THREADS = 512;
+constexpr int PCG_WAVES = PCG_THREADS / 64;
 
 // Sum over the 64 lanes of a wavefront (fixed butterfly; every lane gets it).
 __device__ inline double wave_sum(double v) {
@@ -1156,73 +1143,91 @@ __device__ inline void st_cu(unsigned long long* p, unsigned long long v) {
 // coherent stores are then visible to every device-coherent load).
 __device__ inline void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-// Grid-wide all-reduce of two values per workgroup for a persistent kernel
-// whose G <= 256 workgroups of 256 threads are all resident.  Mailboxes are
-// 128-byte lines of 64-bit words holding MB_EMPTY (a NaN pattern no
-// arithmetic produces) until written: at barrier j workgroup g writes its
-// values to line (g, j mod 3), and thread t of every workgroup polls line
-// (t, j mod 3) and reads producer t's values; every workgroup then adds the
-// G values in the same fixed order, so all hold identical sums.  A writer
-// clears its line (g, (j + 1) mod 3), last written at barrier j - 2, before
-// writing barrier j: having passed barrier j - 1 it has seen every
-// workgroup's barrier j - 1 value, each written after its writer finished
-// reading barrier j - 2, so no reader still needs the cleared line, and the
-// clear completes before the next value is written.  Every wait is bounded
-// (FLAG_SOLVE on a timeout).  Ordering without cache maintenance: the data a
-// workgroup shares is written with device-coherent stores that complete
-// (vmcnt) before its mailbox value is written, and read with device-coherent
-// loads issued after all values were seen, so every shared write before the
-// barrier is visible to every workgroup after it.
+// Grid-wide sum of two values per thread for a persistent kernel whose
+// G <= 256 workgroups are all resident.  Mailboxes are 128-byte lines of
+// 64-bit words holding MB_EMPTY (a NaN pattern no arithmetic produces) until
+// written: at barrier j workgroup g writes its sums to line (g, j mod 4), and
+// thread t of every workgroup polls line (t, j mod 4) and reads producer t's
+// values; every workgroup then adds the G values in the same fixed order, so
+// all hold identical sums.  A writer clears its line (g, (j + 2) mod 4), last
+// written at barrier j - 2, behind its value of barrier j: having passed
+// barrier j - 1 it has seen every workgroup's barrier j - 1 value, each
+// written after its writer finished reading barrier j - 2, so no reader still
+// needs the cleared line; and the clear completes (the wait at the head of
+// barrier j + 1) before the value of barrier j + 1 is written, which every
+// reader has seen before it polls for barrier j + 2.  With three lines the
+// clear has to complete before the value of its own barrier, one more trip to
+// memory in each barrier.  Every wait is bounded (FLAG_SOLVE on a timeout).
+// Ordering without cache maintenance: the data a workgroup shares is written
+// with device-coherent stores that complete (vmcnt) before its mailbox value
+// is written, and read with device-coherent loads issued after all values
+// were seen, so every shared write before the barrier is visible to every
+// workgroup after it.
 constexpr unsigned long long MB_EMPTY = 0x7ff0deadbeef0001ull;
 constexpr int MB_LINE = 16;                  // 64-bit words per 128-byte line
-constexpr int MB_WORDS = 3 * 256 * MB_LINE;  // lines (g, k), k < 3, at (3 g + k) MB_LINE
+constexpr int MB_WORDS = 4 * 256 * MB_LINE;  // lines (g, k), k < 4, at (4 g + k) MB_LINE
 
+// red: 4 PCG_WAVES doubles of LDS, used in halves by the barrier's parity, so
+// that a barrier writes the half that was last read before the barrier ahead
+// of it.
 __device__ bool grid_allreduce2(double v0, double v1, double* sums, unsigned long long* mb, int j, int* flags,
                                 double* red) {
-    __shared__ int bad_s;
-    const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, k = j % 3;
-    if (tid == 0) bad_s = 0;  // every thread read the previous value before the last call's final barrier
+    const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, k = j & 3;
+    double* const rd = red + (j & 1) * 2 * PCG_WAVES;
+    v0 = wave_sum(v0);
+    v1 = wave_sum(v1);
+    if ((tid & 63) == 0) {
+        rd[tid >> 6] = v0;
+        rd[PCG_WAVES + (tid >> 6)] = v1;
+    }
     wait_vm();
     __syncthreads();
     if (tid == 0) {
-        unsigned long long* const own = mb + (3 * g + k) * MB_LINE;
-        unsigned long long* const old = mb + (3 * g + (k + 1) % 3) * MB_LINE;
+        unsigned long long* const own = mb + (4 * g + k) * MB_LINE;
+        unsigned long long* const old = mb + (4 * g + ((k + 2) & 3)) * MB_LINE;
+        double s0 = rd[0], s1 = rd[PCG_WAVES];
+#pragma unroll
+        for (int w = 1; w < PCG_WAVES; ++w) {
+            s0 += rd[w];
+            s1 += rd[PCG_WAVES + w];
+        }
+        st_cu(own, __double_as_longlong(s0));
+        st_cu(own + 1, __double_as_longlong(s1));
         st_cu(old, MB_EMPTY);
         st_cu(old + 1, MB_EMPTY);
-        wait_vm();
-        st_cu(own, __double_as_longlong(v0));
-        st_cu(own + 1, __double_as_longlong(v1));
     }
     double u0 = 0.0, u1 = 0.0;
+    int bad = 0;
     if (tid < G) {
-        const unsigned long long* const in = mb + (3 * tid + k) * MB_LINE;
+        const unsigned long long* const in = mb + (4 * tid + k) * MB_LINE;
         unsigned long long a0 = MB_EMPTY, a1 = MB_EMPTY;
         for (int it = 0;; ++it) {
             a0 = ld_cu(in);
             a1 = ld_cu(in + 1);
             if (a0 != MB_EMPTY && a1 != MB_EMPTY) break;
-            if (it > SPIN_MAX || (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_SOLVE)) {
-                bad_s = 1;
+            if (it > SPIN_MAX ||
+                ((it & 63) == 63 &&
+                 (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_SOLVE))) {
+                bad = 1;
                 atomicOr(flags, FLAG_SOLVE);
                 break;
             }
-            __builtin_amdgcn_s_sleep(1);
         }
         u0 = __longlong_as_double(a0);
         u1 = __longlong_as_double(a1);
     }
-    u0 = wave_sum(u0);
-    u1 = wave_sum(u1);
-    __syncthreads();
-    if ((tid & 63) == 0) {
-        red[tid >> 6] = u0;
-        red[4 + (tid >> 6)] = u1;
+    __syncthreads();  // thread 0 has read this workgroup's partial sums
+    if (tid < 256) {
+        u0 = wave_sum(u0);
+        u1 = wave_sum(u1);
+        if ((tid & 63) == 0) {
+            rd[tid >> 6] = u0;
+            rd[PCG_WAVES + (tid >> 6)] = u1;
+        }
     }
-    __syncthreads();
-    sums[0] = (red[0] + red[1]) + (red[2] + red[3]);
-    sums[1] = (red[4] + red[5]) + (red[6] + red[7]);
-    const bool ok = bad_s == 0;
-    __syncthreads();
+    const bool ok = __syncthreads_or(bad) == 0;
+    sums[0] = (rd[0] + rd[1]) + (rd[2] + rd[3]);
+    sums[1] = (rd[PCG_WAVES] + rd[PCG_WAVES + 1]) + (rd[PCG_WAVES + 2] + rd[PCG_WAVES + 3]);
     return ok;
 }
 
@@ -1271,10 +1276,54 @@ __device__ void bjacobi_apply(const double* __restrict__ Li, const double* rb, d
 // and read with device-coherent accesses (ld_c, st_c); an owner keeps its
 // rows of x and r, and the Linv of a single owned block, in LDS for the
 // whole solve and writes x at the end.
+//
+// RES: every wavefront has at most one block (np <= 4032 with 2048
+// wavefronts), which it loads into registers once and keeps there, with its
+// slices of p, for the whole solve: an iteration then reads only z and the
+// partials.  Otherwise the matrix streams through once per iteration; eight
+// wavefronts per workgroup (two per SIMD) let one load while the other
+// multiplies.
+//
+// Preconditioner.  M = D, the diagonal blocks of R, cuts a fragment of more
+// than 64 variables into pieces, and every variable of the fragment carries
+// the terms of the same last atom l, R = A - u 1^T - 1 u^T + A_ll 1 1^T: the
+// rank-one part couples all pieces.  Over such "split" fragments f
+// (SM) M = D + sum_f A_ll(f) 1_f 1_f^T with D the diagonal blocks of A
+// itself within the fragment (k_bjacobi_setup), and by Sherman-Morrison
+//   z = y - sum_f sigma_f s_f w_f,  y = D^-1 r, w_f = D^-1 1_f,
+//   s_f = 1_f . y,  sigma_f = 1 / (1 / A_ll(f) + 1_f . w_f),
+//   r.z = r.y - sum_f sigma_f s_f^2.
+// Owners publish y and their pieces' parts of s_f; after the barrier every
+// workgroup forms the same sigma_f s_f, and z on the fly.  Together with the
+// order of the variables along the bond graph (reduced_order): 80 chains of
+// C80H162 (mixed) 467 -> 76 iterations and 159 -> 27 ms, C300H602 148 -> 38,
+// H-(Gly)200-OH 97 -> 39, C40H82 39 -> 15.
 constexpr int PCG_MAXB = 8;
 constexpr double PCG_TOL_FP64 = 1e-13;   // default |r| / |b| of the FP64 path
 constexpr double PCG_TOL_MIXED = 1e-10;  // default of the mixed path (EEQ energy is variational in q)
 constexpr int PCG_MAXIT = 1000;
+constexpr int SM_MAXF = 512;        // split fragments and 64-variable blocks of the Sherman-Morrison form
+constexpr int SM_MAXB = 1024;       // (beyond: plain diagonal blocks)
+constexpr int SM_MAXP = SM_MAXB + SM_MAXF;  // pieces: one per block and one more per fragment boundary inside a block
+
+struct PcgArgs {
+    int np, maxit;
+    double tol2;
+    const double *Rp, *Lj, *b;
+    double *x, *z, *pb, *part;
+    unsigned long long* mb;
+    int *iters, *flags;
+    // split fragments
+    int nsf;
+    const int* rowf;     // [np] 2 f + slot of the row's piece in its block, or -1
+    const int* poff;     // [nsf + 1] pieces of a fragment in pidx
+    const int* pidx;     // a piece's place 2 block + slot
+    const double* w;     // [np] D^-1 1_f (k_bjacobi_setup)
+    const double* w1;    // [2 nbk] 1_f . w of each piece
+    const double* all;   // [nsf] A_ll of the fragment's last atom
+    const int* smon;     // [nbk] 0: the block's A was not positive definite and its R was factored instead
+    double* sp;          // [2 nbk] parts of s_f
+};
 
 // Sum of 8 per-lane values v[k] over the 8 lanes that differ in lane bits
 // s, s + 1, s + 2 (recursive halving): lane l ends with the total of
@@ -1297,29 +1346,54 @@ __device__ inline double tr_reduce8(const double (&v)[8], int l) {
     return (h0 ? a2[1] : a2[0]) + __shfl_xor(h0 ? a2[0] : a2[1], 1 << S);
 }
 
-__global__ __launch_bounds__(256) void k_eeq_pcg(int np, const double* __restrict__ Rp,
-                                                 const double* __restrict__ Lj, const double* __restrict__ b,
-                                                 double* __restrict__ x, double* __restrict__ z,
-                                                 double* __restrict__ pb,
-                                                 double* __restrict__ part, unsigned long long* __restrict__ mb,
-                                                 int* __restrict__ iters, double tol2, int maxit,
-                                                 int* __restrict__ flags) {
-    __shared__ double red[256];
+// sigma_f s_f of every split fragment into sfs, from the published parts;
+// returns sum_f sigma_f s_f^2 (the same in every workgroup).  sig: sigma_f.
+__device__ double sm_gather(const PcgArgs& a, int npc, double* sfs, const double* sig, double* pbuf, double* red) {
+    const int tid = threadIdx.x, l8 = tid & 7;
+    for (int k = tid; k < npc; k += PCG_THREADS) pbuf[k] = ld_c(a.sp + a.pidx[k]);
+    __syncthreads();
+    double e = 0.0;
+    for (int f0 = 0; f0 < a.nsf; f0 += PCG_THREADS / 8) {
+        const int f = f0 + (tid >> 3);
+        double s = 0.0;
+        if (f < a.nsf)
+            for (int k = a.poff[f] + l8; k < a.poff[f + 1]; k += 8) s += pbuf[k];
+        s += __shfl_xor(s, 1);
+        s += __shfl_xor(s, 2);
+        s += __shfl_xor(s, 4);
+        if (f < a.nsf && l8 == 0) {
+            sfs[f] = sig[f] * s;
+            e += sig[f] * s * s;
+        }
+    }
+    e = wave_sum(e);
+    if ((tid & 63) == 0) red[tid >> 6] = e;
+    __syncthreads();
+    double t = red[0];
+#pragma unroll
+    for (int w = 1; w < PCG_WAVES; ++w) t += red[w];
+    return t;
+}
+
+template <bool RES, bool SM>
+__global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
+    __shared__ double red[4 * PCG_WAVES], red2[2][PCG_WAVES];
     __shared__ double pown[PCG_MAXB][NB];
-    __shared__ double qs[4][NB];
+    __shared__ double qs[PCG_WAVES][NB];
     __shared__ double rb[NB], wb[NB], zb[NB];
     __shared__ double xo[PCG_MAXB][NB], ro[PCG_MAXB][NB];  // owned rows of x and r, resident for the solve
     __shared__ double Lc[NB * NB];                          // Linv of the owned block when there is one
-    __shared__ __align__(16) double pw[4][2][NB];            // per wavefront: p of the block's rows and columns
+    __shared__ __align__(16) double pw[PCG_WAVES][2][NB];    // per wavefront: p of the block's rows and columns
+    __shared__ double sfs[SM ? SM_MAXF : 1], sig[SM ? SM_MAXF : 1], pbuf[SM ? SM_MAXP : 1];
     // a diagonal block that is not positive definite (FLAG_CHOL, set before
     // this launch, so every workgroup reads the same value) leaves the solve to
     // the LU fallback that follows
-    if (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) return;
-    const int G = gridDim.x, g = blockIdx.x, nbk = np / NB;
+    if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) return;
+    const int np = a.np, G = gridDim.x, g = blockIdx.x, nbk = np / NB;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int nown = (nbk - g + G - 1) / G;
     // this wavefront's blocks of the packed order: [t0, t1)
-    const long T = (long)nbk * (nbk + 1) / 2, W = 4L * G, gw = 4L * g + wv;
+    const long T = (long)nbk * (nbk + 1) / 2, W = (long)PCG_WAVES * G, gw = (long)PCG_WAVES * g + wv;
     const int t0 = (int)(T * gw / W), t1 = (int)(T * (gw + 1) / W);
     int I0 = (int)((sqrt(8.0 * t0 + 1.0) - 1.0) * 0.5);
     while ((long)(I0 + 1) * (I0 + 2) / 2 <= t0) ++I0;
@@ -1328,66 +1402,105 @@ __global__ __launch_bounds__(256) void k_eeq_pcg(int np, const double* __restric
     // lane (rg, cg) holds rows 8 rg + i (i < 8) and columns 2 cg + (k & 1) + 16 (k >> 1) (k < 8) of a
     // block: every 16-byte load instruction reads whole 128-byte row segments
     const int rg = l >> 3, cg = l & 7;
+    double rv[8][8];
+    auto load_block = [&](int t) {
+        const double2* Rb = reinterpret_cast<const double2*>(a.Rp + (size_t)t * NB * NB);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const double2 v2 = Rb[((8 * rg + i) * NB + 16 * j + 2 * cg) / 2];
+                rv[i][2 * j] = v2.x;
+                rv[i][2 * j + 1] = v2.y;
+            }
+    };
+    double pir = 0.0, pjr = 0.0;  // RES: p of row I0 64 + l and column J0 64 + l
+    if (RES && t1 > t0) load_block(t0);
     const bool lcache = nown == 1;
     if (lcache)
-        for (int e = tid; e < NB * NB; e += 256) Lc[e] = Lj[(size_t)g * NB * NB + e];
+        for (int e = tid; e < NB * NB; e += PCG_THREADS) Lc[e] = a.Lj[(size_t)g * NB * NB + e];
+    const int npc = SM ? a.poff[a.nsf] : 0;
+    if (SM)
+        for (int f = tid; f < a.nsf; f += PCG_THREADS) {
+            double s = 1.0 / a.all[f];
+            for (int k = a.poff[f]; k < a.poff[f + 1]; ++k) s += a.w1[a.pidx[k]];
+            sig[f] = 1.0 / s;
+        }
+    // z of a row: y, less the fragment's rank-one part
+    auto zrow = [&](int row) {
+        double v = ld_c(a.z + row);
+        if (SM) {
+            const int rf = a.rowf[row];
+            if (rf >= 0) v -= sfs[rf >> 1] * a.w[row];
+        }
+        return v;
+    };
+    // owners publish y = D^-1 r of a block (rb -> z) and its pieces' parts of s_f
+    auto publish = [&](int kb, double& lrz, double& lrr) {
+        bjacobi_apply(lcache ? Lc : a.Lj + (size_t)kb * NB * NB, rb, wb, zb);
+        if (tid < NB) {
+            const double y = zb[tid], r = rb[tid];
+            st_c(a.z + kb * NB + tid, y);
+            lrz += r * y;
+            lrr += r * r;
+            if (SM) {
+                const int rf = a.smon[kb] ? a.rowf[kb * NB + tid] : -1;
+                const double s0 = wave_sum(rf >= 0 && !(rf & 1) ? y : 0.0), s1 = wave_sum(rf >= 0 && (rf & 1) ? y : 0.0);
+                if (tid < 2) st_c(a.sp + 2 * kb + tid, tid ? s1 : s0);
+            }
+        }
+    };
     // init: x = 0, r = b, z = M^-1 b; partials r.z and b.b
     double lrz = 0.0, lbb = 0.0;
     for (int o = 0; o < nown; ++o) {
         const int kb = g + o * G;
         if (tid < NB) {
-            const double bv = b[kb * NB + tid];
+            const double bv = a.b[kb * NB + tid];
             rb[tid] = bv;
             xo[o][tid] = 0.0;
             ro[o][tid] = bv;
         }
         __syncthreads();
-        bjacobi_apply(lcache ? Lc : Lj + (size_t)kb * NB * NB, rb, wb, zb);
-        if (tid < NB) {
-            st_c(z + kb * NB + tid, zb[tid]);
-            lrz += rb[tid] * zb[tid];
-            lbb += rb[tid] * rb[tid];
-        }
+        publish(kb, lrz, lbb);
     }
     int nbar = 0;  // barriers passed
     double sums[2];
-    const double s_rz = wg_sum256(lrz, red), s_bb = wg_sum256(lbb, red);
-    if (!grid_allreduce2(s_rz, s_bb, sums, mb, nbar++, flags, red)) return;
+    if (!grid_allreduce2(lrz, lbb, sums, a.mb, nbar++, a.flags, red)) return;
     double rz = sums[0];
     const double bb = sums[1];
+    if (SM) rz -= sm_gather(a, npc, sfs, sig, pbuf, red2[0]);
     double beta = 0.0;
     int it = 0;
     bool done = !(bb > 0.0);
-    for (; !done && it < maxit; ++it) {
-        const double* pprev = pb + (size_t)((it + 1) & 1) * np;
-        double* pcur = pb + (size_t)(it & 1) * np;
+    for (; !done && it < a.maxit; ++it) {
+        const double* pprev = a.pb + (size_t)((it + 1) & 1) * np;
+        double* pcur = a.pb + (size_t)(it & 1) * np;
         // (1) owners: p rows; every wavefront: its blocks' products
         for (int o = 0; o < nown; ++o) {
             if (tid < NB) {
                 const int row = (g + o * G) * NB + tid;
-                const double pc = (it == 0) ? 0.0 : ld_c(pprev + row);
-                const double pv = ld_c(z + row) + beta * pc;
+                const double pc = (it == 0) ? 0.0 : pown[o][tid];
+                const double pv = zrow(row) + beta * pc;
                 pown[o][tid] = pv;
-                st_c(pcur + row, pv);
+                if (!RES) st_c(pcur + row, pv);
             }
         }
         double lpq = 0.0;
         int I = I0, J = J0;
         for (int t = t0; t < t1; ++t) {
-            const double2* Rb = reinterpret_cast<const double2*>(Rp + (size_t)t * NB * NB);
-            double rv[8][8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const double2 v2 = Rb[((8 * rg + i) * NB + 16 * j + 2 * cg) / 2];
-                    rv[i][2 * j] = v2.x;
-                    rv[i][2 * j + 1] = v2.y;
-                }
-            const double pcj = (it == 0) ? 0.0 : ld_c(pprev + J * NB + l);
-            const double pjl = ld_c(z + J * NB + l) + beta * pcj;  // p of column J * 64 + l
-            const double pci = (it == 0) ? 0.0 : ld_c(pprev + I * NB + l);
-            const double pil = ld_c(z + I * NB + l) + beta * pci;  // p of row I * 64 + l
+            if (!RES) load_block(t);
+            double pil, pjl;  // p of row I * 64 + l and column J * 64 + l
+            if (RES) {
+                pjr = zrow(J * NB + l) + beta * pjr;
+                pir = zrow(I * NB + l) + beta * pir;
+                pjl = pjr;
+                pil = pir;
+            } else {
+                const double pcj = (it == 0) ? 0.0 : ld_c(pprev + J * NB + l);
+                pjl = zrow(J * NB + l) + beta * pcj;
+                const double pci = (it == 0) ? 0.0 : ld_c(pprev + I * NB + l);
+                pil = zrow(I * NB + l) + beta * pci;
+            }
             pw[wv][0][l] = pil;
             pw[wv][1][l] = pjl;
             __builtin_amdgcn_wave_barrier();
@@ -1403,21 +1516,21 @@ __global__ __launch_bounds__(256) void k_eeq_pcg(int np, const double* __restric
             double rs8[8], cs8[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                double a = 0.0, c = 0.0;
+                double ra = 0.0, c = 0.0;
 #pragma unroll
                 for (int m = 0; m < 8; ++m) {
-                    a += rv[k][m] * pj[m];
+                    ra += rv[k][m] * pj[m];
                     c += rv[m][k] * pi[m];
                 }
-                rs8[k] = a;
+                rs8[k] = ra;
                 cs8[k] = c;
             }
             const double rs = tr_reduce8<0>(rs8, l);  // row 8 rg + cg = l
-            st_c(part + ((size_t)I * nbk + J) * NB + l, rs);
+            st_c(a.part + ((size_t)I * nbk + J) * NB + l, rs);
             lpq += pil * rs;
             if (I != J) {
                 const double cs = tr_reduce8<3>(cs8, l);  // column cend
-                st_c(part + ((size_t)J * nbk + I) * NB + cend, cs);
+                st_c(a.part + ((size_t)J * nbk + I) * NB + cend, cs);
                 lpq += pjc * cs;
             }
             if (++J > I) {
@@ -1425,8 +1538,7 @@ __global__ __launch_bounds__(256) void k_eeq_pcg(int np, const double* __restric
                 J = 0;
             }
         }
-        const double s_pq = wg_sum256(lpq, red);
-        if (!grid_allreduce2(s_pq, 0.0, sums, mb, nbar++, flags, red)) return;
+        if (!grid_allreduce2(lpq, 0.0, sums, a.mb, nbar++, a.flags, red)) return;
         const double pq = sums[0];
         const double alpha = rz / pq;
         // (2) owners: q rows from the partials (Y order), x, r, z and the
@@ -1435,45 +1547,43 @@ __global__ __launch_bounds__(256) void k_eeq_pcg(int np, const double* __restric
         for (int o = 0; o < nown; ++o) {
             const int kb = g + o * G;
             {
-                // thread (row l, part wv) adds Y = wv, wv + 4, ... in batches of 32 loads
-                const double* pr = part + (size_t)kb * nbk * NB + l;
+                // thread (row l, part wv) adds Y = wv, wv + PCG_WAVES, ... in batches of 16 loads
+                const double* pr = a.part + (size_t)kb * nbk * NB + l;
                 double acc = 0.0;
-                for (int y0 = wv; y0 < nbk; y0 += 128) {
-                    double t32[32];
+                for (int y0 = wv; y0 < nbk; y0 += 16 * PCG_WAVES) {
+                    double t16[16];
 #pragma unroll
-                    for (int u = 0; u < 32; ++u) t32[u] = ld_c(pr + (size_t)min(y0 + 4 * u, nbk - 1) * NB);
+                    for (int u = 0; u < 16; ++u) t16[u] = ld_c(pr + (size_t)min(y0 + PCG_WAVES * u, nbk - 1) * NB);
 #pragma unroll
-                    for (int u = 0; u < 32; ++u) acc += (y0 + 4 * u < nbk) ? t32[u] : 0.0;
+                    for (int u = 0; u < 16; ++u) acc += (y0 + PCG_WAVES * u < nbk) ? t16[u] : 0.0;
                 }
                 qs[wv][l] = acc;
             }
             __syncthreads();
             if (tid < NB) {
-                const double qv = (qs[0][tid] + qs[1][tid]) + (qs[2][tid] + qs[3][tid]);
+                double qv = qs[0][tid];
+#pragma unroll
+                for (int w = 1; w < PCG_WAVES; ++w) qv += qs[w][tid];
                 xo[o][tid] += alpha * pown[o][tid];
-                const double rv = ro[o][tid] - alpha * qv;
-                ro[o][tid] = rv;
-                rb[tid] = rv;
+                const double rn = ro[o][tid] - alpha * qv;
+                ro[o][tid] = rn;
+                rb[tid] = rn;
             }
             __syncthreads();
-            bjacobi_apply(lcache ? Lc : Lj + (size_t)kb * NB * NB, rb, wb, zb);
-            if (tid < NB) {
-                st_c(z + kb * NB + tid, zb[tid]);
-                lrz2 += rb[tid] * zb[tid];
-                lrr += rb[tid] * rb[tid];
-            }
+            publish(kb, lrz2, lrr);
         }
-        const double s_rz2 = wg_sum256(lrz2, red), s_rr = wg_sum256(lrr, red);
-        if (!grid_allreduce2(s_rz2, s_rr, sums, mb, nbar++, flags, red)) return;
-        const double rz2 = sums[0], rr = sums[1];
+        if (!grid_allreduce2(lrz2, lrr, sums, a.mb, nbar++, a.flags, red)) return;
+        const double rr = sums[1];
+        double rz2 = sums[0];
+        done = rr <= a.tol2 * bb;
+        if (SM && !done) rz2 -= sm_gather(a, npc, sfs, sig, pbuf, red2[it & 1]);
         beta = rz2 / rz;
         rz = rz2;
-        done = rr <= tol2 * bb;
     }
     for (int o = 0; o < nown; ++o)
-        if (tid < NB) x[(g + o * G) * NB + tid] = xo[o][tid];
-    if (g == 0 && tid == 0) iters[0] = it;
-    if (!done && g == 0 && tid == 0) atomicOr(flags, FLAG_SOLVE);
+        if (tid < NB) a.x[(g + o * G) * NB + tid] = xo[o][tid];
+    if (g == 0 && tid == 0) a.iters[0] = it;
+    if (!done && g == 0 && tid == 0) atomicOr(a.flags, FLAG_SOLVE);
 }
 
 // ---------------------------------------------------------------------------
@@ -5157,6 +5267,104 @@ __global__ __launch_bounds__(256) void k_solv_red_add(int nr, int np, const int*
     }
 }
 
+// Preconditioner of the iterative EEQ solve: the inverse factors of the
+// 64 x 64 diagonal blocks D of k_eeq_pcg (one workgroup per block; R is left
+// intact).  Rows of split fragments (rowf >= 0) take A of their own fragment
+// instead of R and nothing of the others; such a block also gets w = D^-1 1_f
+// and 1_f . w for its pieces.  A need not be positive definite where R is: a
+// block whose D fails is factored as it stands in R and takes no part in the
+// rank-one terms (smon 0).
+__global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ Rp, double* __restrict__ Lj,
+                                                       int* __restrict__ flags, int nsf, PcgArgs pa,
+                                                       const int* __restrict__ ra, const int* __restrict__ rl,
+                                                       const double* __restrict__ x, const double* __restrict__ alp,
+                                                       const double* __restrict__ diag, int solv, SolvArgs sv,
+                                                       double* __restrict__ w, double* __restrict__ w1,
+                                                       double* __restrict__ all, int* __restrict__ smon) {
+    __shared__ double sL[NB][NB + 1];
+    __shared__ double col[2][NB];
+    __shared__ double rdiag[NB];
+    __shared__ int bad;
+    const size_t I = blockIdx.x;
+    double* const Rb = Rp + (I * (I + 1) / 2 + I) * NB * NB;
+    double* const Li = Lj + I * NB * NB;
+    const int tid = threadIdx.x;
+    bool any = false;
+    if (nsf > 0) any = __syncthreads_or(pa.rowf[I * NB + (tid & 63)] >= 0);
+    if (!any) {  // uniform over the workgroup
+        if (nsf > 0 && tid == 0) smon[I] = 0;
+        chol_diag_block<double>(NB, 0, Rb, Li, flags, sL, col, rdiag, false);
+        return;
+    }
+    if (tid == 0) bad = 0;
+    // D into Li, which chol_diag_block reads before it writes the inverse there
+    for (int e = tid; e < NB * NB; e += 256) {
+        const int r = e >> 6, c = e & 63, fr = pa.rowf[I * NB + r], fc = pa.rowf[I * NB + c];
+        double v;
+        if (fr < 0 && fc < 0) {
+            v = Rb[e];
+        } else if (fr >= 0 && fr == fc) {
+            const int ia = ra[I * NB + r], ib = ra[I * NB + c];
+            v = eeq_a(ia, ib, x, alp, diag);
+            if (solv) v += born_b(sv, ia, ib);
+        } else {
+            v = 0.0;
+        }
+        Li[e] = v;
+        // the fragment's last atom, by its first row
+        if (c == 0 && fr >= 0 && pa.pidx[pa.poff[fr >> 1]] == (int)(2 * I + (fr & 1)) &&
+            (r == 0 || pa.rowf[I * NB + r - 1] != fr)) {
+            const int la = rl[I * NB + r];
+            const double d = diag[la] + (solv ? born_b(sv, la, la) : 0.0);
+            all[fr >> 1] = d > 0.0 ? d : diag[la];
+        }
+    }
+    __syncthreads();
+    chol_diag_block<double>(NB, 0, Li, Li, &bad, sL, col, rdiag, false);
+    __syncthreads();
+    const bool on = bad == 0;
+    if (!on) chol_diag_block<double>(NB, 0, Rb, Li, flags, sL, col, rdiag, false);
+    __syncthreads();
+    if (tid == 0) smon[I] = on;
+    // w = L^-T (L^-1 1_f) per piece, the pieces of a block being disjoint: one
+    // pass with both indicators, thread (t, q) a quarter of row t's products
+    double* const v0 = &sL[0][0];  // LDS of the factor, no longer read
+    const int t = tid >> 2, q = tid & 3;
+    double p0 = 0.0, p1 = 0.0;
+    for (int u = 0; u < NB / 4; ++u) {
+        const int c = 4 * u + q, fc = pa.rowf[I * NB + c];
+        const double lv = Li[t * NB + c];
+        if (fc >= 0) (fc & 1 ? p1 : p0) += lv;
+    }
+    p0 += __shfl_xor(p0, 1);
+    p0 += __shfl_xor(p0, 2);
+    p1 += __shfl_xor(p1, 1);
+    p1 += __shfl_xor(p1, 2);
+    if (q == 0) {
+        v0[t] = p0;
+        v0[NB + t] = p1;
+    }
+    __syncthreads();
+    // rows of one piece couple only to their own indicator (D is block diagonal over the fragments)
+    const int ft = pa.rowf[I * NB + t];
+    double wt = 0.0;
+    for (int u = 0; u < NB / 4; ++u) wt += Li[(4 * u + q) * NB + t] * v0[(ft & 1) * NB + 4 * u + q];
+    wt += __shfl_xor(wt, 1);
+    wt += __shfl_xor(wt, 2);
+    if (ft < 0 || !on) wt = 0.0;
+    __syncthreads();
+    if (q == 0) {
+        w[I * NB + t] = wt;
+        v0[t] = wt;
+    }
+    __syncthreads();
+    if (tid < NB) {
+        const int f = pa.rowf[I * NB + tid];
+        const double s0 = wave_sum(f >= 0 && !(f & 1) ? v0[tid] : 0.0), s1 = wave_sum(f >= 0 && (f & 1) ? v0[tid] : 0.0);
+        if (tid < 2) w1[2 * I + tid] = tid ? s1 : s0;
+    }
+}
+
 // Charged fragments: the Born part of A qp leaves the right-hand side
 __global__ __launch_bounds__(256) void k_solv_rhs(SolvArgs a, const double* __restrict__ qp, double* __restrict__ r) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -5411,6 +5619,10 @@ struct DeviceEngine {
     double* cg_part = nullptr;          // block-product partials [nbk][nbk][64]
     unsigned long long* cg_mb = nullptr;  // all-reduce mailboxes of the persistent PCG
     int* cg_iters = nullptr;
+    PcgArgs cg{};                       // k_eeq_pcg
+    bool cg_res = false;                // its blocks stay in registers
+    double *cg_w = nullptr, *cg_w1 = nullptr, *cg_all = nullptr;
+    int* cg_smon = nullptr;
     int* ready = nullptr;               // per-block ready flags of the solve sweeps
     // batches of molecules (nmol > 1)
     int nmol = 1, nbtiles = 0;
@@ -5566,6 +5778,50 @@ struct DeviceEngine {
     }
 };
 
+// Order of the reduced variables of the iterative solve: the atoms of a
+// fragment of more than 64 variables in breadth-first order over its bonds
+// from an end of the molecule (the last atom of two searches), so that a
+// 64-variable block holds neighbouring atoms; in an alkane's own order one
+// block holds carbons and another their hydrogens, and the block-Jacobi
+// preconditioner misses the coupling between them.  The last atom, whose
+// variable is eliminated, stays the last.
+static void reduced_order(const ParamSet& P, std::vector<std::vector<int>>& fa) {
+    std::vector<std::vector<int>> nb;
+    for (std::vector<int>& at : fa) {
+        if ((int)at.size() - 1 <= NB) continue;
+        if (nb.empty()) {
+            nb.resize(P.n);
+            for (size_t k = 0; k + 1 < P.bond_ij.size(); k += 2) {
+                nb[P.bond_ij[k]].push_back(P.bond_ij[k + 1]);
+                nb[P.bond_ij[k + 1]].push_back(P.bond_ij[k]);
+            }
+            for (auto& v : nb) std::sort(v.begin(), v.end());
+        }
+        const int last = at.back();
+        std::vector<int> order;
+        std::vector<char> seen(P.n, 0), mine(P.n, 0);
+        for (int i : at) mine[i] = 1;
+        int start = at[0];
+        for (int pass = 0; pass < 3; ++pass) {
+            order.assign(1, start);
+            std::fill(seen.begin(), seen.end(), 0);
+            seen[start] = 1;
+            for (size_t k = 0; k < order.size(); ++k)
+                for (int j : nb[order[k]])
+                    if (mine[j] && !seen[j]) {
+                        seen[j] = 1;
+                        order.push_back(j);
+                    }
+            start = order.back();
+        }
+        for (int i : at)  // atoms that no bond of the list reaches keep their order
+            if (!seen[i]) order.push_back(i);
+        order.erase(std::find(order.begin(), order.end(), last));
+        order.push_back(last);
+        at.swap(order);
+    }
+}
+
 DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt, int& status, std::string& msg) {
     const bool lookahead = opt.cholesky_lookahead;
     const int solver = opt.eeq_solver;
@@ -5639,6 +5895,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         for (int i = 0; i < n; ++i) fa[P.frag[i]].push_back(i);
         std::vector<int> red_atom, red_last, red_of(n, -1), foff(P.nfrag + 1, 0), fatoms;
         std::vector<double> qp(n, 0.0);
+        if (E->use_cg) reduced_order(P, fa);
         for (int f = 0; f < P.nfrag; ++f) {
             int m = (int)fa[f].size();
             int last = fa[f].back();
@@ -6174,14 +6431,20 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             int dev = 0, ncu = 0, per_cu = 0;
             if (hipGetDevice(&dev) != hipSuccess ||
                 hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eeq_pcg, PCG_THREADS, 0) != hipSuccess) {
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eeq_pcg<false, true>, PCG_THREADS, 0) !=
+                    hipSuccess) {
                 status = kErrDevice;
                 msg = "PCG occupancy query failed";
                 delete E;
                 return nullptr;
             }
             const long T = (long)nbk * (nbk + 1) / 2;
-            E->cg_groups = (int)std::min<long>({(long)ncu * per_cu, 256L, T});
+            // workgroups: enough wavefronts for one block each, so that the blocks
+            // stay in registers, and two per owned 64-row block; more only add lines
+            // to the all-reduce (512 H2O, 136 blocks: 16 groups 354 us per
+            // evaluation, 32 312, 136 320; H-(Gly)200-OH, 253 blocks: 32 734, 64 726,
+            // 253 782; 8 chains, 496 blocks: 32 1220, 64 925, 256 1045)
+            E->cg_groups = (int)std::min<long>({(long)ncu * per_cu, 256L, T, std::max(2L * nbk, (T + PCG_WAVES - 1) / PCG_WAVES)});
             if (opt.pcg_groups > 0) E->cg_groups = std::min(E->cg_groups, opt.pcg_groups);
             if (E->cg_groups < 1 || cdiv(nbk, E->cg_groups) > PCG_MAXB) E->use_cg = false;
             if (E->use_cg) E->mat_size = (size_t)T * NB * NB;  // packed symmetric storage
@@ -6204,6 +6467,52 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             E->cg_part = E->alloc<double>((size_t)(E->np / NB) * E->np);
             E->cg_mb = E->alloc<unsigned long long>(MB_WORDS);
             E->cg_iters = E->alloc<int>(1);
+            const int nbk = E->np / NB;
+            E->cg_res = (long)nbk * (nbk + 1) / 2 <= (long)PCG_WAVES * E->cg_groups;
+            // split fragments: more than 64 variables, so never inside one block
+            std::vector<int> rowf(E->np, -1), poff(1, 0), pidx;
+            int nsf = 0;
+            for (int r0 = 0; r0 < E->nr;) {
+                int r1 = r0 + 1;
+                while (r1 < E->nr && red_last[r1] == red_last[r0]) ++r1;
+                if (r1 - r0 > NB) {
+                    for (int r = r0; r < r1; ++r) {
+                        const int bk = r / NB;
+                        // second piece of its block when another split fragment, which then
+                        // holds the block's first row, comes before it there
+                        const int slot = rowf[bk * NB] >= 0 && (rowf[bk * NB] >> 1) != nsf ? 1 : 0;
+                        rowf[r] = 2 * nsf + slot;
+                        if (r == r0 || r % NB == 0) pidx.push_back(2 * bk + slot);
+                    }
+                    poff.push_back((int)pidx.size());
+                    ++nsf;
+                }
+                r0 = r1;
+            }
+            PcgArgs& a = E->cg;
+            a.np = E->np;
+            a.maxit = PCG_MAXIT;
+            a.tol2 = E->cg_tol2;
+            a.Rp = E->Ared;
+            a.Lj = E->Linv;
+            a.b = E->b;
+            a.x = E->xbuf;
+            a.z = E->cg_z;
+            a.pb = E->cg_p;
+            a.part = E->cg_part;
+            a.mb = E->cg_mb;
+            a.iters = E->cg_iters;
+            a.nsf = (nsf <= SM_MAXF && nbk <= SM_MAXB) ? nsf : 0;
+            if (a.nsf > 0) {
+                a.rowf = E->upload(rowf);
+                a.poff = E->upload(poff);
+                a.pidx = E->upload(pidx);
+                a.w = E->cg_w = E->alloc<double>(E->np);
+                a.w1 = E->cg_w1 = E->alloc<double>(2 * (size_t)nbk);
+                a.all = E->cg_all = E->alloc<double>(nsf);
+                a.smon = E->cg_smon = E->alloc<int>(nbk);
+                a.sp = E->alloc<double>(2 * (size_t)nbk);
+            }
         } else if (E->mixed && E->nmol > 1 && E->batch_fp32 && E->batch_solver != 2 && E->batch_solver < 4) {
             E->Ared32 = E->alloc<float>(E->mat_size);  // FP32 copies of the molecules' matrices and factors
             E->Linv32 = E->alloc<float>((size_t)E->np * NB);
@@ -6368,6 +6677,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->flags = E->alloc<int>(1);
         E->sticky = E->alloc<int>(1);
         E->sa.flags = E->flags;
+        E->cg.flags = E->flags;
         if (hipStreamCreate(&E->own) != hipSuccess || hipStreamCreate(&E->la.side) != hipSuccess ||
             hipEventCreateWithFlags(&E->la.fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&E->la.join, hipEventDisableTiming) != hipSuccess ||
@@ -6644,7 +6954,9 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
         if (E->use_cg) {
             // block-Jacobi factors of R's diagonal blocks and the solver's
             // mailboxes, also off the evaluation stream
-            LAUNCH(KC_CHOL_DIAG, k_bjacobi_setup, dim3(nbk), dim3(256), E->side, E->Ared, E->Linv, E->flags);
+            LAUNCH(KC_CHOL_DIAG, k_bjacobi_setup, dim3(nbk), dim3(256), E->side, E->Ared, E->Linv, E->flags,
+                   E->cg.nsf, E->cg, E->red_atom, E->red_last, E->x, E->alp, E->diag, E->solv ? 1 : 0, E->sa, E->cg_w,
+                   E->cg_w1, E->cg_all, E->cg_smon);
             hipLaunchKernelGGL(k_fill_u64, dim3(cdiv(MB_WORDS, 256)), dim3(256), 0, E->side, MB_WORDS, E->cg_mb,
                                MB_EMPTY);
         }
@@ -6788,8 +7100,15 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
                    E->mmo, E->mvo, E->Ared, E->Linv, (const double*)nullptr, E->b, E->xbuf);
     } else if (E->use_cg) {
         // the persistent PCG (block-Jacobi factors and mailboxes were set up on the side stream)
-        LAUNCH(KC_PCG, k_eeq_pcg, dim3(E->cg_groups), dim3(PCG_THREADS), s, np, E->Ared, E->Linv, E->b, E->xbuf,
-               E->cg_z, E->cg_p, E->cg_part, E->cg_mb, E->cg_iters, E->cg_tol2, PCG_MAXIT, E->flags);
+        const dim3 grid(E->cg_groups), block(PCG_THREADS);
+        if (E->cg_res && E->cg.nsf)
+            LAUNCH(KC_PCG, (k_eeq_pcg<true, true>), grid, block, s, E->cg);
+        else if (E->cg_res)
+            LAUNCH(KC_PCG, (k_eeq_pcg<true, false>), grid, block, s, E->cg);
+        else if (E->cg.nsf)
+            LAUNCH(KC_PCG, (k_eeq_pcg<false, true>), grid, block, s, E->cg);
+        else
+            LAUNCH(KC_PCG, (k_eeq_pcg<false, false>), grid, block, s, E->cg);
     } else if (!E->mixed) {
         if (E->lu_src)
             LAUNCH(KC_CHOL_DIAG, k_copy, dim3(cdiv((long)E->mat_size, 256)), dim3(256), s, (int)E->mat_size, E->Ared,
