@@ -539,10 +539,9 @@ __global__ __launch_bounds__(256) void k_eeq_rhs_qp(int n, const double* __restr
     r[i] = rhs[i] - s;
 }
 
-__global__ __launch_bounds__(256) void k_eeq_rhs_reduce(int nr, int np, const int* __restrict__ ra,
-                                                        const int* __restrict__ rl, const double* __restrict__ r,
-                                                        double* __restrict__ b) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void rhs_reduce_entry(int a, int nr, int np, const int* __restrict__ ra,
+                                                 const int* __restrict__ rl, const double* __restrict__ r,
+                                                 double* __restrict__ b) {
     if (a >= np) return;
     b[a] = (a < nr && ra[a] >= 0) ? r[ra[a]] - r[rl[a]] : 0.0;  // ra < 0: padding of a batched block
 }
@@ -1882,11 +1881,10 @@ __device__ inline void pair_range(const PairArgs& a, int cj, int& j0, int& j1) {
 //   dh[i][e][b] = sum_a dgw_i[a] c6ref[ei, e, a, b]
 // so that C6_ij = h[i][ej] . gw_j and dC6_ij/dCN_i = dh[i][ej] . gw_j
 // (the reference's half-contraction, d4param_generator.cpp:1235).
-__global__ __launch_bounds__(256) void k_d4_half(int n, int ne, const int* __restrict__ elem,
-                                                 const int* __restrict__ nref, const double* __restrict__ c6ref,
-                                                 const double* __restrict__ gw, const double* __restrict__ dgw,
-                                                 double* __restrict__ h, double* __restrict__ dh) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void d4_half_entry(int t, int n, int ne, const int* __restrict__ elem,
+                                              const int* __restrict__ nref, const double* __restrict__ c6ref,
+                                              const double* __restrict__ gw, const double* __restrict__ dgw,
+                                              double* __restrict__ h, double* __restrict__ dh) {
     if (t >= n * ne) return;
     int i = t / ne, e = t % ne;
     int ei = elem[i], nri = nref[ei];
@@ -2563,15 +2561,14 @@ __device__ inline void nbrep_fix_atom(int i, const double* __restrict__ x, const
 // lanes stride the bond's hydrogen-bond partner list (HB coordination and
 // its gradient), fixed butterflies; lane 0 writes the bond's own slots
 
-__global__ __launch_bounds__(256) void k_bonds(int nsel, const int* __restrict__ bsel, const int* __restrict__ ij,
-                                               const double* __restrict__ par,
-                                               const int* __restrict__ hb_off, const int* __restrict__ hb_B,
-                                               const int* __restrict__ slot0, const double* __restrict__ x,
-                                               const double* __restrict__ cn, const double* __restrict__ rcov_d3,
-                                               const int* __restrict__ bond_H, double* __restrict__ slots,
-                                               double* __restrict__ dcn_slot, double* __restrict__ e_out) {
+__device__ __forceinline__ void bond_hb_wave(int w, int nsel, const int* __restrict__ bsel,
+                                             const int* __restrict__ ij, const double* __restrict__ par,
+                                             const int* __restrict__ hb_off, const int* __restrict__ hb_B,
+                                             const int* __restrict__ slot0, const double* __restrict__ x,
+                                             const double* __restrict__ cn, const double* __restrict__ rcov_d3,
+                                             const int* __restrict__ bond_H, double* __restrict__ slots,
+                                             double* __restrict__ dcn_slot, double* __restrict__ e_out) {
     const int lane = threadIdx.x & 63;
-    const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (w >= nsel) return;
     const int b = bsel[w];
     int i = ij[2 * b], j = ij[2 * b + 1];
@@ -2639,15 +2636,13 @@ __global__ __launch_bounds__(256) void k_bonds(int nsel, const int* __restrict__
 
 // bonds without HB coordination (no X-H hydrogen, or an empty partner list,
 // where hbcn = 0 leaves alpha = a0 exactly; bsel: their indices), one thread
-// each: the arithmetic of k_bonds' lane 0; an X-H bond's hydrogen slot gets
+// each: the arithmetic of bond_hb_wave's lane 0; an X-H bond's hydrogen slot gets
 // its zero gradient
-__global__ __launch_bounds__(256) void k_bonds_plain(int nsel, const int* __restrict__ bsel,
-                                                     const int* __restrict__ ij, const double* __restrict__ par,
-                                                     const int* __restrict__ slot0, const int* __restrict__ bond_H,
-                                                     const double* __restrict__ x, const double* __restrict__ cn,
-                                                     double* __restrict__ slots, double* __restrict__ dcn_slot,
-                                                     double* __restrict__ e_out) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void bond_plain(int t, int nsel, const int* __restrict__ bsel, const int* __restrict__ ij,
+                                           const double* __restrict__ par, const int* __restrict__ slot0,
+                                           const int* __restrict__ bond_H, const double* __restrict__ x,
+                                           const double* __restrict__ cn, double* __restrict__ slots,
+                                           double* __restrict__ dcn_slot, double* __restrict__ e_out) {
     if (t >= nsel) return;
     const int b = bsel[t];
     const int i = ij[2 * b], j = ij[2 * b + 1];
@@ -2670,11 +2665,10 @@ __global__ __launch_bounds__(256) void k_bonds_plain(int nsel, const int* __rest
 }
 
 // angles: ff_workspace_gfnff.cpp:187-275
-__global__ __launch_bounds__(256) void k_angles(int na, const int* __restrict__ ijk, const double* __restrict__ par,
-                                                const int* __restrict__ slot0, const double* __restrict__ x,
-                                                const double* __restrict__ rcov_d3, double* __restrict__ slots,
-                                                double* __restrict__ e_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void angle_entry(int t, int na, const int* __restrict__ ijk,
+                                            const double* __restrict__ par, const int* __restrict__ slot0,
+                                            const double* __restrict__ x, const double* __restrict__ rcov_d3,
+                                            double* __restrict__ slots, double* __restrict__ e_out) {
     if (t >= na) return;
     int i = ijk[3 * t], j = ijk[3 * t + 1], k = ijk[3 * t + 2];
     double fc = par[2 * t], th0 = par[2 * t + 1];
@@ -2738,11 +2732,10 @@ __device__ __forceinline__ double dihed(double3 ri, double3 rj, double3 rk, doub
 }
 
 // torsions (primary and extra): ff_workspace_gfnff.cpp:282-482
-__global__ __launch_bounds__(256) void k_tors(int nt, const int* __restrict__ ijkl, const double* __restrict__ par,
-                                              const int* __restrict__ slot0, const double* __restrict__ x,
-                                              const double* __restrict__ rcov_d3, double* __restrict__ slots,
-                                              double* __restrict__ e_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void torsion_entry(int t, int nt, const int* __restrict__ ijkl,
+                                              const double* __restrict__ par, const int* __restrict__ slot0,
+                                              const double* __restrict__ x, const double* __restrict__ rcov_d3,
+                                              double* __restrict__ slots, double* __restrict__ e_out) {
     if (t >= nt) return;
     int id[4] = {ijkl[4 * t], ijkl[4 * t + 1], ijkl[4 * t + 2], ijkl[4 * t + 3]};
     const double* p = par + 4 * t;
@@ -2804,11 +2797,10 @@ __device__ __forceinline__ double oop(double3 ri, double3 rj, double3 rk, double
 // inversions: ff_workspace_gfnff.cpp:489-604.  par: fc, omega0, type
 // (0: V (1 - cos w), -1: V (cos w - cos w0)^2); damping over the distances of
 // the first neighbour j to the centre and the other two neighbours.
-__global__ __launch_bounds__(256) void k_inv(int nv, const int* __restrict__ ijkl, const double* __restrict__ par,
-                                             const int* __restrict__ slot0, const double* __restrict__ x,
-                                             const double* __restrict__ rcov_d3, double* __restrict__ slots,
-                                             double* __restrict__ e_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void inversion_entry(int t, int nv, const int* __restrict__ ijkl,
+                                                const double* __restrict__ par, const int* __restrict__ slot0,
+                                                const double* __restrict__ x, const double* __restrict__ rcov_d3,
+                                                double* __restrict__ slots, double* __restrict__ e_out) {
     if (t >= nv) return;
     int id[4] = {ijkl[4 * t], ijkl[4 * t + 1], ijkl[4 * t + 2], ijkl[4 * t + 3]};
     const double* p = par + 3 * t;
@@ -2856,10 +2848,10 @@ __global__ __launch_bounds__(256) void k_inv(int nv, const int* __restrict__ ijk
 
 // triple-bond torsions: ff_workspace_gfnff.cpp:611-648 (undamped),
 // E = erefhalf (1 - cos 2 phi)
-__global__ __launch_bounds__(256) void k_stors(int nt, const int* __restrict__ ijkl, const double* __restrict__ eh,
-                                               const int* __restrict__ slot0, const double* __restrict__ x,
-                                               double* __restrict__ slots, double* __restrict__ e_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void stors_entry(int t, int nt, const int* __restrict__ ijkl,
+                                            const double* __restrict__ eh, const int* __restrict__ slot0,
+                                            const double* __restrict__ x, double* __restrict__ slots,
+                                            double* __restrict__ e_out) {
     if (t >= nt) return;
     double3 gp[4];
     bool ok;
@@ -2873,10 +2865,9 @@ __global__ __launch_bounds__(256) void k_stors(int nt, const int* __restrict__ i
 }
 
 // bonded repulsion: ff_workspace_gfnff.cpp:774-807
-__global__ __launch_bounds__(256) void k_brep(int nb, const int* __restrict__ ij, const double* __restrict__ par,
-                                              const int* __restrict__ slot0, const double* __restrict__ x,
-                                              double* __restrict__ slots, double* __restrict__ e_out) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void brep_entry(int b, int nb, const int* __restrict__ ij, const double* __restrict__ par,
+                                           const int* __restrict__ slot0, const double* __restrict__ x,
+                                           double* __restrict__ slots, double* __restrict__ e_out) {
     if (b >= nb) return;
     int i = ij[2 * b], j = ij[2 * b + 1];
     double3 d = ld3(x, i) - ld3(x, j);
@@ -3127,11 +3118,10 @@ __device__ double hb_core(int A, int H, int B, int cs, const HBArgs& a, const do
 // the reference's: its short- and long-range damping derivatives
 // (-12 f_s t_s / (r (1 + t_s)) and -12 r f_l t_l / (70 (1 + t_l))) are kept as
 // they are, so along r_XB it is not the derivative of the energy.
-__global__ __launch_bounds__(256) void k_xb(int nx, const int* __restrict__ axb, const double* __restrict__ par,
-                                            const int* __restrict__ slot0, const double* __restrict__ x,
-                                            const double* __restrict__ hb_rad, double* __restrict__ slots,
-                                            double* __restrict__ e_out) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void xb_entry(int b, int nx, const int* __restrict__ axb, const double* __restrict__ par,
+                                         const int* __restrict__ slot0, const double* __restrict__ x,
+                                         const double* __restrict__ hb_rad, double* __restrict__ slots,
+                                         double* __restrict__ e_out) {
     if (b >= nx) return;
     int A = axb[3 * b], X = axb[3 * b + 1], B = axb[3 * b + 2];
     const double* p = par + 3 * b;
@@ -3394,11 +3384,10 @@ struct HBRoles {
     int ng0, ng1, ngt;  // role A chunks [0, ng0), H [ng0, ng1), B [ng1, ngt)
 };
 template <int ROLE, typename T>
-__global__ __launch_bounds__(256) void k_hb_role(HBRoles r, HBArgs a, const double* __restrict__ x,
-                                                 double* __restrict__ gout, double* __restrict__ egrp) {
+__device__ __forceinline__ void hb_role_chunk(int w, const HBRoles& r, const HBArgs& a, const double* __restrict__ x,
+                                              double* __restrict__ gout, double* __restrict__ egrp) {
     const int lane = threadIdx.x & 63;
-    const int g0 = (ROLE == 0) ? 0 : (ROLE == 1 ? r.ng0 : r.ng1), g1 = (ROLE == 0) ? r.ng0 : (ROLE == 1 ? r.ng1 : r.ngt);
-    const int w = g0 + blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int g1 = (ROLE == 0) ? r.ng0 : (ROLE == 1 ? r.ng1 : r.ngt);
     if (w >= g1) return;
     const int at = r.gatom[w], e0 = r.goff[w], e1 = r.goff[w + 1];
     double3 g = make_double3(0, 0, 0);
@@ -3428,6 +3417,21 @@ __global__ __launch_bounds__(256) void k_hb_role(HBRoles r, HBArgs a, const doub
         st3(gout, w, g);
         if (ROLE == 0) egrp[w] = E;
     }
+}
+
+// the three roles in one launch (four chunks per workgroup, a role's last
+// workgroup partly idle): the roles' tails overlap
+template <typename T>
+__global__ __launch_bounds__(256) void k_hb_roles(HBRoles r, HBArgs a, const double* __restrict__ x,
+                                                  double* __restrict__ gout, double* __restrict__ egrp) {
+    const int b0 = (r.ng0 + 3) / 4, b1 = b0 + (r.ng1 - r.ng0 + 3) / 4, wv = threadIdx.x >> 6;
+    const int blk = blockIdx.x;
+    if (blk < b0)
+        hb_role_chunk<0, T>(blk * 4 + wv, r, a, x, gout, egrp);
+    else if (blk < b1)
+        hb_role_chunk<1, T>(r.ng0 + (blk - b0) * 4 + wv, r, a, x, gout, egrp);
+    else
+        hb_role_chunk<2, T>(r.ng1 + (blk - b1) * 4 + wv, r, a, x, gout, egrp);
 }
 
 // Hydrogen bonds of cases 2-4, one thread each: energy, and the gradient in
@@ -3462,21 +3466,29 @@ __global__ __launch_bounds__(256, 2) void k_hb_full(int nh, const int* __restric
 // case-1 chunk results in roles A, H, B (chunks [crange[r (n + 1) + i],
 // crange[r (n + 1) + i + 1])) and its slots of cases 2-4; lanes stride the
 // lists, fixed butterfly
+struct HBGather {
+    const int* crange;  // nullptr: no hydrogen bonds
+    const double* gout;
+    const int *xoff, *xidx;
+    const double* xslots;
+};
 template <int LPA>
-__global__ __launch_bounds__(256) void k_hb_gather(int n, const int* __restrict__ crange,
-                                                   const double* __restrict__ gout, const int* __restrict__ xoff,
-                                                   const int* __restrict__ xidx, const double* __restrict__ xslots,
-                                                   double* __restrict__ g) {
-    const int lane = threadIdx.x & (LPA - 1);
-    const int i = blockIdx.x * (256 / LPA) + threadIdx.x / LPA;
-    if (i >= n) return;
+__device__ __forceinline__ double3 hb_gather(int i, int lane, int n, const HBGather& h) {
     double3 s = make_double3(0, 0, 0);
 #pragma unroll
     for (int role = 0; role < 3; ++role) {
-        const int* cr = crange + role * (n + 1);
-        for (int k = cr[i] + lane; k < cr[i + 1]; k += LPA) s = s + ld3(gout, k);
+        const int* cr = h.crange + role * (n + 1);
+        for (int k = cr[i] + lane; k < cr[i + 1]; k += LPA) s = s + ld3(h.gout, k);
     }
-    for (int k = xoff[i] + lane; k < xoff[i + 1]; k += LPA) s = s + ld3(xslots, xidx[k]);
+    for (int k = h.xoff[i] + lane; k < h.xoff[i + 1]; k += LPA) s = s + ld3(h.xslots, h.xidx[k]);
+    return s;
+}
+template <int LPA>
+__global__ __launch_bounds__(256) void k_hb_gather(int n, HBGather h, double* __restrict__ g) {
+    const int lane = threadIdx.x & (LPA - 1);
+    const int i = blockIdx.x * (256 / LPA) + threadIdx.x / LPA;
+    if (i >= n) return;
+    double3 s = hb_gather<LPA>(i, lane, n, h);
 #pragma unroll
     for (int o = LPA / 2; o > 0; o >>= 1) {
         s.x += __shfl_xor(s.x, o);
@@ -3498,13 +3510,12 @@ __device__ inline double c6_pair(int i, int j, int ne, const int* elem, const in
     return s;
 }
 
-__global__ __launch_bounds__(256) void k_atm(int nt, const int* __restrict__ ijk, const double* __restrict__ sc,
-                                             const int* __restrict__ slot0, const double* __restrict__ x,
-                                             const double* __restrict__ rcov_d3, int ne, const int* __restrict__ elem,
-                                             const int* __restrict__ nref, const double* __restrict__ c6ref,
-                                             const double* __restrict__ gw, double* __restrict__ slots,
-                                             double* __restrict__ e_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void atm_entry(int t, int nt, const int* __restrict__ ijk, const double* __restrict__ sc,
+                                          const int* __restrict__ slot0, const double* __restrict__ x,
+                                          const double* __restrict__ rcov_d3, int ne, const int* __restrict__ elem,
+                                          const int* __restrict__ nref, const double* __restrict__ c6ref,
+                                          const double* __restrict__ gw, double* __restrict__ slots,
+                                          double* __restrict__ e_out) {
     if (t >= nt) return;
     int i = ijk[3 * t], j = ijk[3 * t + 1], k = ijk[3 * t + 2];
     double c9 = sqrt(fabs(c6_pair(i, j, ne, elem, nref, c6ref, gw) * c6_pair(i, k, ne, elem, nref, c6ref, gw) *
@@ -3541,11 +3552,10 @@ __global__ __launch_bounds__(256) void k_atm(int nt, const int* __restrict__ ijk
     st3(slots, q + 2, a2 * vik + a3 * vjk);
 }
 
-__global__ __launch_bounds__(256) void k_batm(int nt, const int* __restrict__ ijk, const double* __restrict__ zb,
-                                              const int* __restrict__ slot0, const double* __restrict__ x,
-                                              const double* __restrict__ qa, double* __restrict__ slots,
-                                              double* __restrict__ e_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void batm_entry(int t, int nt, const int* __restrict__ ijk, const double* __restrict__ zb,
+                                           const int* __restrict__ slot0, const double* __restrict__ x,
+                                           const double* __restrict__ qa, double* __restrict__ slots,
+                                           double* __restrict__ e_out) {
     if (t >= nt) return;
     int i = ijk[3 * t], j = ijk[3 * t + 1], k = ijk[3 * t + 2];
     double3 vij = ld3(x, j) - ld3(x, i), vik = ld3(x, k) - ld3(x, i), vjk = ld3(x, k) - ld3(x, j);
@@ -3575,6 +3585,93 @@ __global__ __launch_bounds__(256) void k_batm(int nt, const int* __restrict__ ij
     st3(slots, q, gij + gik);                 // i
     st3(slots, q + 1, (-1.0) * gij + gjk);    // j
     st3(slots, q + 2, (-1.0) * (gik + gjk));  // k
+}
+
+// Every list term that needs only coordinates, CN and D4 weights, the D4 half
+// contraction and the reduced EEQ right-hand side in one launch: the lists are
+// short next to the chip (hundreds of entries for 100 atoms, one wavefront or
+// two per list and SIMD), and ten launches of 4 to 18 us in a row took 60 to
+// 90 us where the longest single chain, a torsion's or an ATM triple's, takes
+// about 16.  Workgroups are dealt to the lists in the order below, the
+// longest chains first.  Launches of many workgroups are bound by throughput
+// instead: there each list runs in a launch of its own with its own register
+// count (the torsions' 114 registers hold the fused kernel at four wavefronts
+// per SIMD): 4096 molecules, 52,000 workgroups, 6.51 against 6.65 ms fused;
+// 122 to 1536 atoms, up to 500 workgroups, 331 -> 280 us fused on 512 H2O.
+constexpr int TERMS_FUSED_MAX = 2048;
+struct TermArgs {
+    int end[12];  // workgroups of the sections 0 .. k
+    int n, ne, nr, np;
+    int nb_hb, nb_plain, nangle, ntors, ninv, nstors, nxb, nbrep, natm, nbatm;
+    const double *x, *cn, *rcov_d3, *hb_rad, *gw, *dgw, *qa, *c6ref;
+    const int *elem, *nref;
+    const int *bsel_hb, *bsel_plain, *bond_ij, *bond_H, *bond_hboff, *bond_hbB, *bond_slot;
+    const double* bond_par;
+    const int *ang_ijk, *ang_slot, *tor_ijkl, *tor_slot, *inv_ijkl, *inv_slot, *st_ijkl, *st_slot, *xb_axb, *xb_slot;
+    const double *ang_par, *tor_par, *inv_par, *st_par, *xb_par;
+    const int *brep_ij, *brep_slot, *atm_ijk, *atm_slot, *batm_ijk, *batm_slot;
+    const double *brep_par, *atm_sc, *batm_zb;
+    double *slots, *dcn_slot, *e_bond, *e_ang, *e_tor, *e_inv, *e_st, *e_xb, *e_brep, *e_atm, *e_batm;
+    double *h6, *dh6;
+    const int *red_atom, *red_last;
+    const double* rhs;
+    double* b;
+};
+// ONE >= 0: that section alone (blockIdx.x counts its workgroups)
+template <int ONE>
+__global__ __launch_bounds__(256) void k_terms(TermArgs a) {
+    int sec = ONE, first = 0;
+    if (ONE < 0) {
+        sec = 0;
+#pragma unroll
+        for (int k = 0; k < 11; ++k)
+            if ((int)blockIdx.x >= a.end[k]) {
+                sec = k + 1;
+                first = a.end[k];
+            }
+    }
+    const int blk = blockIdx.x - first, t = blk * 256 + threadIdx.x;
+    switch (sec) {
+        case 0:
+            atm_entry(t, a.natm, a.atm_ijk, a.atm_sc, a.atm_slot, a.x, a.rcov_d3, a.ne, a.elem, a.nref, a.c6ref, a.gw,
+                      a.slots, a.e_atm);
+            break;
+        case 1:
+            torsion_entry(t, a.ntors, a.tor_ijkl, a.tor_par, a.tor_slot, a.x, a.rcov_d3, a.slots, a.e_tor);
+            break;
+        case 2:
+            bond_hb_wave(blk * 4 + (threadIdx.x >> 6), a.nb_hb, a.bsel_hb, a.bond_ij, a.bond_par, a.bond_hboff,
+                         a.bond_hbB, a.bond_slot, a.x, a.cn, a.rcov_d3, a.bond_H, a.slots, a.dcn_slot, a.e_bond);
+            break;
+        case 3:
+            inversion_entry(t, a.ninv, a.inv_ijkl, a.inv_par, a.inv_slot, a.x, a.rcov_d3, a.slots, a.e_inv);
+            break;
+        case 4:
+            stors_entry(t, a.nstors, a.st_ijkl, a.st_par, a.st_slot, a.x, a.slots, a.e_st);
+            break;
+        case 5:
+            xb_entry(t, a.nxb, a.xb_axb, a.xb_par, a.xb_slot, a.x, a.hb_rad, a.slots, a.e_xb);
+            break;
+        case 6:
+            angle_entry(t, a.nangle, a.ang_ijk, a.ang_par, a.ang_slot, a.x, a.rcov_d3, a.slots, a.e_ang);
+            break;
+        case 7:
+            batm_entry(t, a.nbatm, a.batm_ijk, a.batm_zb, a.batm_slot, a.x, a.qa, a.slots, a.e_batm);
+            break;
+        case 8:
+            brep_entry(t, a.nbrep, a.brep_ij, a.brep_par, a.brep_slot, a.x, a.slots, a.e_brep);
+            break;
+        case 9:
+            bond_plain(t, a.nb_plain, a.bsel_plain, a.bond_ij, a.bond_par, a.bond_slot, a.bond_H, a.x, a.cn, a.slots,
+                       a.dcn_slot, a.e_bond);
+            break;
+        case 10:
+            d4_half_entry(t, a.n, a.ne, a.elem, a.nref, a.c6ref, a.gw, a.dgw, a.h6, a.dh6);
+            break;
+        default:
+            rhs_reduce_entry(t, a.nr, a.np, a.red_atom, a.red_last, a.rhs, a.b);
+            break;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -4749,15 +4846,18 @@ __device__ inline double group_sum(double v) {
     return v;
 }
 // Per-atom sum of the bonded-list gradient slots (every slot writer runs
-// before the EEQ solve, so this gather runs there too, off the solve's path).
+// before the EEQ solve, so this gather runs there too, off the solve's path),
+// and of a single molecule's hydrogen-bond gradients (h.crange nullptr: none).
 template <int LPA>
 __global__ __launch_bounds__(256) void k_slot_gather(int n, const int* __restrict__ soff, const int* __restrict__ sidx,
-                                                     const double* __restrict__ slots, double* __restrict__ gslot) {
+                                                     const double* __restrict__ slots, HBGather h,
+                                                     double* __restrict__ gslot) {
     const int lane = threadIdx.x & (LPA - 1);
     const int i = blockIdx.x * (256 / LPA) + threadIdx.x / LPA;
     if (i >= n) return;
     double3 g = make_double3(0, 0, 0);
     for (int k = soff[i] + lane; k < soff[i + 1]; k += LPA) g = g + ld3(slots, sidx[k]);
+    if (h.crange) g = g + hb_gather<LPA>(i, lane, n, h);
     g.x = group_sum<LPA>(g.x);
     g.y = group_sum<LPA>(g.y);
     g.z = group_sum<LPA>(g.z);
@@ -4793,7 +4893,8 @@ __global__ __launch_bounds__(256) void k_finish(int n, const double* __restrict_
     g.y = group_sum<LPA>(g.y);
     g.z = group_sum<LPA>(g.z);
     if (lane == 0) {
-        g = g + ld3(gslot, i) + ld3(gpair, i) + ld3(ghb, i);
+        g = g + ld3(gslot, i) + ld3(gpair, i);
+        if (ghb) g = g + ld3(ghb, i);
         st3(grad, i, g);
     }
 }
@@ -5621,6 +5722,7 @@ struct DeviceEngine {
     int* cg_iters = nullptr;
     PcgArgs cg{};                       // k_eeq_pcg
     bool cg_res = false;                // its blocks stay in registers
+    TermArgs terms{};                   // k_terms
     double *cg_w = nullptr, *cg_w1 = nullptr, *cg_all = nullptr;
     int* cg_smon = nullptr;
     int* ready = nullptr;               // per-block ready flags of the solve sweeps
@@ -6678,6 +6780,33 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->sticky = E->alloc<int>(1);
         E->sa.flags = E->flags;
         E->cg.flags = E->flags;
+        {
+            TermArgs& a = E->terms;
+            const int cnt[12] = {cdiv(E->natm, 256),  cdiv(E->ntors, 256), cdiv(E->nb_hb, 4),   cdiv(E->ninv, 256),
+                                 cdiv(E->nstors, 256), cdiv(E->nxb, 256),  cdiv(E->nangle, 256), cdiv(E->nbatm, 256),
+                                 cdiv(E->nbrep, 256), cdiv(E->nb_plain, 256), cdiv(n * E->nelem, 256), cdiv(E->np, 256)};
+            for (int k = 0, at = 0; k < 12; ++k) a.end[k] = at += cnt[k];
+            a.n = n; a.ne = E->nelem; a.nr = E->nr; a.np = E->np;
+            a.nb_hb = E->nb_hb; a.nb_plain = E->nb_plain; a.nangle = E->nangle; a.ntors = E->ntors;
+            a.ninv = E->ninv; a.nstors = E->nstors; a.nxb = E->nxb; a.nbrep = E->nbrep; a.natm = E->natm;
+            a.nbatm = E->nbatm;
+            a.x = E->x; a.cn = E->cn; a.rcov_d3 = E->rcov_d3; a.hb_rad = E->hb_rad; a.gw = E->gw; a.dgw = E->dgw;
+            a.qa = E->qa; a.c6ref = E->c6ref; a.elem = E->elem; a.nref = E->nref;
+            a.bsel_hb = E->bsel_hb; a.bsel_plain = E->bsel_plain; a.bond_ij = E->bond_ij; a.bond_H = E->bond_H;
+            a.bond_hboff = E->bond_hboff; a.bond_hbB = E->bond_hbB; a.bond_slot = E->bond_slot; a.bond_par = E->bond_par;
+            a.ang_ijk = E->ang_ijk; a.ang_slot = E->ang_slot; a.ang_par = E->ang_par;
+            a.tor_ijkl = E->tor_ijkl; a.tor_slot = E->tor_slot; a.tor_par = E->tor_par;
+            a.inv_ijkl = E->inv_ijkl; a.inv_slot = E->inv_slot; a.inv_par = E->inv_par;
+            a.st_ijkl = E->st_ijkl; a.st_slot = E->st_slot; a.st_par = E->st_par;
+            a.xb_axb = E->xb_axb; a.xb_slot = E->xb_slot; a.xb_par = E->xb_par;
+            a.brep_ij = E->brep_ij; a.brep_slot = E->brep_slot; a.brep_par = E->brep_par;
+            a.atm_ijk = E->atm_ijk; a.atm_slot = E->atm_slot; a.atm_sc = E->atm_sc;
+            a.batm_ijk = E->batm_ijk; a.batm_slot = E->batm_slot; a.batm_zb = E->batm_zb;
+            a.slots = E->slots; a.dcn_slot = E->dcn_slot; a.e_bond = E->e_bond; a.e_ang = E->e_ang; a.e_tor = E->e_tor;
+            a.e_inv = E->e_inv; a.e_st = E->e_st; a.e_xb = E->e_xb; a.e_brep = E->e_brep; a.e_atm = E->e_atm;
+            a.e_batm = E->e_batm; a.h6 = E->h6; a.dh6 = E->dh6;
+            a.red_atom = E->red_atom; a.red_last = E->red_last; a.b = E->b;
+        }
         if (hipStreamCreate(&E->own) != hipSuccess || hipStreamCreate(&E->la.side) != hipSuccess ||
             hipEventCreateWithFlags(&E->la.fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&E->la.join, hipEventDisableTiming) != hipSuccess ||
@@ -6986,54 +7115,39 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
         if (E->solv) LAUNCH(KC_SOLV, k_solv_rhs, dim3(cdiv(n, 256)), dim3(256), s, E->sa, E->qp, E->rres);
         rsrc = E->rres;
     }
-    LAUNCH(KC_EEQ_BUILD, k_eeq_rhs_reduce, dim3(cdiv(np, 256)), dim3(256), s, E->nr, np, E->red_atom, E->red_last,
-                       rsrc, E->b);
-    // D4 half contractions need only CN: evaluated before the solve
-    LAUNCH(KC_PAIRS_AUX, k_d4_half, dim3(cdiv(n * E->nelem, 256)), dim3(256), s, n, E->nelem, E->elem, E->nref,
-           E->c6ref, E->gw, E->dgw, E->h6, E->dh6);
     const PairArgs pa = E->pair_args();
-    // bonded lists
-    if (E->nbond) {
-        if (E->nb_hb)
-            LAUNCH(KC_BONDS, k_bonds, dim3(cdiv(E->nb_hb, 4)), dim3(256), s, E->nb_hb, E->bsel_hb, E->bond_ij,
-                   E->bond_par, E->bond_hboff, E->bond_hbB, E->bond_slot, E->x, E->cn, E->rcov_d3, E->bond_H,
-                   E->slots, E->dcn_slot, E->e_bond);
-        if (E->nb_plain)
-            LAUNCH(KC_BONDS, k_bonds_plain, dim3(cdiv(E->nb_plain, 256)), dim3(256), s, E->nb_plain,
-                   E->bsel_plain, E->bond_ij, E->bond_par, E->bond_slot, E->bond_H, E->x, E->cn, E->slots,
-                   E->dcn_slot, E->e_bond);
+    {
+        TermArgs ta = E->terms;
+        ta.rhs = rsrc;
+        if (ta.end[11] <= TERMS_FUSED_MAX) {
+            LAUNCH(KC_BONDS, k_terms<-1>, dim3(ta.end[11]), dim3(256), s, ta);
+        } else {
+            auto wgs = [&](int k) { return dim3(ta.end[k] - (k ? ta.end[k - 1] : 0)); };
+            LAUNCH(KC_EEQ_BUILD, k_terms<11>, wgs(11), dim3(256), s, ta);
+            LAUNCH(KC_PAIRS_AUX, k_terms<10>, wgs(10), dim3(256), s, ta);
+            if (ta.nb_hb) LAUNCH(KC_BONDS, k_terms<2>, wgs(2), dim3(256), s, ta);
+            if (ta.nb_plain) LAUNCH(KC_BONDS, k_terms<9>, wgs(9), dim3(256), s, ta);
+            if (ta.nangle) LAUNCH(KC_ANGLES, k_terms<6>, wgs(6), dim3(256), s, ta);
+            if (ta.ntors) LAUNCH(KC_TORS, k_terms<1>, wgs(1), dim3(256), s, ta);
+            if (ta.ninv) LAUNCH(KC_TORS, k_terms<3>, wgs(3), dim3(256), s, ta);
+            if (ta.nstors) LAUNCH(KC_TORS, k_terms<4>, wgs(4), dim3(256), s, ta);
+            if (ta.nxb) LAUNCH(KC_HB, k_terms<5>, wgs(5), dim3(256), s, ta);
+            if (ta.nbrep) LAUNCH(KC_BREP, k_terms<8>, wgs(8), dim3(256), s, ta);
+            if (ta.natm) LAUNCH(KC_ATM, k_terms<0>, wgs(0), dim3(256), s, ta);
+            if (ta.nbatm) LAUNCH(KC_BATM, k_terms<7>, wgs(7), dim3(256), s, ta);
+        }
     }
-    if (E->nangle)
-        LAUNCH(KC_ANGLES, k_angles, dim3(cdiv(E->nangle, 256)), dim3(256), s, E->nangle, E->ang_ijk, E->ang_par,
-                           E->ang_slot, E->x, E->rcov_d3, E->slots, E->e_ang);
-    if (E->ntors)
-        LAUNCH(KC_TORS, k_tors, dim3(cdiv(E->ntors, 256)), dim3(256), s, E->ntors, E->tor_ijkl, E->tor_par,
-                           E->tor_slot, E->x, E->rcov_d3, E->slots, E->e_tor);
-    if (E->ninv)
-        LAUNCH(KC_TORS, k_inv, dim3(cdiv(E->ninv, 256)), dim3(256), s, E->ninv, E->inv_ijkl, E->inv_par, E->inv_slot,
-               E->x, E->rcov_d3, E->slots, E->e_inv);
-    if (E->nstors)
-        LAUNCH(KC_TORS, k_stors, dim3(cdiv(E->nstors, 256)), dim3(256), s, E->nstors, E->st_ijkl, E->st_par,
-               E->st_slot, E->x, E->slots, E->e_st);
-    if (E->nxb)
-        LAUNCH(KC_HB, k_xb, dim3(cdiv(E->nxb, 256)), dim3(256), s, E->nxb, E->xb_axb, E->xb_par, E->xb_slot, E->x,
-               E->hb_rad, E->slots, E->e_xb);
-    if (E->nbrep)
-        LAUNCH(KC_BREP, k_brep, dim3(cdiv(E->nbrep, 256)), dim3(256), s, E->nbrep, E->brep_ij, E->brep_par,
-                           E->brep_slot, E->x, E->slots, E->e_brep);
-    if (E->natm)
-        LAUNCH(KC_ATM, k_atm, dim3(cdiv(E->natm, 256)), dim3(256), s, E->natm, E->atm_ijk, E->atm_sc,
-                           E->atm_slot, E->x, E->rcov_d3, E->nelem, E->elem, E->nref, E->c6ref, E->gw, E->slots,
-                           E->e_atm);
-    if (E->nbatm)
-        LAUNCH(KC_BATM, k_batm, dim3(cdiv(E->nbatm, 256)), dim3(256), s, E->nbatm, E->batm_ijk, E->batm_zb,
-                           E->batm_slot, E->x, E->qa, E->slots, E->e_batm);
-    if (E->fin_lpa == 64)
-        LAUNCH(KC_CHAIN, k_slot_gather<64>, dim3(cdiv(n, 4)), dim3(256), s, n, E->slot_off, E->slot_idx, E->slots,
-               E->gslot);
-    else
-        LAUNCH(KC_CHAIN, k_slot_gather<16>, dim3(cdiv(n, 16)), dim3(256), s, n, E->slot_off, E->slot_idx, E->slots,
-               E->gslot);
+    // a single molecule's hydrogen bonds are gathered with the slots (below)
+    const HBGather hg{E->nhb ? E->hb_crange : nullptr, E->hb_gout, E->hb_xoff, E->hb_xidx, E->hb_xslots};
+    auto slot_gather = [&](const HBGather& h, int lpa) {
+        if (lpa == 64)
+            LAUNCH(KC_CHAIN, k_slot_gather<64>, dim3(cdiv(n, 4)), dim3(256), s, n, E->slot_off, E->slot_idx, E->slots,
+                   h, E->gslot);
+        else
+            LAUNCH(KC_CHAIN, k_slot_gather<16>, dim3(cdiv(n, 16)), dim3(256), s, n, E->slot_off, E->slot_idx, E->slots,
+                   h, E->gslot);
+    };
+    if (E->nmol > 1) slot_gather(HBGather{}, E->fin_lpa);
     // pair_split: the charge-independent pair terms (dispersion, repulsion)
     // last before the solve, beside the factorisation's smaller column blocks
     if (E->pair_split) queue_pairs_sym(E, s, pa, E->ps_part2, PT_DISP | PT_REP);
@@ -7048,20 +7162,13 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
         HBArgs ha{E->hb_cb, E->hb_ca, E->hb_Qh, E->hb_Qab, E->hb_nboff, E->hb_nbidx, E->hb_parc,
                   E->hb_nbcoff, E->hb_nbcidx, E->hb_rad, E->hb_lpd, E->Z, E->hb_pk, E->hb_qh32};
         HBRoles hr{E->hb_ent, E->hb_goff, E->hb_gatom, E->hb_ng0, E->hb_ng1, E->hb_ngt};
-        // case-1 role kernels (FP32 terms on the mixed path, FP64 otherwise)
-        const int gr0[3] = {0, E->hb_ng0, E->hb_ng1}, gr1[3] = {E->hb_ng0, E->hb_ng1, E->hb_ngt};
-        for (int role = 0; role < 3; ++role) {
-            const dim3 grid(cdiv(gr1[role] - gr0[role], 4));
-            if (gr1[role] <= gr0[role]) continue;
-            if (E->mixed) {
-                if (role == 0) LAUNCH(KC_HB, (k_hb_role<0, float>), grid, dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
-                if (role == 1) LAUNCH(KC_HB, (k_hb_role<1, float>), grid, dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
-                if (role == 2) LAUNCH(KC_HB, (k_hb_role<2, float>), grid, dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
-            } else {
-                if (role == 0) LAUNCH(KC_HB, (k_hb_role<0, double>), grid, dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
-                if (role == 1) LAUNCH(KC_HB, (k_hb_role<1, double>), grid, dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
-                if (role == 2) LAUNCH(KC_HB, (k_hb_role<2, double>), grid, dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
-            }
+        // case-1 roles (FP32 terms on the mixed path, FP64 otherwise)
+        const int nrole = cdiv(E->hb_ng0, 4) + cdiv(E->hb_ng1 - E->hb_ng0, 4) + cdiv(E->hb_ngt - E->hb_ng1, 4);
+        if (nrole) {
+            if (E->mixed)
+                LAUNCH(KC_HB, k_hb_roles<float>, dim3(nrole), dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
+            else
+                LAUNCH(KC_HB, k_hb_roles<double>, dim3(nrole), dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
         }
         // cases 2-4: on the mixed path the case-2 entries by the lean FP32
         // kernel and those of cases 3 and 4 by the FP64 one
@@ -7076,12 +7183,15 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
             LAUNCH(KC_HB, (k_hb_full<double, 2>), dim3(cdiv(n34, 256)), dim3(256), hs, n34, E->hb_ord + E->nhb2_c2,
                    E->hb_ahbc, E->hb_s0, ha, E->x, E->hb_xslots, E->e_hb2);
     }
-    if (E->hbg_lpa == 64)
-        LAUNCH(KC_HB, k_hb_gather<64>, dim3(cdiv(n, 4)), dim3(256), hs, n, E->hb_crange, E->hb_gout, E->hb_xoff,
-               E->hb_xidx, E->hb_xslots, E->ghb);
-    else
-        LAUNCH(KC_HB, k_hb_gather<16>, dim3(cdiv(n, 16)), dim3(256), hs, n, E->hb_crange, E->hb_gout, E->hb_xoff,
-               E->hb_xidx, E->hb_xslots, E->ghb);
+    if (E->nmol == 1)
+        slot_gather(hg, E->nhb ? std::max(E->fin_lpa, E->hbg_lpa) : E->fin_lpa);
+    else if (E->nhb) {
+        if (E->hbg_lpa == 64)
+            LAUNCH(KC_HB, k_hb_gather<64>, dim3(cdiv(n, 4)), dim3(256), hs, n, hg, E->ghb);
+        else
+            LAUNCH(KC_HB, k_hb_gather<16>, dim3(cdiv(n, 16)), dim3(256), hs, n, hg, E->ghb);
+    }
+    const double* ghb = (E->nmol > 1 && E->nhb) ? E->ghb : nullptr;
     HIP_OK(hipEventRecord(E->ev_join, E->side));
     // batches wait here for the factorisation only; the hydrogen-bond work
     // queued behind it on the side stream joins before k_finish
@@ -7175,10 +7285,10 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
     if (split) HIP_OK(hipStreamWaitEvent(s, E->ev_join, 0));
     if (E->fin_lpa == 64)
         LAUNCH(KC_CHAIN, k_finish<64>, dim3(cdiv(n, 4)), dim3(256), s, n, E->x, E->rcov_cn, E->dlog, E->vchain,
-                       E->nbn, E->nbl, E->gslot, E->gpair, E->ghb, E->grad);
+                       E->nbn, E->nbl, E->gslot, E->gpair, ghb, E->grad);
     else
         LAUNCH(KC_CHAIN, k_finish<16>, dim3(cdiv(n, 16)), dim3(256), s, n, E->x, E->rcov_cn, E->dlog, E->vchain,
-                       E->nbn, E->nbl, E->gslot, E->gpair, E->ghb, E->grad);
+                       E->nbn, E->nbl, E->gslot, E->gpair, ghb, E->grad);
     if (E->solv) {
         LAUNCH(KC_SOLV, k_solv_pairs, dim3(cdiv(n, 4)), dim3(256), s, E->sa, E->q);
         LAUNCH(KC_SOLV, k_solv_energy, dim3(1), dim3(256), s, E->sa, E->q);

@@ -74,3 +74,18 @@ def test_small_batch_sizes(precision, oracle):
         m._energy, m._grad = e[k], g[off[k]:off[k + 1]]
         m.getCharges = lambda: q[off[k]:off[k + 1]]
         check(m, z, x, ref, precision)
+
+
+def test_split_fragment_not_positive_definite(oracle):
+    """70 hydrogens 0.74 A apart, bonded into one chain: A and the reduced matrix
+    are indefinite (lowest eigenvalue -0.05), so the preconditioner's blocks fail
+    and the dense fallback gives the charges, as in the oracle."""
+    n = 70
+    xyz = np.zeros((n, 3))
+    xyz[:, 0] = 0.74 * np.arange(n)
+    Z = np.ones(n, dtype=np.int32)
+    m = GFNFFMethod()
+    assert m.setMolecule(Mol(Z, xyz, bonds=[(i, i + 1) for i in range(n - 1)])), m.getErrorMessage()
+    m.calculateEnergy(True)
+    assert not m.hasError(), m.getErrorMessage()
+    check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), "fp64")
