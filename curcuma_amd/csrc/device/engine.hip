@@ -66,7 +66,9 @@ constexpr double SQRTPI_TRUNC = 1.77245385091;   // constant used by the referen
 constexpr double TSQRT2PI = 0.797884560802866;
 constexpr double TSQRT2PI_SELF = 0.797884560802865;
 
-enum Flag { FLAG_CHOL = 1, FLAG_CNOVF = 2, FLAG_SOLVE = 4 };
+// FLAG_LU: the dense fallback has solved what FLAG_CHOL reports (never leaves an evaluation)
+enum Flag { FLAG_CHOL = 1, FLAG_CNOVF = 2, FLAG_SOLVE = 4, FLAG_LU = 32 };
+__host__ __device__ inline int final_flags(int f) { return f & FLAG_LU ? f & ~(FLAG_LU | FLAG_CHOL | FLAG_SOLVE) : f; }
 
 // ---------------------------------------------------------------------------
 // small helpers
@@ -103,12 +105,23 @@ __device__ void cn_atom_finish(int i, double raw, int cnt, const int* __restrict
                                double* __restrict__ gw, double* __restrict__ dgw, double* __restrict__ rhs,
                                int* __restrict__ nbn, int* __restrict__ flags);
 
-// exact bounding boxes of the 256-atom tiles of the atom order (k_cn's
-// partner tiles): bb[6 t] = (min x, min y, min z, max x, max y, max z)
-__global__ __launch_bounds__(256) void k_tile_box(int n, const double* __restrict__ x, double* __restrict__ bb) {
+// Head of an evaluation, one launch: the coordinates into the engine's buffer,
+// the status flags and the arrival counter of the energy reduction (k_finish)
+// cleared, and for a single molecule (bb != nullptr) the exact bounding boxes
+// of the 256-atom tiles of the atom order (k_cn's partner tiles):
+// bb[6 t] = (min x, min y, min z, max x, max y, max z).
+__global__ __launch_bounds__(256) void k_start(int n, const double* __restrict__ xin, double* __restrict__ x,
+                                               int* __restrict__ flags, int* __restrict__ arrived,
+                                               double* __restrict__ bb) {
     __shared__ double red[6][256];
-    const int t = blockIdx.x, tid = threadIdx.x, j = min(t * 256 + tid, n - 1);
-    const double3 p = ld3(x, j);
+    const int t = blockIdx.x, tid = threadIdx.x, e = t * 256 + tid;
+    if (e == 0) {
+        flags[0] = 0;
+        arrived[0] = 0;
+    }
+    if (e < 3 * n) x[e] = xin[e];
+    if (!bb || t * 256 >= n) return;  // uniform over the workgroup
+    const double3 p = ld3(xin, min(e, n - 1));
     red[0][tid] = p.x;
     red[1][tid] = p.y;
     red[2][tid] = p.z;
@@ -1256,6 +1269,130 @@ __device__ void bjacobi_apply(const double* __restrict__ Li, const double* rb, d
     __syncthreads();
 }
 
+// Fallback solve of a reduced EEQ system that is not positive definite
+// (FLAG_CHOL raised by the Cholesky of a diagonal block or of the matrix): the
+// reference falls back to an LU with partial pivoting of its bordered system
+// when the Cholesky of A fails (eeq_solver.cpp:2143-2165, the augmented-system
+// PartialPivLU).  The reduced system R p = b is the bordered system with the
+// constraints eliminated, so Gaussian elimination with partial pivoting on it
+// gives the same charges.  One workgroup: behind the Cholesky solve a kernel
+// that does nothing unless the flag is set and clears it when it succeeds (a
+// zero pivot keeps it: singular system); in the iterative solve the first
+// workgroup of k_eeq_pcg, which leaves the flag to the workgroups that have
+// yet to read it and raises FLAG_LU beside it.
+// R: layout 0 = packed lower 64x64 blocks (block I >= J at (I(I+1)/2 + J) 64^2,
+// row-major inside), layout 1 = row-major np x np, lower triangle used.
+// W: nr x (nr + 1) work (the system augmented with b).  nr <= LU_MAX.
+constexpr int LU_MAX = 1024;
+constexpr int LU_T = 1024;
+template <int NT>
+__device__ __noinline__ bool eeq_lu(int np, int nr, int layout, const double* __restrict__ R,
+                                    const double* __restrict__ b, double* __restrict__ W, double* __restrict__ x) {
+    __shared__ int s_piv;
+    __shared__ double s_best[NT / 64];
+    __shared__ int s_idx[NT / 64];
+    __shared__ double xs[LU_MAX];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int m = nr, ld = nr + 1;
+    for (long e = tid; e < (long)m * m; e += NT) {
+        const int i = (int)(e / m), j = (int)(e % m);
+        const int r = max(i, j), c = min(i, j);
+        double v;
+        if (layout == 0) {
+            const long I = r / NB, J = c / NB;
+            v = R[(I * (I + 1) / 2 + J) * NB * NB + (r % NB) * NB + (c % NB)];
+        } else {
+            v = R[(long)r * np + c];
+        }
+        W[(long)i * ld + j] = v;
+    }
+    for (int i = tid; i < m; i += NT) W[(long)i * ld + m] = b[i];
+    __syncthreads();
+    int ok = 1;
+    for (int k = 0; k < m; ++k) {
+        // pivot row: largest |W(i, k)| for i >= k, the lowest index on ties
+        double best = -1.0;
+        int bi = m;
+        for (int i = k + tid; i < m; i += NT) {
+            const double a = fabs(W[(long)i * ld + k]);
+            if (a > best) {
+                best = a;
+                bi = i;
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const double ob = __shfl_xor(best, o);
+            const int oi = __shfl_xor(bi, o);
+            if (ob > best || (ob == best && oi < bi)) {
+                best = ob;
+                bi = oi;
+            }
+        }
+        if (lane == 0) {
+            s_best[wv] = best;
+            s_idx[wv] = bi;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            double bb = s_best[0];
+            int ii = s_idx[0];
+            for (int w = 1; w < NT / 64; ++w)
+                if (s_best[w] > bb || (s_best[w] == bb && s_idx[w] < ii)) {
+                    bb = s_best[w];
+                    ii = s_idx[w];
+                }
+            s_piv = (bb > 0.0 && ii < m) ? ii : -1;
+        }
+        __syncthreads();
+        const int p = s_piv;
+        if (p < 0) {
+            ok = 0;
+            break;
+        }
+        if (p != k)
+            for (int j = k + tid; j <= m; j += NT) {
+                const double t = W[(long)k * ld + j];
+                W[(long)k * ld + j] = W[(long)p * ld + j];
+                W[(long)p * ld + j] = t;
+            }
+        __syncthreads();
+        const double inv = 1.0 / W[(long)k * ld + k];
+        const int cols = m - k;  // columns k+1 .. m (the last is b)
+        for (long e = tid; e < (long)(m - k - 1) * cols; e += NT) {
+            const int i = k + 1 + (int)(e / cols), j = k + 1 + (int)(e % cols);
+            W[(long)i * ld + j] -= (W[(long)i * ld + k] * inv) * W[(long)k * ld + j];
+        }
+        __syncthreads();
+    }
+    if (!ok) return false;
+    for (int i = m - 1; i >= 0; --i) {
+        double sacc = 0.0;
+        for (int j = i + 1 + tid; j < m; j += NT) sacc += W[(long)i * ld + j] * xs[j];
+        for (int o = 32; o > 0; o >>= 1) sacc += __shfl_xor(sacc, o);
+        if (lane == 0) s_best[wv] = sacc;
+        __syncthreads();
+        if (tid == 0) {
+            double t = 0.0;
+            for (int w = 0; w < NT / 64; ++w) t += s_best[w];
+            xs[i] = (W[(long)i * ld + m] - t) / W[(long)i * ld + i];
+        }
+        __syncthreads();
+    }
+    for (int i = tid; i < np; i += NT) x[i] = (i < m) ? xs[i] : 0.0;
+    return true;
+}
+
+__global__ __launch_bounds__(LU_T) void k_eeq_lu_fallback(int np, int nr, const double* __restrict__ R,
+                                                          const double* __restrict__ b, double* __restrict__ W,
+                                                          double* __restrict__ x, int* __restrict__ flags) {
+    __shared__ int s_flag;
+    if (threadIdx.x == 0) s_flag = __hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (!(s_flag & FLAG_CHOL) || nr > LU_MAX) return;
+    // the LU result replaces whatever the failed solve left (its bounded waits included)
+    if (eeq_lu<LU_T>(np, nr, 1, R, b, W, x) && threadIdx.x == 0) atomicAnd(flags, ~(FLAG_CHOL | FLAG_SOLVE));
+}
+
 // Persistent PCG on R x = b with R in packed symmetric storage: the 64x64
 // blocks (I, J), I >= J, at Rp + (I (I + 1) / 2 + J) 64^2, row-major, the
 // diagonal blocks full.  Workgroup g owns the 64-row blocks g, g + G, ... (at
@@ -1306,7 +1443,8 @@ constexpr int SM_MAXB = 1024;       // (beyond: plain diagonal blocks)
 constexpr int SM_MAXP = SM_MAXB + SM_MAXF;  // pieces: one per block and one more per fragment boundary inside a block
 
 struct PcgArgs {
-    int np, maxit;
+    int np, nr, maxit;
+    double* lu_w;        // work of the dense fallback (nullptr: nr > LU_MAX)
     double tol2;
     const double *Rp, *Lj, *b;
     double *x, *z, *pb, *part;
@@ -1385,9 +1523,13 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
     __shared__ __align__(16) double pw[PCG_WAVES][2][NB];    // per wavefront: p of the block's rows and columns
     __shared__ double sfs[SM ? SM_MAXF : 1], sig[SM ? SM_MAXF : 1], pbuf[SM ? SM_MAXP : 1];
     // a diagonal block that is not positive definite (FLAG_CHOL, set before
-    // this launch, so every workgroup reads the same value) leaves the solve to
-    // the LU fallback that follows
-    if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) return;
+    // this launch and not cleared in it, so every workgroup reads the same
+    // value) leaves the solve to the dense fallback
+    if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) {
+        if (blockIdx.x == 0 && a.lu_w && eeq_lu<PCG_THREADS>(a.np, a.nr, 0, a.Rp, a.b, a.lu_w, a.x) && threadIdx.x == 0)
+            atomicOr(a.flags, FLAG_LU);
+        return;
+    }
     const int np = a.np, G = gridDim.x, g = blockIdx.x, nbk = np / NB;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int nown = (nbk - g + G - 1) / G;
@@ -1668,154 +1810,43 @@ __global__ __launch_bounds__(256) void k_to_f32(int n, const double* __restrict_
 // ---------------------------------------------------------------------------
 // K5: charges, self energy (ff_workspace.cpp:426-449) and qtmp (:459-507)
 // ---------------------------------------------------------------------------
-// Fallback solve of a reduced EEQ system that is not positive definite
-// (FLAG_CHOL raised by the Cholesky of a diagonal block or of the matrix): the
-// reference falls back to an LU with partial pivoting of its bordered system
-// when the Cholesky of A fails (eeq_solver.cpp:2143-2165, the augmented-system
-// PartialPivLU).  The reduced system R p = b is the bordered system with the
-// constraints eliminated, so Gaussian elimination with partial pivoting on it
-// gives the same charges.  One workgroup; does nothing unless the flag is set;
-// clears FLAG_CHOL (and FLAG_SOLVE of the failed solve) when it succeeds (a
-// zero pivot keeps it: singular system).
-// R: layout 0 = packed lower 64x64 blocks (block I >= J at (I(I+1)/2 + J) 64^2,
-// row-major inside), layout 1 = row-major np x np, lower triangle used.
-// W: nr x (nr + 1) work (the system augmented with b).  nr <= LU_MAX.
-constexpr int LU_MAX = 1024;
-constexpr int LU_T = 1024;
-__global__ __launch_bounds__(LU_T) void k_eeq_lu_fallback(int np, int nr, int layout, const double* __restrict__ R,
-                                                          const double* __restrict__ b, double* __restrict__ W,
-                                                          double* __restrict__ x, int* __restrict__ flags) {
-    __shared__ int s_flag, s_piv;
-    __shared__ double s_best[LU_T / 64];
-    __shared__ int s_idx[LU_T / 64];
-    __shared__ double xs[LU_MAX];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    if (tid == 0) s_flag = __hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (!(s_flag & FLAG_CHOL) || nr > LU_MAX) return;
-    const int m = nr, ld = nr + 1;
-    for (long e = tid; e < (long)m * m; e += LU_T) {
-        const int i = (int)(e / m), j = (int)(e % m);
-        const int r = max(i, j), c = min(i, j);
-        double v;
-        if (layout == 0) {
-            const long I = r / NB, J = c / NB;
-            v = R[(I * (I + 1) / 2 + J) * NB * NB + (r % NB) * NB + (c % NB)];
-        } else {
-            v = R[(long)r * np + c];
-        }
-        W[(long)i * ld + j] = v;
-    }
-    for (int i = tid; i < m; i += LU_T) W[(long)i * ld + m] = b[i];
-    __syncthreads();
-    int ok = 1;
-    for (int k = 0; k < m; ++k) {
-        // pivot row: largest |W(i, k)| for i >= k, the lowest index on ties
-        double best = -1.0;
-        int bi = m;
-        for (int i = k + tid; i < m; i += LU_T) {
-            const double a = fabs(W[(long)i * ld + k]);
-            if (a > best) {
-                best = a;
-                bi = i;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const double ob = __shfl_xor(best, o);
-            const int oi = __shfl_xor(bi, o);
-            if (ob > best || (ob == best && oi < bi)) {
-                best = ob;
-                bi = oi;
-            }
-        }
-        if (lane == 0) {
-            s_best[wv] = best;
-            s_idx[wv] = bi;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double bb = s_best[0];
-            int ii = s_idx[0];
-            for (int w = 1; w < LU_T / 64; ++w)
-                if (s_best[w] > bb || (s_best[w] == bb && s_idx[w] < ii)) {
-                    bb = s_best[w];
-                    ii = s_idx[w];
-                }
-            s_piv = (bb > 0.0 && ii < m) ? ii : -1;
-        }
-        __syncthreads();
-        const int p = s_piv;
-        if (p < 0) {
-            ok = 0;
-            break;
-        }
-        if (p != k)
-            for (int j = k + tid; j <= m; j += LU_T) {
-                const double t = W[(long)k * ld + j];
-                W[(long)k * ld + j] = W[(long)p * ld + j];
-                W[(long)p * ld + j] = t;
-            }
-        __syncthreads();
-        const double inv = 1.0 / W[(long)k * ld + k];
-        const int cols = m - k;  // columns k+1 .. m (the last is b)
-        for (long e = tid; e < (long)(m - k - 1) * cols; e += LU_T) {
-            const int i = k + 1 + (int)(e / cols), j = k + 1 + (int)(e % cols);
-            W[(long)i * ld + j] -= (W[(long)i * ld + k] * inv) * W[(long)k * ld + j];
-        }
-        __syncthreads();
-    }
-    if (!ok) return;
-    for (int i = m - 1; i >= 0; --i) {
-        double sacc = 0.0;
-        for (int j = i + 1 + tid; j < m; j += LU_T) sacc += W[(long)i * ld + j] * xs[j];
-        for (int o = 32; o > 0; o >>= 1) sacc += __shfl_xor(sacc, o);
-        if (lane == 0) s_best[wv] = sacc;
-        __syncthreads();
-        if (tid == 0) {
-            double t = 0.0;
-            for (int w = 0; w < LU_T / 64; ++w) t += s_best[w];
-            xs[i] = (W[(long)i * ld + m] - t) / W[(long)i * ld + i];
-        }
-        __syncthreads();
-    }
-    for (int i = tid; i < np; i += LU_T) x[i] = (i < m) ? xs[i] : 0.0;
-    // the LU result replaces whatever the failed solve left (its bounded waits included)
-    if (tid == 0) atomicAnd(flags, ~(FLAG_CHOL | FLAG_SOLVE));
+// Charges from the reduced solution, one thread per atom; the last atom of a
+// fragment takes qp minus the sum over the others, formed by a wavefront per
+// fragment (workgroups natb ..: lanes stride the fragment's atoms, fixed
+// butterfly) that also finishes that atom.
+struct ChargeArgs {
+    int n, nfrag, natb;
+    const int *frag_off, *frag_atoms, *red_of;
+    const double *qp, *p, *chi_base, *cnf, *gam, *alp, *cn;
+    double *q, *e_self, *qtmp;
+};
+__device__ inline void charge_atom(const ChargeArgs& a, int i, double qi) {
+    a.q[i] = qi;
+    const double c = a.cn[i];
+    const double chi = a.chi_base[i] + a.cnf[i] * sqrt(fmax(c, 0.0));
+    a.e_self[i] = -qi * chi + 0.5 * qi * qi * (a.gam[i] + TSQRT2PI_SELF / sqrt(a.alp[i]));
+    a.qtmp[i] = qi * a.cnf[i] / (2.0 * sqrt(fmax(c, 0.0)) + 1e-16);
 }
-
-// Per fragment f, the sum of the reduced solution over its atoms (the last
-// atom's charge is qp minus it): one wavefront per fragment, lanes striding
-// the fragment's atom list, fixed butterfly.
-__global__ __launch_bounds__(256) void k_frag_sum(int nfrag, const int* __restrict__ frag_off,
-                                                  const int* __restrict__ frag_atoms, const int* __restrict__ red_of,
-                                                  const double* __restrict__ p, double* __restrict__ fsum) {
-    const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (f >= nfrag) return;
+__global__ __launch_bounds__(256) void k_charges(ChargeArgs a) {
+    if ((int)blockIdx.x < a.natb) {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (i >= a.n) return;
+        const int ri = a.red_of[i];
+        if (ri >= 0) charge_atom(a, i, a.qp[i] + a.p[ri]);
+        return;
+    }
+    const int f = (blockIdx.x - a.natb) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (f >= a.nfrag) return;
     double s = 0.0;
-    for (int k = frag_off[f] + lane; k < frag_off[f + 1]; k += 64) {
-        const int ra = red_of[frag_atoms[k]];
-        if (ra >= 0) s += p[ra];
+    for (int k = a.frag_off[f] + lane; k < a.frag_off[f + 1]; k += 64) {
+        const int ra = a.red_of[a.frag_atoms[k]];
+        if (ra >= 0) s += a.p[ra];
     }
     s = wave_sum(s);
-    if (lane == 0) fsum[f] = s;
-}
-
-__global__ __launch_bounds__(256) void k_charges(int n, const int* __restrict__ red_of,
-                                                 const double* __restrict__ fsum, const int* __restrict__ frag,
-                                                 const double* __restrict__ qp, const double* __restrict__ p,
-                                                 const double* __restrict__ chi_base, const double* __restrict__ cnf,
-                                                 const double* __restrict__ gam, const double* __restrict__ alp,
-                                                 const double* __restrict__ cn, double* __restrict__ q,
-                                                 double* __restrict__ e_self, double* __restrict__ qtmp) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int ri = red_of[i];
-    const double qi = (ri >= 0) ? qp[i] + p[ri] : qp[i] - fsum[frag[i]];  // ri < 0: last atom of its fragment
-    q[i] = qi;
-    double c = cn[i];
-    double chi = chi_base[i] + cnf[i] * sqrt(fmax(c, 0.0));
-    e_self[i] = -qi * chi + 0.5 * qi * qi * (gam[i] + TSQRT2PI_SELF / sqrt(alp[i]));
-    qtmp[i] = qi * cnf[i] / (2.0 * sqrt(fmax(c, 0.0)) + 1e-16);
+    if (lane == 0) {
+        const int i = a.frag_atoms[a.frag_off[f + 1] - 1];
+        charge_atom(a, i, a.qp[i] - s);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2420,99 +2451,18 @@ static int ps_split(int ntiles) {
     return split;
 }
 
-// Per atom a = A 64 + l: the row-side partials of tiles (A, C), C = 0 .. A,
-// then the column-side partials of tiles (R, A), R = A .. nb - 1, in that
-// order; one wavefront per block per quarter of the tiles, the four quarters
-// added in order.
-// Batches (blocks != nullptr): one workgroup per 64-atom block {a0, n, A, base}
-// of a molecule (atoms a0 .. a0 + n - 1, its tiles numbered from base).
-// part2 (nullable): a second set of tile partials (the split pair terms),
-// added tile by tile after the first.
-__global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const double* __restrict__ part,
-                                                          const double* __restrict__ part2,
-                                                          double* __restrict__ g, double* __restrict__ dEdcn,
-                                                          double* __restrict__ e_coul, double* __restrict__ e_disp,
-                                                          double* __restrict__ e_rep, const int4* __restrict__ blocks,
-                                                          int split) {
-    __shared__ double qs[4][PART_K][PS_B];
-    int A = blockIdx.x, a0 = 0, base = 0;
-    if (blocks) {
-        const int4 bb = blocks[blockIdx.x];
-        a0 = bb.x;
-        n = bb.y;
-        A = bb.z;
-        base = bb.w;
-        nb = (n + PS_B - 1) / PS_B;
-    }
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int nset = (nb + 1) * split;  // A + 1 row-side tiles and nb - A column-side tiles, split sets each
-    double s[PART_K] = {0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 2
-    for (int v = w; v < nset; v += 4) {
-        const int u = v / split, sub = v % split;
-        const bool rowside = u <= A;
-        const int Rr = u - 1;  // column side: tile (R, A), R = u - 1 = A .. nb - 1
-        const int t = base + (rowside ? A * (A + 1) / 2 + u : Rr * (Rr + 1) / 2 + A);
-        const size_t o = (((size_t)t * split + sub) * 2 + (rowside ? 0 : 1)) * PART_K * PS_B + l;
-        const double* p = part + o;
-#pragma unroll
-        for (int k = 0; k < PART_K; ++k) s[k] += p[k * PS_B];
-        if (part2) {
-#pragma unroll
-            for (int k = 0; k < PART_K; ++k) s[k] += part2[o + k * PS_B];
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < PART_K; ++k) qs[w][k][l] = s[k];
-    __syncthreads();
-    if (threadIdx.x >= PS_B || A * PS_B + (int)threadIdx.x >= n) return;
-    const int i = a0 + A * PS_B + threadIdx.x;
-    double v[PART_K];
-#pragma unroll
-    for (int k = 0; k < PART_K; ++k) v[k] = (qs[0][k][l] + qs[1][k][l]) + (qs[2][k][l] + qs[3][k][l]);
-    g[3 * i] = v[0];
-    g[3 * i + 1] = v[1];
-    g[3 * i + 2] = v[2];
-    dEdcn[i] = v[3];
-    e_coul[i] = v[4];
-    e_disp[i] = v[5];
-    e_rep[i] = v[6];
-}
-
-// Sums the j-chunk partials of k_pairs_part in chunk order.
-__global__ __launch_bounds__(256) void k_pairs_reduce(int n, int nchunk, const double* __restrict__ part,
-                                                      double* __restrict__ g, double* __restrict__ dEdcn,
-                                                      double* __restrict__ e_coul, double* __restrict__ e_disp,
-                                                      double* __restrict__ e_rep) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double acc[PART_K] = {};
-    for (int c = 0; c < nchunk; ++c) {
-        const double* p = part + (size_t)c * PART_K * n + i;
-#pragma unroll
-        for (int k = 0; k < PART_K; ++k) acc[k] += p[(size_t)k * n];
-    }
-    g[3 * i] = acc[0];
-    g[3 * i + 1] = acc[1];
-    g[3 * i + 2] = acc[2];
-    dEdcn[i] = acc[3];
-    e_coul[i] = acc[4];
-    e_disp[i] = acc[5];
-    e_rep[i] = acc[6];
-}
-
 // ---------------------------------------------------------------------------
 // K7: repulsion corrections over the topological neighbourhood
 // (gfnff_method.cpp:9781-9872: bonded pairs excluded, H-H 1,3 / 1,4 factors)
 // ---------------------------------------------------------------------------
-__device__ inline void nbrep_fix_atom(int i, const double* __restrict__ x, const int* __restrict__ Z,
+// share w of nw of atom i's neighbours: out = gradient and energy corrections
+__device__ inline void nbrep_fix_part(int i, int w, int nw, const double* __restrict__ x, const int* __restrict__ Z,
                                       const int* __restrict__ metal, const double* __restrict__ anb,
                                       const double* __restrict__ repz, const int* __restrict__ toff,
-                                      const int* __restrict__ tidx, const int* __restrict__ tdist,
-                                      double* __restrict__ g, double* __restrict__ e_rep) {
+                                      const int* __restrict__ tidx, const int* __restrict__ tdist, double out[4]) {
     double3 xi = ld3(x, i);
     double gx = 0, gy = 0, gz = 0, er = 0;
-    for (int k = toff[i]; k < toff[i + 1]; ++k) {
+    for (int k = toff[i] + w; k < toff[i + 1]; k += nw) {
         int j = tidx[k], td = tdist[k];
         int zi = Z[i], zj = Z[j];
         double fgen = rep_ff(zi, zj, metal[i], metal[j]);
@@ -2545,10 +2495,142 @@ __device__ inline void nbrep_fix_atom(int i, const double* __restrict__ x, const
         gy += s * d.y;
         gz += s * d.z;
     }
-    g[3 * i] += gx;
-    g[3 * i + 1] += gy;
-    g[3 * i + 2] += gz;
-    e_rep[i] += er;
+    out[0] = gx;
+    out[1] = gy;
+    out[2] = gz;
+    out[3] = er;
+}
+__device__ inline void nbrep_fix_atom(int i, const double* __restrict__ x, const int* __restrict__ Z,
+                                      const int* __restrict__ metal, const double* __restrict__ anb,
+                                      const double* __restrict__ repz, const int* __restrict__ toff,
+                                      const int* __restrict__ tidx, const int* __restrict__ tdist,
+                                      double* __restrict__ g, double* __restrict__ e_rep) {
+    double o[4];
+    nbrep_fix_part(i, 0, 1, x, Z, metal, anb, repz, toff, tidx, tdist, o);
+    g[3 * i] += o[0];
+    g[3 * i + 1] += o[1];
+    g[3 * i + 2] += o[2];
+    e_rep[i] += o[3];
+}
+
+// Tail of an atom after the pair terms: the repulsion corrections of its
+// topological neighbourhood (its gradient and e_rep) and its dE/dCN total
+// with the chain vector, which touch disjoint data.
+struct AtomTailArgs {
+    const double* x;
+    const int *Z, *metal;
+    const double *anb, *repz;
+    const int *toff, *tidx, *tdist;
+    double *g, *e_rep;
+    const int *doff, *didx;
+    const double* dcn_slot;
+    double* dEdcn;
+    const double* qtmp;
+    double* v;
+};
+__device__ inline void dcn_total_atom(int i, double s, const AtomTailArgs& a) {
+    for (int k = a.doff[i]; k < a.doff[i + 1]; ++k) s += a.dcn_slot[a.didx[k]];
+    a.dEdcn[i] = s;
+    a.v[i] = s - a.qtmp[i];
+}
+// one thread per atom (behind the row kernels of batches)
+__global__ __launch_bounds__(256) void k_atom_tail(int n, AtomTailArgs a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    nbrep_fix_atom(i, a.x, a.Z, a.metal, a.anb, a.repz, a.toff, a.tidx, a.tdist, a.g, a.e_rep);
+    dcn_total_atom(i, a.dEdcn[i], a);
+}
+
+// Per atom a = A 64 + l: the row-side partials of tiles (A, C), C = 0 .. A,
+// then the column-side partials of tiles (R, A), R = A .. nb - 1, in that
+// order; one wavefront per block per quarter of the tiles, the four quarters
+// added in order.
+// Batches (blocks != nullptr): one workgroup per 64-atom block {a0, n, A, base}
+// of a molecule (atoms a0 .. a0 + n - 1, its tiles numbered from base).
+// part2 (nullable): a second set of tile partials (the split pair terms),
+// added tile by tile after the first.
+// The atom's tail follows in the same launch, its neighbours dealt to the
+// four wavefronts (by one thread per atom in a launch of its own it took 15
+// us at any size: a chain of square roots and exponentials per neighbour).
+__global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const double* __restrict__ part,
+                                                          const double* __restrict__ part2,
+                                                          double* __restrict__ e_coul, double* __restrict__ e_disp,
+                                                          const int4* __restrict__ blocks, int split, AtomTailArgs at) {
+    __shared__ double qs[4][PART_K][PS_B], fs[4][4][PS_B];
+    int A = blockIdx.x, a0 = 0, base = 0;
+    if (blocks) {
+        const int4 bb = blocks[blockIdx.x];
+        a0 = bb.x;
+        n = bb.y;
+        A = bb.z;
+        base = bb.w;
+        nb = (n + PS_B - 1) / PS_B;
+    }
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nset = (nb + 1) * split;  // A + 1 row-side tiles and nb - A column-side tiles, split sets each
+    double s[PART_K] = {0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 2
+    for (int v = w; v < nset; v += 4) {
+        const int u = v / split, sub = v % split;
+        const bool rowside = u <= A;
+        const int Rr = u - 1;  // column side: tile (R, A), R = u - 1 = A .. nb - 1
+        const int t = base + (rowside ? A * (A + 1) / 2 + u : Rr * (Rr + 1) / 2 + A);
+        const size_t o = (((size_t)t * split + sub) * 2 + (rowside ? 0 : 1)) * PART_K * PS_B + l;
+        const double* p = part + o;
+#pragma unroll
+        for (int k = 0; k < PART_K; ++k) s[k] += p[k * PS_B];
+        if (part2) {
+#pragma unroll
+            for (int k = 0; k < PART_K; ++k) s[k] += part2[o + k * PS_B];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < PART_K; ++k) qs[w][k][l] = s[k];
+    {
+        double o[4] = {0, 0, 0, 0};
+        if (A * PS_B + l < n)
+            nbrep_fix_part(a0 + A * PS_B + l, w, 4, at.x, at.Z, at.metal, at.anb, at.repz, at.toff, at.tidx, at.tdist, o);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) fs[w][k][l] = o[k];
+    }
+    __syncthreads();
+    if (threadIdx.x >= PS_B || A * PS_B + (int)threadIdx.x >= n) return;
+    const int i = a0 + A * PS_B + threadIdx.x;
+    double v[PART_K];
+#pragma unroll
+    for (int k = 0; k < PART_K; ++k) v[k] = (qs[0][k][l] + qs[1][k][l]) + (qs[2][k][l] + qs[3][k][l]);
+    double c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = (fs[0][k][l] + fs[1][k][l]) + (fs[2][k][l] + fs[3][k][l]);
+    at.g[3 * i] = v[0] + c[0];
+    at.g[3 * i + 1] = v[1] + c[1];
+    at.g[3 * i + 2] = v[2] + c[2];
+    e_coul[i] = v[4];
+    e_disp[i] = v[5];
+    at.e_rep[i] = v[6] + c[3];
+    dcn_total_atom(i, v[3], at);
+}
+
+// Sums the j-chunk partials of k_pairs_part in chunk order.
+__global__ __launch_bounds__(256) void k_pairs_reduce(int n, int nchunk, const double* __restrict__ part,
+                                                      double* __restrict__ g, double* __restrict__ dEdcn,
+                                                      double* __restrict__ e_coul, double* __restrict__ e_disp,
+                                                      double* __restrict__ e_rep) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double acc[PART_K] = {};
+    for (int c = 0; c < nchunk; ++c) {
+        const double* p = part + (size_t)c * PART_K * n + i;
+#pragma unroll
+        for (int k = 0; k < PART_K; ++k) acc[k] += p[(size_t)k * n];
+    }
+    g[3 * i] = acc[0];
+    g[3 * i + 1] = acc[1];
+    g[3 * i + 2] = acc[2];
+    dEdcn[i] = acc[3];
+    e_coul[i] = acc[4];
+    e_disp[i] = acc[5];
+    e_rep[i] = acc[6];
 }
 
 // ---------------------------------------------------------------------------
@@ -4508,9 +4590,7 @@ struct MolEnergyArgs {
     const double* list_terms[11];
     double* e_mol;
 };
-__global__ __launch_bounds__(256) void k_mol_energy(MolEnergyArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
+__device__ inline void mol_energy(const MolEnergyArgs& a, int m, int lane) {
     if (m >= a.nmol) return;
     double acc = 0.0;
     for (int k = 0; k < 4; ++k)
@@ -4802,40 +4882,9 @@ __global__ __launch_bounds__(64) void k_adj_reduce(int n, int nchunk, const doub
 }
 
 // ---------------------------------------------------------------------------
-// K9: gradient assembly: slot gather, bond dE/dCN gather, CN chain rule with
-// Coulomb term 1b (ff_workspace.cpp:459-507), fixed order per atom.
+// K9: gradient assembly: CN chain rule with Coulomb term 1b
+// (ff_workspace.cpp:459-507), fixed order per atom, and the energies.
 // ---------------------------------------------------------------------------
-__device__ inline void dcn_total_atom(int i, const int* __restrict__ doff, const int* __restrict__ didx,
-                                      const double* __restrict__ dcn_slot, double* __restrict__ dEdcn,
-                                      const double* __restrict__ qtmp, double* __restrict__ v) {
-    double s = dEdcn[i];
-    for (int k = doff[i]; k < doff[i + 1]; ++k) s += dcn_slot[didx[k]];
-    dEdcn[i] = s;
-    v[i] = s - qtmp[i];
-}
-
-// Per-atom tail after the pair terms, one thread per atom: the repulsion
-// corrections of the atom's topological neighbourhood (its gradient and
-// e_rep) and its dE/dCN total with the chain vector, which touch disjoint data.
-struct AtomTailArgs {
-    const double* x;
-    const int *Z, *metal;
-    const double *anb, *repz;
-    const int *toff, *tidx, *tdist;
-    double *g, *e_rep;
-    const int *doff, *didx;
-    const double* dcn_slot;
-    double* dEdcn;
-    const double* qtmp;
-    double* v;
-};
-__global__ __launch_bounds__(256) void k_atom_tail(int n, AtomTailArgs a) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    nbrep_fix_atom(i, a.x, a.Z, a.metal, a.anb, a.repz, a.toff, a.tidx, a.tdist, a.g, a.e_rep);
-    dcn_total_atom(i, a.doff, a.didx, a.dcn_slot, a.dEdcn, a.qtmp, a.v);
-}
-
 // LPA lanes per atom (64: one wavefront; 16 for short lists, four atoms per
 // wavefront): lanes stride the atom's slot list and its CN neighbour list
 // (chain rule), fixed butterfly over the atom's lanes
@@ -4864,95 +4913,77 @@ __global__ __launch_bounds__(256) void k_slot_gather(int n, const int* __restric
     if (lane == 0) st3(gslot, i, g);
 }
 
-// CN chain rule over the atom's neighbour list plus the gathered slot, pair
-// and hydrogen-bond gradients
-template <int LPA>
-__global__ __launch_bounds__(256) void k_finish(int n, const double* __restrict__ x, const double* __restrict__ rcov,
-                                                const double* __restrict__ dlog, const double* __restrict__ v,
-                                                const int* __restrict__ nbn, const int* __restrict__ nbl,
-                                                const double* __restrict__ gslot, const double* __restrict__ gpair,
-                                                const double* __restrict__ ghb, double* __restrict__ grad) {
-    const int lane = threadIdx.x & (LPA - 1);
-    const int i = blockIdx.x * (256 / LPA) + threadIdx.x / LPA;
-    if (i >= n) return;
-    double3 g = make_double3(0, 0, 0);
-    const double3 xi = ld3(x, i);
-    const double ai = dlog[i] * v[i];
-    const int nn = nbn[i];
-    for (int k = lane; k < nn; k += LPA) {
-        int j = nbl[(size_t)i * MAXNB_CN + k];
-        double3 d = ld3(x, j) - xi;
-        double r = nrm(d);
-        double rs = rcov[i] + rcov[j];
-        double dr = (r - rs) / rs;
-        double dd = (KN / SQRTPI_TRUNC) * exp(-KN * KN * dr * dr) / rs;
-        double s = dd * (ai + dlog[j] * v[j]);
-        g = g + (-s / r) * d;
-    }
-    g.x = group_sum<LPA>(g.x);
-    g.y = group_sum<LPA>(g.y);
-    g.z = group_sum<LPA>(g.z);
-    if (lane == 0) {
-        g = g + ld3(gslot, i) + ld3(gpair, i);
-        if (ghb) g = g + ld3(ghb, i);
-        st3(grad, i, g);
-    }
-}
-
-// fixed-shape reduction of up to 16 segments into out[seg]; one workgroup
-// per segment, strided partial sums then a tree in LDS
-struct Segs {
-    const double* p[16];
-    int n[16];
-    int dst[16];
-};
+// Last launch of an evaluation, workgroups dealt to three jobs that do not
+// depend on each other:
+//  * the energies: NPARTS segments of up to RED_BLOCKS workgroups each, fixed
+//    shape; the last workgroup to arrive adds the partial sums in a fixed order
+//    and forms out[0] = total and out[1..15] = terms.  The partials are written
+//    and read with device-coherent accesses, complete before the arrival is
+//    counted, so no cache maintenance is needed;
+//  * batches: the energy of every molecule, a wavefront each;
+//  * the gradient: CN chain rule over an atom's neighbour list plus the
+//    gathered slot, pair, hydrogen-bond and solvation gradients, LPA lanes per atom.
+// Results go to the engine's buffers and to the caller's (out2, grad2).  Five
+// launches of 4.5 us each before, for 122 atoms 24 us behind the pair terms.
 constexpr int RED_BLOCKS = 64;
 constexpr int NPARTS = 16;  // energy segments reduced per evaluation
-// stage 1: segment sg, block b reduces the fixed chunk b of the segment
-__global__ __launch_bounds__(256) void k_reduce1(Segs s, double* __restrict__ part) {
+struct FinishArgs {
+    int n, nred, nmolb;  // workgroups per energy segment, and of the molecules' energies
+    const double *x, *rcov, *dlog, *v;
+    const int *nbn, *nbl;
+    const double *gslot, *gpair, *ghb, *gsolv;
+    double *grad, *grad2;
+    const double* seg[NPARTS];
+    int cnt[NPARTS];
+    double *part, *out, *out2;
+    const int* flags;
+    int *sticky, *arrived;
+    MolEnergyArgs mol;
+};
+
+__device__ void reduce_segment(const FinishArgs& a, int sg, int b) {
     __shared__ double red[256];
-    int sg = blockIdx.y, b = blockIdx.x;
-    const double* p = s.p[sg];
-    int n = s.n[sg];
-    int chunk = (n + RED_BLOCKS - 1) / RED_BLOCKS;
-    int lo = b * chunk, hi = min(n, lo + chunk);
+    __shared__ int last;
+    const double* p = a.seg[sg];
+    const int n = a.cnt[sg], nb = a.nred, tid = threadIdx.x;
+    const int chunk = (n + nb - 1) / nb;
+    const int lo = b * chunk, hi = min(n, lo + chunk);
     // eight independent partial sums per thread keep eight loads in flight
     double a8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int k = lo + threadIdx.x; k < hi; k += 8 * 256) {
+    for (int k = lo + tid; k < hi; k += 8 * 256) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const double v = p[min(k + u * 256, hi - 1)];  // unconditional load, masked add
             a8[u] += (k + u * 256 < hi) ? v : 0.0;
         }
     }
-    double acc = ((a8[0] + a8[1]) + (a8[2] + a8[3])) + ((a8[4] + a8[5]) + (a8[6] + a8[7]));
-    red[threadIdx.x] = acc;
+    red[tid] = ((a8[0] + a8[1]) + (a8[2] + a8[3])) + ((a8[4] + a8[5]) + (a8[6] + a8[7]));
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        if (tid < w) red[tid] += red[tid + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[sg * RED_BLOCKS + b] = red[0];
-}
-// stage 2 and the term table, one workgroup: wavefront sg adds segment sg's
-// block partials with a fixed tree; thread 0 then forms out[0] = total and
-// out[1..15] = terms (term index + 1) in a fixed summation order
-__global__ __launch_bounds__(NPARTS * 64) void k_reduce_final(Segs s, const double* __restrict__ part,
-                                                               double* __restrict__ parts, double* __restrict__ out,
-                                                               const int* __restrict__ flags, int* __restrict__ sticky) {
-    __shared__ double sp[NPARTS];
-    const int sg = threadIdx.x >> 6, l = threadIdx.x & 63;
-    double v = part[sg * RED_BLOCKS + l];
-    for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
-    if (l == 0) {
-        sp[s.dst[sg]] = v;
-        parts[s.dst[sg]] = v;
+    if (tid == 0) {
+        st_c(a.part + sg * RED_BLOCKS + b, red[0]);
+        wait_vm();
+        last = __hip_atomic_fetch_add(a.arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == NPARTS * nb - 1;
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
+    if (!last) return;
+    // 16 lanes per segment
+    __shared__ double sp[NPARTS];
+    {
+        const int g = tid >> 4, l = tid & 15;
+        double v = 0.0;
+        for (int k = l; k < nb; k += 16) v += ld_c(a.part + g * RED_BLOCKS + k);
+        v = group_sum<16>(v);
+        if (l == 0) sp[g] = v;
+    }
+    __syncthreads();
+    if (tid != 0) return;
     double t[GFNFF_NTERMS];
     for (int k = 0; k < GFNFF_NTERMS; ++k) t[k] = 0.0;
-    // parts: 0 bond,1 angle,2 tors,3 inv,4 disp(pairs),5 brep,6 nbrep(pairs incl fix),7 coul pairs,
+    // segments: 0 bond,1 angle,2 tors,3 inv,4 disp(pairs),5 brep,6 nbrep(pairs incl fix),7 coul pairs,
     // 8 self,9 hb case 1,10 atm,11 batm,12 triple-bond torsions,13 xb,14 hb cases 2-4,15 solvation
     t[GFNFF_E_BOND] = sp[0];
     t[GFNFF_E_ANGLE] = sp[1];
@@ -4973,32 +5004,66 @@ __global__ __launch_bounds__(NPARTS * 64) void k_reduce_final(Segs s, const doub
     // a status flag raised in this evaluation (CN list overflow, EEQ pivot,
     // solver timeout) makes the total NaN and is kept in the sticky word
     // until the host reads and clears it
-    const int f = __hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int f = final_flags(__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     if (f) {
         tot = __builtin_nan("");
-        atomicOr(sticky, f);
+        atomicOr(a.sticky, f);
     }
-    out[0] = tot;
-    for (int k = 0; k < GFNFF_NTERMS; ++k) out[1 + k] = t[k];
+    a.out[0] = tot;
+    for (int k = 0; k < GFNFF_NTERMS; ++k) a.out[1 + k] = t[k];
+    if (a.out2) {
+        a.out2[0] = tot;
+        for (int k = 0; k < GFNFF_NTERMS; ++k) a.out2[1 + k] = t[k];
+    }
+}
+
+template <int LPA>
+__global__ __launch_bounds__(256) void k_finish(FinishArgs a) {
+    int blk = blockIdx.x;
+    if (blk < NPARTS * a.nred) {
+        reduce_segment(a, blk / a.nred, blk % a.nred);
+        return;
+    }
+    blk -= NPARTS * a.nred;
+    if (blk < a.nmolb) {
+        mol_energy(a.mol, blk * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+        return;
+    }
+    blk -= a.nmolb;
+    const int lane = threadIdx.x & (LPA - 1);
+    const int i = blk * (256 / LPA) + threadIdx.x / LPA;
+    if (i >= a.n) return;
+    double3 g = make_double3(0, 0, 0);
+    const double3 xi = ld3(a.x, i);
+    const double ai = a.dlog[i] * a.v[i];
+    const int nn = a.nbn[i];
+    for (int k = lane; k < nn; k += LPA) {
+        int j = a.nbl[(size_t)i * MAXNB_CN + k];
+        double3 d = ld3(a.x, j) - xi;
+        double r = nrm(d);
+        double rs = a.rcov[i] + a.rcov[j];
+        double dr = (r - rs) / rs;
+        double dd = (KN / SQRTPI_TRUNC) * exp(-KN * KN * dr * dr) / rs;
+        double s = dd * (ai + a.dlog[j] * a.v[j]);
+        g = g + (-s / r) * d;
+    }
+    g.x = group_sum<LPA>(g.x);
+    g.y = group_sum<LPA>(g.y);
+    g.z = group_sum<LPA>(g.z);
+    if (lane == 0) {
+        g = g + ld3(a.gslot, i) + ld3(a.gpair, i);
+        if (a.ghb) g = g + ld3(a.ghb, i);
+        if (a.gsolv) g = g + ld3(a.gsolv, i);
+        st3(a.grad, i, g);
+        if (a.grad2) st3(a.grad2, i, g);
+    }
 }
 
 __global__ void k_copy(int n, const double* __restrict__ a, double* __restrict__ b) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) b[i] = a[i];
 }
-// coordinates of one evaluation into the engine's buffer; thread 0 also
-// clears the status flags (one launch at the head of the evaluation)
-__global__ void k_copy_start(int n, const double* __restrict__ a, double* __restrict__ b, int* __restrict__ flags) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) flags[0] = 0;
-    if (i < n) b[i] = a[i];
-}
 __global__ void k_fill_i(int n, int* __restrict__ a, int v) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = v;
-}
-
-__global__ void k_fill_u64(int n, unsigned long long* __restrict__ a, unsigned long long v) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = v;
 }
@@ -5390,6 +5455,7 @@ __global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ R
     double* const Rb = Rp + (I * (I + 1) / 2 + I) * NB * NB;
     double* const Li = Lj + I * NB * NB;
     const int tid = threadIdx.x;
+    for (int k = (int)I * 256 + tid; k < MB_WORDS; k += gridDim.x * 256) pa.mb[k] = MB_EMPTY;  // the solver's mailboxes
     bool any = false;
     if (nsf > 0) any = __syncthreads_or(pa.rowf[I * NB + (tid & 63)] >= 0);
     if (!any) {  // uniform over the workgroup
@@ -5559,8 +5625,9 @@ __global__ __launch_bounds__(256) void k_solv_energy(SolvArgs a, const double* _
 // Solvation gradient of atom k (one wavefront): the Born-radius chain rule
 // over all partners within lrcut, the surface terms of k's own sphere and of
 // every neighbour's sphere (k's slot in the neighbour's ascending list by
-// bisection), the direct pair gradient and the shape term; added to grad.
-__global__ __launch_bounds__(256) void k_solv_grad(SolvArgs a, double* __restrict__ grad) {
+// bisection), the direct pair gradient and the shape term, into gs (k_finish
+// adds it).
+__global__ __launch_bounds__(256) void k_solv_grad(SolvArgs a) {
     const int k = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
     if (k >= a.n) return;
     const double3 xk = ld3(a.x, k);
@@ -5612,9 +5679,9 @@ __global__ __launch_bounds__(256) void k_solv_grad(SolvArgs a, double* __restric
     const double r3 = rvk * rvk * rvk * s[14];
     const double vx = xk.x - s[2], vy = xk.y - s[3], vz = xk.z - s[4];
     const double* D = s + 15;
-    grad[3 * k] += (gx + a.gs[3 * k]) + r3 * (D[0] * vx + D[1] * vy + D[2] * vz);
-    grad[3 * k + 1] += (gy + a.gs[3 * k + 1]) + r3 * (D[3] * vx + D[4] * vy + D[5] * vz);
-    grad[3 * k + 2] += (gz + a.gs[3 * k + 2]) + r3 * (D[6] * vx + D[7] * vy + D[8] * vz);
+    a.gs[3 * k] += gx + r3 * (D[0] * vx + D[1] * vy + D[2] * vz);
+    a.gs[3 * k + 1] += gy + r3 * (D[3] * vx + D[4] * vy + D[5] * vz);
+    a.gs[3 * k + 2] += gz + r3 * (D[6] * vx + D[7] * vy + D[8] * vz);
 }
 
 inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
@@ -5758,7 +5825,6 @@ struct DeviceEngine {
     int *Z, *elem, *nref, *metal, *frag, *toff, *tidx, *tdist;
     double *chi_base, *gam, *alp, *cnf, *rcov_cn, *rcov_d3, *hb_rad, *hb_lpd, *qa, *zeta, *szr, *anb, *repz, *refcn, *c6ref;
     int *red_atom, *red_last, *red_of, *frag_off, *frag_atoms;
-    double* fsum = nullptr;  // per fragment: the reduced solution summed over its atoms
     int *red_lidx, *red_ul, *red_nul;  // distinct last atoms per 64-block of reduced variables
     double* qp;
     int *bond_ij, *bond_H, *bond_hboff, *bond_hbB, *bond_slot;
@@ -5792,8 +5858,9 @@ struct DeviceEngine {
     // work
     double *x, *cn, *dlog, *gw, *dgw, *rhs, *Ared, *Linv, *b, *rres, *q, *eself, *qtmp, *gpair, *dEdcn, *vchain,
         *slots, *dcn_slot, *grad, *e_coul, *e_disp, *e_rep, *e_bond, *e_ang, *e_tor, *e_brep, *e_hb, *e_atm,
-        *e_batm, *e_inv, *e_st, *e_xb, *parts, *rpart, *out, *diag, *ghb, *gslot, *ybuf, *xbuf, *h6, *dh6, *ppart;
+        *e_batm, *e_inv, *e_st, *e_xb, *rpart, *out, *diag, *ghb, *gslot, *ybuf, *xbuf, *h6, *dh6, *ppart;
     int *nbn, *nbl, *flags;
+    int* arrived = nullptr;  // workgroups of the energy reduction that have arrived (k_finish)
     int* sticky = nullptr;  // status flags of every evaluation since the last device_status read
     double *lu_w = nullptr, *lu_src = nullptr;  // LU fallback of a non-SPD reduced system (nr <= LU_MAX)
 
@@ -6193,7 +6260,6 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->frag_off = E->upload(foff);
         E->frag_atoms = E->upload(fatoms);
         E->qp = E->upload(qp);
-        E->fsum = E->alloc<double>(std::max(P.nfrag, 1));
 
         // term lists and gradient slots
         int slot = 0;
@@ -6593,6 +6659,8 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             }
             PcgArgs& a = E->cg;
             a.np = E->np;
+            a.nr = E->nr;
+            a.lu_w = E->lu_w;
             a.maxit = PCG_MAXIT;
             a.tol2 = E->cg_tol2;
             a.Rp = E->Ared;
@@ -6725,7 +6793,6 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->e_hb = E->alloc<double>(std::max(E->hb_ng0, 1));
         E->e_atm = E->alloc<double>(std::max(E->natm, 1));
         E->e_batm = E->alloc<double>(std::max(E->nbatm, 1));
-        E->parts = E->alloc<double>(16);
         if (P.solv.n > 0) {
             if (P.nmol != 1 || P.solv.n != n) {
                 status = kErrUnsupported;
@@ -6778,6 +6845,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->nbl = E->alloc<int>((size_t)n * MAXNB_CN);
         E->flags = E->alloc<int>(1);
         E->sticky = E->alloc<int>(1);
+        E->arrived = E->alloc<int>(1);
         E->sa.flags = E->flags;
         E->cg.flags = E->flags;
         {
@@ -7055,9 +7123,13 @@ static void queue_pairs_sym(DeviceEngine* E, hipStream_t s, const PairArgs& pa, 
     }
 }
 
-static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::string& msg) {
+// One evaluation of the coordinates xin (device-accessible) on stream s; the
+// energy terms and the gradient also go to energy_out and grad_out (nullable).
+static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, double* grad_out, hipStream_t s,
+                       std::string& msg) {
     const int n = E->n;
-    hipLaunchKernelGGL(k_copy_start, dim3(cdiv(3 * n, 256)), dim3(256), 0, s, 3 * n, xin, E->x, E->flags);
+    hipLaunchKernelGGL(k_start, dim3(cdiv(3 * n, 256)), dim3(256), 0, s, n, xin, E->x, E->flags, E->arrived,
+                       E->mol_of ? (double*)nullptr : E->tbox);
     // The reduced EEQ matrix needs only the coordinates: it is built on the
     // side stream while this stream computes CN, the EEQ right-hand side and
     // every term that does not depend on the EEQ charges; the solve waits
@@ -7086,8 +7158,6 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
             LAUNCH(KC_CHOL_DIAG, k_bjacobi_setup, dim3(nbk), dim3(256), E->side, E->Ared, E->Linv, E->flags,
                    E->cg.nsf, E->cg, E->red_atom, E->red_last, E->x, E->alp, E->diag, E->solv ? 1 : 0, E->sa, E->cg_w,
                    E->cg_w1, E->cg_all, E->cg_smon);
-            hipLaunchKernelGGL(k_fill_u64, dim3(cdiv(MB_WORDS, 256)), dim3(256), 0, E->side, MB_WORDS, E->cg_mb,
-                               MB_EMPTY);
         }
     }
     else if (E->batch_solver < 4)  // batch_solver 4 and 5 form the matrix inside their factorisations
@@ -7099,7 +7169,6 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
         queue_batch_factor(E, E->side);
         HIP_OK(hipEventRecord(E->ev_fact, E->side));
     }
-    if (!E->mol_of) LAUNCH(KC_CN, k_tile_box, dim3(cdiv(n, 256)), dim3(256), s, n, E->x, E->tbox);
     if (E->cn_by_mol)
         LAUNCH_SHM(KC_CN, k_cn_mol, dim3(E->nmol), dim3(256), (size_t)E->cn_cap * CNMOL_LDS_BYTES, s, E->cn_cap,
                    E->mol_off, E->x, E->rcov_cn, E->elem, E->nref,
@@ -7241,19 +7310,24 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
             }
         }
     }
-    if (E->lu_w)  // no work unless the system was found not positive definite
-        LAUNCH(KC_CHARGES, k_eeq_lu_fallback, dim3(1), dim3(LU_T), s, np, E->nr, E->use_cg ? 0 : 1,
-               E->use_cg ? E->Ared : (E->lu_src ? E->lu_src : E->Ared), E->b, E->lu_w, E->xbuf, E->flags);
-    LAUNCH(KC_CHARGES, k_frag_sum, dim3(cdiv(E->nfrag, 4)), dim3(256), s, E->nfrag, E->frag_off, E->frag_atoms,
-           E->red_of, E->xbuf, E->fsum);
-    LAUNCH(KC_CHARGES, k_charges, dim3(cdiv(n, 256)), dim3(256), s, n, E->red_of, E->fsum, E->frag, E->qp, E->xbuf,
-           E->chi_base, E->cnf, E->gam, E->alp, E->cn, E->q, E->eself, E->qtmp);
+    if (E->lu_w && !E->use_cg)  // no work unless the system was found not positive definite
+        LAUNCH(KC_CHARGES, k_eeq_lu_fallback, dim3(1), dim3(LU_T), s, np, E->nr,
+               E->lu_src ? E->lu_src : E->Ared, E->b, E->lu_w, E->xbuf, E->flags);
+    {
+        const int natb = cdiv(n, 256);
+        const ChargeArgs ca{n,     E->nfrag,  natb,        E->frag_off, E->frag_atoms, E->red_of, E->qp, E->xbuf,
+                            E->chi_base, E->cnf, E->gam, E->alp, E->cn, E->q, E->eself, E->qtmp};
+        LAUNCH(KC_CHARGES, k_charges, dim3(natb + cdiv(E->nfrag, 4)), dim3(256), s, ca);
+    }
     // pair terms
+    const AtomTailArgs tail{E->x,    E->Z,       E->metal,   E->anb,      E->repz,  E->toff,
+                            E->tidx, E->tdist,   E->gpair,   E->e_rep,    E->dcn_off, E->dcn_idx,
+                            E->dcn_slot, E->dEdcn, E->qtmp, E->vchain};
     if (E->ps_ntiles > 0) {  // each unordered pair once (single molecules; batches unless batch_pairs = 1)
         queue_pairs_sym(E, s, pa, E->ps_part, E->pair_split ? PT_COUL : PT_ALL);
         LAUNCH(KC_PAIRS_AUX, k_pairs_sym_reduce, dim3(E->ps_nblocks), dim3(256), s, n, E->ps_nb, E->ps_part,
-               E->pair_split ? (const double*)E->ps_part2 : nullptr,
-               E->gpair, E->dEdcn, E->e_coul, E->e_disp, E->e_rep, E->ps_blocks, E->ps_split);
+               E->pair_split ? (const double*)E->ps_part2 : nullptr, E->e_coul, E->e_disp, E->ps_blocks, E->ps_split,
+               tail);
     } else {
         const dim3 grid(cdiv(n, TILE), E->pair_nchunk);
         if (!E->mixed) {
@@ -7275,41 +7349,48 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
         }
         LAUNCH(KC_PAIRS_AUX, k_pairs_reduce, dim3(cdiv(n, 256)), dim3(256), s, n, E->pair_nchunk, E->ppart, E->gpair,
                E->dEdcn, E->e_coul, E->e_disp, E->e_rep);
-    }
-    {
-        const AtomTailArgs ta{E->x,    E->Z,       E->metal,   E->anb,      E->repz,  E->toff,
-                              E->tidx, E->tdist,   E->gpair,   E->e_rep,    E->dcn_off, E->dcn_idx,
-                              E->dcn_slot, E->dEdcn, E->qtmp, E->vchain};
-        LAUNCH(KC_CHAIN, k_atom_tail, dim3(cdiv(n, 256)), dim3(256), s, n, ta);
+        LAUNCH(KC_CHAIN, k_atom_tail, dim3(cdiv(n, 256)), dim3(256), s, n, tail);
     }
     if (split) HIP_OK(hipStreamWaitEvent(s, E->ev_join, 0));
-    if (E->fin_lpa == 64)
-        LAUNCH(KC_CHAIN, k_finish<64>, dim3(cdiv(n, 4)), dim3(256), s, n, E->x, E->rcov_cn, E->dlog, E->vchain,
-                       E->nbn, E->nbl, E->gslot, E->gpair, ghb, E->grad);
-    else
-        LAUNCH(KC_CHAIN, k_finish<16>, dim3(cdiv(n, 16)), dim3(256), s, n, E->x, E->rcov_cn, E->dlog, E->vchain,
-                       E->nbn, E->nbl, E->gslot, E->gpair, ghb, E->grad);
     if (E->solv) {
         LAUNCH(KC_SOLV, k_solv_pairs, dim3(cdiv(n, 4)), dim3(256), s, E->sa, E->q);
         LAUNCH(KC_SOLV, k_solv_energy, dim3(1), dim3(256), s, E->sa, E->q);
-        LAUNCH(KC_SOLV, k_solv_grad, dim3(cdiv(n, 4)), dim3(256), s, E->sa, E->grad);
+        LAUNCH(KC_SOLV, k_solv_grad, dim3(cdiv(n, 4)), dim3(256), s, E->sa);
     }
-    Segs sg;
+    FinishArgs fa{};
+    fa.n = n;
+    fa.x = E->x;
+    fa.rcov = E->rcov_cn;
+    fa.dlog = E->dlog;
+    fa.v = E->vchain;
+    fa.nbn = E->nbn;
+    fa.nbl = E->nbl;
+    fa.gslot = E->gslot;
+    fa.gpair = E->gpair;
+    fa.ghb = ghb;
+    fa.gsolv = E->solv ? E->sa.gs : nullptr;
+    fa.grad = E->grad;
+    fa.grad2 = grad_out;
     const double* ptrs[NPARTS] = {E->e_bond, E->e_ang,  E->e_tor, E->e_inv, E->e_disp, E->e_brep,
                                   E->e_rep,  E->e_coul, E->eself, E->e_hb,  E->e_atm,  E->e_batm,
                                   E->e_st,   E->e_xb,   E->e_hb2, E->solv ? E->sa.e_solv : E->e_bond};
-    int cnts[NPARTS] = {E->nbond, E->nangle, E->ntors, E->ninv, n, E->nbrep, n, n, n, E->hb_ng0, E->natm, E->nbatm,
-                        E->nstors, E->nxb, E->nhb2, E->solv ? 1 : 0};
+    const int cnts[NPARTS] = {E->nbond, E->nangle, E->ntors, E->ninv, n, E->nbrep, n, n, n, E->hb_ng0, E->natm,
+                              E->nbatm, E->nstors, E->nxb, E->nhb2, E->solv ? 1 : 0};
+    int most = 0;
     for (int k = 0; k < NPARTS; ++k) {
-        sg.p[k] = ptrs[k];
-        sg.n[k] = cnts[k];
-        sg.dst[k] = k;
+        fa.seg[k] = ptrs[k];
+        fa.cnt[k] = cnts[k];
+        most = std::max(most, cnts[k]);
     }
-    LAUNCH(KC_REDUCE, k_reduce1, dim3(RED_BLOCKS, NPARTS), dim3(256), s, sg, E->rpart);
-    LAUNCH(KC_REDUCE, k_reduce_final, dim3(1), dim3(NPARTS * 64), s, sg, E->rpart, E->parts, E->out, E->flags,
-           E->sticky);
+    fa.nred = std::min(RED_BLOCKS, std::max(1, cdiv(most, 1024)));
+    fa.part = E->rpart;
+    fa.out = E->out;
+    fa.out2 = energy_out;
+    fa.flags = E->flags;
+    fa.sticky = E->sticky;
+    fa.arrived = E->arrived;
     if (E->nmol > 1) {
-        MolEnergyArgs ma;
+        MolEnergyArgs& ma = fa.mol;
         ma.nmol = E->nmol;
         ma.mol_off = E->mol_off;
         ma.seg = E->mol_seg;
@@ -7321,8 +7402,13 @@ static int launch_eval(DeviceEngine* E, const double* xin, hipStream_t s, std::s
                                    E->e_batm, E->e_inv, E->e_st,  E->e_xb,   E->e_hb2};
         for (int k = 0; k < 11; ++k) ma.list_terms[k] = lists[k];
         ma.e_mol = E->e_mol;
-        LAUNCH(KC_REDUCE, k_mol_energy, dim3(cdiv(E->nmol, 4)), dim3(256), s, ma);
+        fa.nmolb = cdiv(E->nmol, 4);
     }
+    const int head = NPARTS * fa.nred + fa.nmolb;
+    if (E->fin_lpa == 64)
+        LAUNCH(KC_CHAIN, k_finish<64>, dim3(head + cdiv(n, 4)), dim3(256), s, fa);
+    else
+        LAUNCH(KC_CHAIN, k_finish<16>, dim3(head + cdiv(n, 16)), dim3(256), s, fa);
     if (hipGetLastError() != hipSuccess) {
         msg = "kernel launch failed";
         return kErrDevice;
@@ -7335,7 +7421,7 @@ int device_eval_host(DeviceEngine* E, const double* xyz_bohr, bool want_grad, do
     const int n = E->n;
     HIP_OK(hipMemcpyAsync(E->gpair, xyz_bohr, 3 * sizeof(double) * n, hipMemcpyHostToDevice, E->own));
     // gpair is overwritten by k_pairs_reduce after the copy kernel has consumed it
-    int st = launch_eval(E, E->gpair, E->own, msg);
+    int st = launch_eval(E, E->gpair, nullptr, nullptr, E->own, msg);
     if (st) return st;
     int flags = 0;
     HIP_OK(hipMemcpyAsync(e_terms, E->out, sizeof(double) * (GFNFF_NTERMS + 1), hipMemcpyDeviceToHost, E->own));
@@ -7344,6 +7430,7 @@ int device_eval_host(DeviceEngine* E, const double* xyz_bohr, bool want_grad, do
     if (q) HIP_OK(hipMemcpyAsync(q, E->q, sizeof(double) * n, hipMemcpyDeviceToHost, E->own));
     if (cn) HIP_OK(hipMemcpyAsync(cn, E->cn, sizeof(double) * n, hipMemcpyDeviceToHost, E->own));
     HIP_OK(hipStreamSynchronize(E->own));
+    flags = final_flags(flags);
     if (flags & FLAG_CHOL) {
         msg = "EEQ matrix is not positive definite on the constraint space";
         return kErrEEQ;
@@ -7362,15 +7449,7 @@ int device_eval_host(DeviceEngine* E, const double* xyz_bohr, bool want_grad, do
 int device_eval(DeviceEngine* E, const double* xyz_bohr_dev, double* energy_dev, double* grad_dev, void* stream,
                 std::string& msg) {
     hipStream_t s = (hipStream_t)stream;
-    int st = launch_eval(E, xyz_bohr_dev, s, msg);
-    if (st) return st;
-    hipLaunchKernelGGL(k_copy, dim3(1), dim3(64), 0, s, GFNFF_NTERMS + 1, E->out, energy_dev);
-    if (grad_dev) hipLaunchKernelGGL(k_copy, dim3(cdiv(3 * E->n, 256)), dim3(256), 0, s, 3 * E->n, E->grad, grad_dev);
-    if (hipGetLastError() != hipSuccess) {
-        msg = "kernel launch failed";
-        return kErrDevice;
-    }
-    return kOk;
+    return launch_eval(E, xyz_bohr_dev, energy_dev, grad_dev, s, msg);
 }
 
 // Records one device-resident evaluation with fixed buffers into a HIP graph
