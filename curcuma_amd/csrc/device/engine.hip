@@ -1161,8 +1161,9 @@ __device__ inline void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 // written: at barrier j workgroup g writes its sums to line (g, j mod 4), and
 // thread t of every workgroup polls line (t, j mod 4) and reads producer t's
 // values; every workgroup then adds the G values in the same fixed order, so
-// all hold identical sums.  A writer clears its line (g, (j + 2) mod 4), last
-// written at barrier j - 2, behind its value of barrier j: having passed
+// all hold identical sums.  (The words of all workgroups side by side were
+// slower: one line then has many writers; H-(Gly)200-OH 660 against 637 us.)
+// A writer clears its line (g, (j + 2) mod 4), last written at barrier j - 2, behind its value of barrier j: having passed
 // barrier j - 1 it has seen every workgroup's barrier j - 1 value, each
 // written after its writer finished reading barrier j - 2, so no reader still
 // needs the cleared line; and the clear completes (the wait at the head of
@@ -1244,14 +1245,16 @@ __device__ bool grid_allreduce2(double v0, double v1, double* sums, unsigned lon
 }
 
 // z_b = Linv_b^T (Linv_b r_b) for the 64-block b (r_b and the result in LDS;
-// threads 0..255 compute, every thread synchronises).
-__device__ void bjacobi_apply(const double* __restrict__ Li, const double* rb, double* wb, double* zb) {
+// threads 0..255 compute, every thread synchronises).  ld: row length of Li
+// (LDC for the copy in LDS, whose rows must not start on the same bank).
+constexpr int LDC = NB + 1;
+__device__ void bjacobi_apply(const double* __restrict__ Li, int ld, const double* rb, double* wb, double* zb) {
     const int tid = threadIdx.x, t = (tid >> 2) & 63, q = tid & 3;
     const bool act = tid < 256;
     double s = 0.0;
     if (act) {
 #pragma unroll
-        for (int u = 0; u < NB / 4; ++u) s += Li[t * NB + 4 * u + q] * rb[4 * u + q];
+        for (int u = 0; u < NB / 4; ++u) s += Li[t * ld + 4 * u + q] * rb[4 * u + q];
     }
     s += __shfl_xor(s, 1);
     s += __shfl_xor(s, 2);
@@ -1261,7 +1264,7 @@ __device__ void bjacobi_apply(const double* __restrict__ Li, const double* rb, d
     s = 0.0;
     if (act) {
 #pragma unroll
-        for (int u = 0; u < NB / 4; ++u) s += Li[(4 * u + q) * NB + t] * wb[4 * u + q];
+        for (int u = 0; u < NB / 4; ++u) s += Li[(4 * u + q) * ld + t] * wb[4 * u + q];
     }
     s += __shfl_xor(s, 1);
     s += __shfl_xor(s, 2);
@@ -1413,12 +1416,8 @@ __global__ __launch_bounds__(LU_T) void k_eeq_lu_fallback(int np, int nr, const 
 // rows of x and r, and the Linv of a single owned block, in LDS for the
 // whole solve and writes x at the end.
 //
-// RES: every wavefront has at most one block (np <= 4032 with 2048
-// wavefronts), which it loads into registers once and keeps there, with its
-// slices of p, for the whole solve: an iteration then reads only z and the
-// partials.  Otherwise the matrix streams through once per iteration; eight
-// wavefronts per workgroup (two per SIMD) let one load while the other
-// multiplies.
+// The matrix streams through once per iteration; eight wavefronts per
+// workgroup (two per SIMD) let one load while the other multiplies.
 //
 // Preconditioner.  M = D, the diagonal blocks of R, cuts a fragment of more
 // than 64 variables into pieces, and every variable of the fragment carries
@@ -1448,7 +1447,8 @@ struct PcgArgs {
     double tol2;
     const double *Rp, *Lj, *b;
     double *x, *z, *pb, *part;
-    unsigned long long* mb;
+    unsigned long long* mb;  // mailboxes; with resident blocks the exchanged vectors z, sp and part lie behind them
+    int nmb;                 // words to clear
     int *iters, *flags;
     // split fragments
     int nsf;
@@ -1483,12 +1483,65 @@ __device__ inline double tr_reduce8(const double (&v)[8], int l) {
     return (h0 ? a2[1] : a2[0]) + __shfl_xor(h0 ? a2[0] : a2[1], 1 << S);
 }
 
+// Products of one 64 x 64 block held as rv by a wavefront (see k_eeq_pcg) with
+// the p of its rows (pw[0]) and columns (pw[1]): rs = (R p_J) of row l and,
+// for an off-diagonal block, cs = (R^T p_I) of column
+// cend = 2 cg + (rg & 1) + 16 (rg >> 1), whose p is pjc.
+__device__ __forceinline__ void block_products(const double (&rv)[8][8], const double (*pw)[NB], int l, bool cols,
+                                               double& rs, double& cs, double& pjc) {
+    const int rg = l >> 3, cg = l & 7;
+    double v[8], o[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = pw[1][2 * cg + (k & 1) + 16 * (k >> 1)];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        double s = 0.0;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) s += rv[k][m] * v[m];
+        o[k] = s;
+    }
+    rs = tr_reduce8<0>(o, l);  // row 8 rg + cg = l
+    __builtin_amdgcn_sched_barrier(0);  // rows before columns: both at once do not fit the registers
+    cs = pjc = 0.0;
+    if (!cols) return;
+    pjc = pw[1][2 * cg + (rg & 1) + 16 * (rg >> 1)];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = pw[0][8 * rg + k];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        double s = 0.0;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) s += rv[m][k] * v[m];
+        o[k] = s;
+    }
+    cs = tr_reduce8<3>(o, l);
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ void load_block(double (&rv)[8][8], const double* __restrict__ R, int l) {
+    const int rg = l >> 3, cg = l & 7;
+    const double2* Rb = reinterpret_cast<const double2*>(R);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const double2 v2 = Rb[((8 * rg + i) * NB + 16 * j + 2 * cg) / 2];
+            rv[i][2 * j] = v2.x;
+            rv[i][2 * j + 1] = v2.y;
+        }
+}
+// block t of the packed lower order: t = I (I + 1) / 2 + J
+__device__ inline void packed_block(int t, int& I, int& J) {
+    I = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+    while ((long)(I + 1) * (I + 2) / 2 <= t) ++I;
+    while ((long)I * (I + 1) / 2 > t) --I;
+    J = t - I * (I + 1) / 2;
+}
+
 // sigma_f s_f of every split fragment into sfs, from the published parts;
 // returns sum_f sigma_f s_f^2 (the same in every workgroup).  sig: sigma_f.
-__device__ double sm_gather(const PcgArgs& a, int npc, double* sfs, const double* sig, double* pbuf, double* red) {
+// pbuf: the parts, in LDS.
+__device__ double sm_sums(const PcgArgs& a, double* sfs, const double* sig, const double* pbuf, double* red) {
     const int tid = threadIdx.x, l8 = tid & 7;
-    for (int k = tid; k < npc; k += PCG_THREADS) pbuf[k] = ld_c(a.sp + a.pidx[k]);
-    __syncthreads();
     double e = 0.0;
     for (int f0 = 0; f0 < a.nsf; f0 += PCG_THREADS / 8) {
         const int f = f0 + (tid >> 3);
@@ -1512,14 +1565,20 @@ __device__ double sm_gather(const PcgArgs& a, int npc, double* sfs, const double
     return t;
 }
 
-template <bool RES, bool SM>
+__device__ double sm_gather(const PcgArgs& a, int npc, double* sfs, const double* sig, double* pbuf, double* red) {
+    for (int k = threadIdx.x; k < npc; k += PCG_THREADS) pbuf[k] = ld_c(a.sp + a.pidx[k]);
+    __syncthreads();
+    return sm_sums(a, sfs, sig, pbuf, red);
+}
+
+template <bool SM>
 __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
     __shared__ double red[4 * PCG_WAVES], red2[2][PCG_WAVES];
     __shared__ double pown[PCG_MAXB][NB];
     __shared__ double qs[PCG_WAVES][NB];
     __shared__ double rb[NB], wb[NB], zb[NB];
     __shared__ double xo[PCG_MAXB][NB], ro[PCG_MAXB][NB];  // owned rows of x and r, resident for the solve
-    __shared__ double Lc[NB * NB];                          // Linv of the owned block when there is one
+    __shared__ double Lc[NB * LDC];                         // Linv of the owned block when there is one
     __shared__ __align__(16) double pw[PCG_WAVES][2][NB];    // per wavefront: p of the block's rows and columns
     __shared__ double sfs[SM ? SM_MAXF : 1], sig[SM ? SM_MAXF : 1], pbuf[SM ? SM_MAXP : 1];
     // a diagonal block that is not positive definite (FLAG_CHOL, set before
@@ -1536,30 +1595,15 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
     // this wavefront's blocks of the packed order: [t0, t1)
     const long T = (long)nbk * (nbk + 1) / 2, W = (long)PCG_WAVES * G, gw = (long)PCG_WAVES * g + wv;
     const int t0 = (int)(T * gw / W), t1 = (int)(T * (gw + 1) / W);
-    int I0 = (int)((sqrt(8.0 * t0 + 1.0) - 1.0) * 0.5);
-    while ((long)(I0 + 1) * (I0 + 2) / 2 <= t0) ++I0;
-    while ((long)I0 * (I0 + 1) / 2 > t0) --I0;
-    const int J0 = t0 - I0 * (I0 + 1) / 2;
+    int I0, J0;
+    packed_block(t0, I0, J0);
     // lane (rg, cg) holds rows 8 rg + i (i < 8) and columns 2 cg + (k & 1) + 16 (k >> 1) (k < 8) of a
     // block: every 16-byte load instruction reads whole 128-byte row segments
     const int rg = l >> 3, cg = l & 7;
     double rv[8][8];
-    auto load_block = [&](int t) {
-        const double2* Rb = reinterpret_cast<const double2*>(a.Rp + (size_t)t * NB * NB);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const double2 v2 = Rb[((8 * rg + i) * NB + 16 * j + 2 * cg) / 2];
-                rv[i][2 * j] = v2.x;
-                rv[i][2 * j + 1] = v2.y;
-            }
-    };
-    double pir = 0.0, pjr = 0.0;  // RES: p of row I0 64 + l and column J0 64 + l
-    if (RES && t1 > t0) load_block(t0);
     const bool lcache = nown == 1;
     if (lcache)
-        for (int e = tid; e < NB * NB; e += PCG_THREADS) Lc[e] = a.Lj[(size_t)g * NB * NB + e];
+        for (int e = tid; e < NB * NB; e += PCG_THREADS) Lc[(e >> 6) * LDC + (e & 63)] = a.Lj[(size_t)g * NB * NB + e];
     const int npc = SM ? a.poff[a.nsf] : 0;
     if (SM)
         for (int f = tid; f < a.nsf; f += PCG_THREADS) {
@@ -1578,7 +1622,7 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
     };
     // owners publish y = D^-1 r of a block (rb -> z) and its pieces' parts of s_f
     auto publish = [&](int kb, double& lrz, double& lrr) {
-        bjacobi_apply(lcache ? Lc : a.Lj + (size_t)kb * NB * NB, rb, wb, zb);
+        bjacobi_apply(lcache ? Lc : a.Lj + (size_t)kb * NB * NB, lcache ? LDC : NB, rb, wb, zb);
         if (tid < NB) {
             const double y = zb[tid], r = rb[tid];
             st_c(a.z + kb * NB + tid, y);
@@ -1623,55 +1667,27 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
                 const double pc = (it == 0) ? 0.0 : pown[o][tid];
                 const double pv = zrow(row) + beta * pc;
                 pown[o][tid] = pv;
-                if (!RES) st_c(pcur + row, pv);
+                st_c(pcur + row, pv);
             }
         }
         double lpq = 0.0;
         int I = I0, J = J0;
         for (int t = t0; t < t1; ++t) {
-            if (!RES) load_block(t);
-            double pil, pjl;  // p of row I * 64 + l and column J * 64 + l
-            if (RES) {
-                pjr = zrow(J * NB + l) + beta * pjr;
-                pir = zrow(I * NB + l) + beta * pir;
-                pjl = pjr;
-                pil = pir;
-            } else {
-                const double pcj = (it == 0) ? 0.0 : ld_c(pprev + J * NB + l);
-                pjl = zrow(J * NB + l) + beta * pcj;
-                const double pci = (it == 0) ? 0.0 : ld_c(pprev + I * NB + l);
-                pil = zrow(I * NB + l) + beta * pci;
-            }
+            load_block(rv, a.Rp + (size_t)t * NB * NB, l);
+            // p of row I * 64 + l and column J * 64 + l
+            const double pcj = (it == 0) ? 0.0 : ld_c(pprev + J * NB + l);
+            const double pjl = zrow(J * NB + l) + beta * pcj;
+            const double pci = (it == 0) ? 0.0 : ld_c(pprev + I * NB + l);
+            const double pil = zrow(I * NB + l) + beta * pci;
             pw[wv][0][l] = pil;
             pw[wv][1][l] = pjl;
             __builtin_amdgcn_wave_barrier();
-            double pi[8], pj[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                pi[k] = pw[wv][0][8 * rg + k];
-                pj[k] = pw[wv][1][2 * cg + (k & 1) + 16 * (k >> 1)];
-            }
-            const int cend = 2 * cg + (rg & 1) + 16 * (rg >> 1);  // the column this lane's column sum ends on
-            const double pjc = pw[wv][1][cend];
-            __builtin_amdgcn_wave_barrier();
-            double rs8[8], cs8[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                double ra = 0.0, c = 0.0;
-#pragma unroll
-                for (int m = 0; m < 8; ++m) {
-                    ra += rv[k][m] * pj[m];
-                    c += rv[m][k] * pi[m];
-                }
-                rs8[k] = ra;
-                cs8[k] = c;
-            }
-            const double rs = tr_reduce8<0>(rs8, l);  // row 8 rg + cg = l
+            double rs, cs, pjc;
+            block_products(rv, pw[wv], l, I != J, rs, cs, pjc);
             st_c(a.part + ((size_t)I * nbk + J) * NB + l, rs);
             lpq += pil * rs;
             if (I != J) {
-                const double cs = tr_reduce8<3>(cs8, l);  // column cend
-                st_c(a.part + ((size_t)J * nbk + I) * NB + cend, cs);
+                st_c(a.part + ((size_t)J * nbk + I) * NB + 2 * cg + (rg & 1) + 16 * (rg >> 1), cs);
                 lpq += pjc * cs;
             }
             if (++J > I) {
@@ -1725,6 +1741,384 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
         if (tid < NB) a.x[(g + o * G) * NB + tid] = xo[o][tid];
     if (g == 0 && tid == 0) a.iters[0] = it;
     if (!done && g == 0 && tid == 0) atomicOr(a.flags, FLAG_SOLVE);
+}
+
+// The same solve with every block resident: each wavefront holds at most one
+// block of R in registers (np <= 4032 with 2048 wavefronts) and its slices of
+// p for the whole solve, and a workgroup owns at most one row block.  An
+// iteration is then bound by the two exchanges between workgroups, each a
+// trip to memory and back, so the exchanged words carry their own arrival:
+// every word of y, of the partial products and of the parts of s_f holds
+// MB_EMPTY until it is written, and its readers poll the words they need
+// (poll_c) instead of waiting for a barrier and then reading: one trip per
+// exchange instead of three (complete the stores; flag; read).  The sums of
+// p.q, r.z and r.r go through the mailboxes of grid_allreduce2.
+// Buffers rotate over four iterations.  A writer clears the words it wrote
+// two iterations ago behind each publication: their readers have since
+// published something the writer has read (an owner's y needs the partials,
+// a partial needs its owners' y, p.q needs the parts of s_f).  The clear is
+// complete (wait_vm) before the writer's next publication, which every reader
+// reads before it polls for the one after, so no reader sees a word of four
+// iterations ago.  Measured, evaluation, against blocks resident behind full
+// barriers: 216 H2O 261 -> 240 us, H-(Gly)200-OH 726 -> 637, C300H602 650 ->
+// 590; two exchanges of about 4 us each bound an iteration.
+__device__ __forceinline__ double poll_c(const double* p, int& bad, const int* flags) {
+    const unsigned long long* u = reinterpret_cast<const unsigned long long*>(p);
+    unsigned long long v = ld_cu(u);
+    for (int it = 0; v == MB_EMPTY; ++it) {
+        if (it > SPIN_MAX ||
+            ((it & 63) == 63 && (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_SOLVE))) {
+            bad = 1;
+            return 0.0;
+        }
+        v = ld_cu(u);
+    }
+    return __longlong_as_double(v);
+}
+__device__ inline void clear_c(double* p) { st_cu(reinterpret_cast<unsigned long long*>(p), MB_EMPTY); }
+// mailbox value of exchange j (thread 0 of the workgroup)
+__device__ inline void mb_put(unsigned long long* mb, int j, double v0, double v1) {
+    unsigned long long* const own = mb + (4 * blockIdx.x + (j & 3)) * MB_LINE;
+    unsigned long long* const old = mb + (4 * blockIdx.x + ((j + 2) & 3)) * MB_LINE;
+    wait_vm();
+    st_cu(own, __double_as_longlong(v0));
+    st_cu(own + 1, __double_as_longlong(v1));
+    st_cu(old, MB_EMPTY);
+    st_cu(old + 1, MB_EMPTY);
+}
+// every workgroup's values of exchange j, summed over each of the first four
+// wavefronts into rd[w], rd[4 + w]
+__device__ inline void mb_get(const unsigned long long* mb, int j, double* rd, int& bad, const int* flags) {
+    const int tid = threadIdx.x;
+    if (tid >= 256) return;
+    double u0 = 0.0, u1 = 0.0;
+    if (tid < (int)gridDim.x) {
+        const double* in = reinterpret_cast<const double*>(mb + (4 * tid + (j & 3)) * MB_LINE);
+        u0 = poll_c(in, bad, flags);
+        u1 = poll_c(in + 1, bad, flags);
+    }
+    u0 = wave_sum(u0);
+    u1 = wave_sum(u1);
+    if ((tid & 63) == 0) {
+        rd[tid >> 6] = u0;
+        rd[4 + (tid >> 6)] = u1;
+    }
+}
+
+template <bool SM>
+__global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg_res(PcgArgs a) {
+    __shared__ double red[2][8], redq[PCG_WAVES], red2[PCG_WAVES];
+    __shared__ double qs[PCG_WAVES][NB];
+    __shared__ double rb[NB], wb[NB], zb[NB];
+    __shared__ double Lc[NB * LDC];
+    __shared__ __align__(16) double pw[PCG_WAVES][2][NB];
+    __shared__ double sfs[SM ? SM_MAXF : 1], sig[SM ? SM_MAXF : 1], pbuf[SM ? SM_MAXP : 1];
+    if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) {
+        if (blockIdx.x == 0 && a.lu_w && eeq_lu<PCG_THREADS>(a.np, a.nr, 0, a.Rp, a.b, a.lu_w, a.x) && threadIdx.x == 0)
+            atomicOr(a.flags, FLAG_LU);
+        return;
+    }
+    const int np = a.np, G = gridDim.x, g = blockIdx.x, nbk = np / NB;
+    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
+    const bool owner = g < nbk;  // of row block g
+    const int T = nbk * (nbk + 1) / 2;
+    // block of this wavefront: workgroup g takes every G-th
+    const int t = wv * G + g;
+    const bool has = t < T;
+    int I = 0, J = 0;
+    double rv[8][8];
+    if (has) {
+        packed_block(t, I, J);
+        load_block(rv, a.Rp + (size_t)t * NB * NB, l);
+    }
+    const int cend = 2 * (l & 7) + ((l >> 3) & 1) + 16 * (l >> 4);
+    const size_t pstride = (size_t)nbk * np;
+    const int npc = SM ? a.poff[a.nsf] : 0;
+    double wI = 0.0, wJ = 0.0, wO = 0.0;  // w and fragment of this lane's rows
+    int fI = -1, fJ = -1, fO = -1, s01 = 0;
+    if (SM) {
+        if (has) {
+            fI = a.rowf[I * NB + l];
+            fJ = a.rowf[J * NB + l];
+            if (fI >= 0) wI = a.w[I * NB + l];
+            if (fJ >= 0) wJ = a.w[J * NB + l];
+        }
+        if (owner) {
+            fO = a.rowf[g * NB + l];
+            if (fO >= 0) wO = a.w[g * NB + l];
+            s01 = a.smon[g];
+        }
+        for (int f = tid; f < a.nsf; f += PCG_THREADS) {
+            double s = 1.0 / a.all[f];
+            for (int k = a.poff[f]; k < a.poff[f + 1]; ++k) s += a.w1[a.pidx[k]];
+            sig[f] = 1.0 / s;
+        }
+    }
+    if (owner)
+        for (int e = tid; e < NB * NB; e += PCG_THREADS) Lc[(e >> 6) * LDC + (e & 63)] = a.Lj[(size_t)g * NB * NB + e];
+    double ro = 0.0, xo = 0.0, po = 0.0;  // the owner's rows of r, x and p (wavefront 0)
+    if (owner && tid < NB) {
+        ro = a.b[g * NB + tid];
+        rb[tid] = ro;
+    }
+    __syncthreads();
+    int nex = 0, bad = 0;  // mailbox exchanges published
+    // y of buffer k from rb, published with its parts of s_f and the sums r.y, r.r
+    auto publish = [&](int k) {
+        if (owner) bjacobi_apply(Lc, LDC, rb, wb, zb);
+        if (tid < NB) {
+            double rz = 0.0, rr = 0.0;
+            if (owner) {
+                const double y = zb[tid];
+                wait_vm();
+                st_c(a.z + (size_t)(k & 3) * np + g * NB + tid, y);
+                if (SM) {
+                    const int rf = s01 ? fO : -1;
+                    const double s0 = wave_sum(rf >= 0 && !(rf & 1) ? y : 0.0);
+                    const double s1 = wave_sum(rf >= 0 && (rf & 1) ? y : 0.0);
+                    if (tid < 2) {
+                        st_c(a.sp + (size_t)(k & 3) * 2 * nbk + 2 * g + tid, tid ? s1 : s0);
+                        clear_c(a.sp + (size_t)((k + 2) & 3) * 2 * nbk + 2 * g + tid);
+                    }
+                }
+                clear_c(a.z + (size_t)((k + 2) & 3) * np + g * NB + tid);
+                rz = wave_sum(ro * y);
+                rr = wave_sum(ro * ro);
+            }
+            if (tid == 0) mb_put(a.mb, nex, rz, rr);
+        }
+        ++nex;
+    };
+    publish(0);
+    double rzold = 1.0, pir = 0.0, pjr = 0.0, bb = 0.0;
+    int it = 0;
+    bool done = false;
+    for (;; ++it) {
+        // y of this lane's rows and columns, the parts of s_f, the sums
+        const double* yb = a.z + (size_t)(it & 3) * np;
+        double yI = 0.0, yJ = 0.0;
+        if (has) {
+            yJ = poll_c(yb + J * NB + l, bad, a.flags);
+            yI = poll_c(yb + I * NB + l, bad, a.flags);
+        }
+        if (SM)
+            for (int k = tid; k < npc; k += PCG_THREADS)
+                pbuf[k] = poll_c(a.sp + (size_t)(it & 3) * 2 * nbk + a.pidx[k], bad, a.flags);
+        mb_get(a.mb, nex - 1, red[0], bad, a.flags);
+        if (__syncthreads_or(bad)) break;
+        double rz = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+        const double rr = (red[0][4] + red[0][5]) + (red[0][6] + red[0][7]);
+        if (it == 0) {
+            bb = rr;
+            done = !(bb > 0.0);
+        } else {
+            done = rr <= a.tol2 * bb;
+        }
+        if (done || it >= a.maxit) break;
+        if (SM) {
+            rz -= sm_sums(a, sfs, sig, pbuf, red2);
+            if (fI >= 0) yI -= sfs[fI >> 1] * wI;
+            if (fJ >= 0) yJ -= sfs[fJ >> 1] * wJ;
+        }
+        const double beta = it == 0 ? 0.0 : rz / rzold;
+        rzold = rz;
+        if (owner && tid < NB) {
+            double z = zb[tid];
+            if (SM && fO >= 0) z -= sfs[fO >> 1] * wO;
+            po = z + beta * po;
+        }
+        double lpq = 0.0;
+        if (has) {
+            pjr = yJ + beta * pjr;
+            pir = yI + beta * pir;
+            pw[wv][0][l] = pir;
+            pw[wv][1][l] = pjr;
+            __builtin_amdgcn_wave_barrier();
+            double rs, cs, pjc;
+            block_products(rv, pw[wv], l, I != J, rs, cs, pjc);
+            double* const pb = a.part + (size_t)(it & 3) * pstride;
+            double* const pc = a.part + (size_t)((it + 2) & 3) * pstride;
+            wait_vm();
+            st_c(pb + ((size_t)I * nbk + J) * NB + l, rs);
+            lpq = pir * rs;
+            if (I != J) {
+                st_c(pb + ((size_t)J * nbk + I) * NB + cend, cs);
+                lpq += pjc * cs;
+                clear_c(pc + ((size_t)J * nbk + I) * NB + cend);
+            }
+            clear_c(pc + ((size_t)I * nbk + J) * NB + l);
+        }
+        lpq = wave_sum(lpq);
+        if (l == 0) redq[wv] = lpq;
+        __syncthreads();
+        if (tid == 0) {
+            double v = redq[0];
+#pragma unroll
+            for (int w = 1; w < PCG_WAVES; ++w) v += redq[w];
+            mb_put(a.mb, nex, v, 0.0);
+        }
+        ++nex;
+        // owners: the products of their rows (thread (row l, part wv): Y = wv, wv + PCG_WAVES, ..)
+        if (owner) {
+            const double* pr = a.part + (size_t)(it & 3) * pstride + (size_t)g * nbk * NB + l;
+            double t8[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t8[u] = ld_c(pr + (size_t)min(wv + PCG_WAVES * u, nbk - 1) * NB);
+            double acc = 0.0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (wv + PCG_WAVES * u < nbk) {
+                    if ((unsigned long long)__double_as_longlong(t8[u]) == MB_EMPTY)
+                        t8[u] = poll_c(pr + (size_t)(wv + PCG_WAVES * u) * NB, bad, a.flags);
+                    acc += t8[u];
+                }
+            qs[wv][l] = acc;
+        }
+        mb_get(a.mb, nex - 1, red[1], bad, a.flags);
+        if (__syncthreads_or(bad)) break;
+        if (owner) {
+            const double alpha = rz / ((red[1][0] + red[1][1]) + (red[1][2] + red[1][3]));
+            if (tid < NB) {
+                double qv = qs[0][tid];
+#pragma unroll
+                for (int w = 1; w < PCG_WAVES; ++w) qv += qs[w][tid];
+                xo += alpha * po;
+                ro -= alpha * qv;
+                rb[tid] = ro;
+            }
+            __syncthreads();
+        }
+        publish(it + 1);
+    }
+    if (owner && tid < NB) a.x[g * NB + tid] = xo;
+    if (g == 0 && tid == 0) a.iters[0] = it;
+    if (!done && tid == 0) atomicOr(a.flags, FLAG_SOLVE);
+}
+
+// And with everything in one workgroup (np <= 64 NBK_ONE): the blocks in the
+// registers of one wavefront each, vectors and factors in LDS, a barrier of
+// the workgroup where the others cross the chip.  122 atoms: 15 iterations
+// 154 -> 30 us, evaluation 297 -> 169 us.  Three row blocks fill the registers
+// and LDS of a compute unit.
+constexpr int NBK_ONE = 3;
+template <int NBK>
+__global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg_one(PcgArgs a) {
+    constexpr int NT = NBK * (NBK + 1) / 2, N = NBK * NB;
+    __shared__ double Ls[NBK][NB * LDC];
+    __shared__ double part[NBK][NBK][NB], pv[N], rvec[N], wv_[N], zv[N], redq[NT], red[2][NBK];
+    __shared__ __align__(16) double pw[NT][2][NB];
+    if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) {
+        if (a.lu_w && eeq_lu<PCG_THREADS>(a.np, a.nr, 0, a.Rp, a.b, a.lu_w, a.x) && threadIdx.x == 0)
+            atomicOr(a.flags, FLAG_LU);
+        return;
+    }
+    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
+    int I = 0, J = 0;
+    double rv[8][8];
+    if (wv < NT) {
+        packed_block(wv, I, J);
+        load_block(rv, a.Rp + (size_t)wv * NB * NB, l);
+    }
+    for (int e = tid; e < NBK * NB * NB; e += PCG_THREADS)
+        Ls[e >> 12][((e >> 6) & 63) * LDC + (e & 63)] = a.Lj[e];
+    double r = 0.0, x = 0.0, p = 0.0, z = 0.0;  // row tid
+    if (tid < N) {
+        r = a.b[tid];
+        rvec[tid] = r;
+    }
+    __syncthreads();
+    const int half = tid >> 8, t = (tid >> 2) & 63, q = tid & 3;
+    // z = M^-1 r (two blocks at a time), and the sums r.z and r.r
+    auto precond = [&](double& rz, double& rr) {
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass) {
+            const double* in = pass ? wv_ : rvec;
+            double* out = pass ? zv : wv_;
+#pragma unroll
+            for (int b0 = 0; b0 < NBK; b0 += 2) {
+                const int b = b0 + half;
+                if (b < NBK) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int u = 0; u < NB / 4; ++u)
+                        s += (pass ? Ls[b][(4 * u + q) * LDC + t] : Ls[b][t * LDC + 4 * u + q]) * in[b * NB + 4 * u + q];
+                    s += __shfl_xor(s, 1);
+                    s += __shfl_xor(s, 2);
+                    if (q == 0) out[b * NB + t] = s;
+                }
+            }
+            __syncthreads();
+        }
+        if (tid < N) {
+            z = zv[tid];
+            const double s0 = wave_sum(r * z), s1 = wave_sum(r * r);
+            if (l == 0) {
+                red[0][wv] = s0;
+                red[1][wv] = s1;
+            }
+        }
+        __syncthreads();
+        rz = red[0][0];
+        rr = red[1][0];
+#pragma unroll
+        for (int w = 1; w < NBK; ++w) {
+            rz += red[0][w];
+            rr += red[1][w];
+        }
+    };
+    double rz, bb;
+    precond(rz, bb);
+    double beta = 0.0;
+    int it = 0;
+    bool done = !(bb > 0.0);
+    for (; !done && it < a.maxit; ++it) {
+        if (tid < N) {
+            p = z + beta * p;
+            pv[tid] = p;
+        }
+        __syncthreads();
+        double lpq = 0.0;
+        if (wv < NT) {
+            const double pil = pv[I * NB + l], pjl = pv[J * NB + l];
+            pw[wv][0][l] = pil;
+            pw[wv][1][l] = pjl;
+            __builtin_amdgcn_wave_barrier();
+            double rs, cs, pjc;
+            block_products(rv, pw[wv], l, I != J, rs, cs, pjc);
+            part[I][J][l] = rs;
+            lpq = pil * rs;
+            if (I != J) {
+                part[J][I][2 * (l & 7) + ((l >> 3) & 1) + 16 * (l >> 4)] = cs;
+                lpq += pjc * cs;
+            }
+            lpq = wave_sum(lpq);
+            if (l == 0) redq[wv] = lpq;
+        }
+        __syncthreads();
+        double pq = redq[0];
+#pragma unroll
+        for (int w = 1; w < NT; ++w) pq += redq[w];
+        const double alpha = rz / pq;
+        if (tid < N) {
+            double qv = part[wv][0][l];
+#pragma unroll
+            for (int c = 1; c < NBK; ++c) qv += part[wv][c][l];
+            x += alpha * p;
+            r -= alpha * qv;
+            rvec[tid] = r;
+        }
+        __syncthreads();
+        double rz2, rr;
+        precond(rz2, rr);
+        beta = rz2 / rz;
+        rz = rz2;
+        done = rr <= a.tol2 * bb;
+    }
+    if (tid < N) a.x[tid] = x;
+    if (tid == 0) {
+        a.iters[0] = it;
+        if (!done) atomicOr(a.flags, FLAG_SOLVE);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -5455,7 +5849,7 @@ __global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ R
     double* const Rb = Rp + (I * (I + 1) / 2 + I) * NB * NB;
     double* const Li = Lj + I * NB * NB;
     const int tid = threadIdx.x;
-    for (int k = (int)I * 256 + tid; k < MB_WORDS; k += gridDim.x * 256) pa.mb[k] = MB_EMPTY;  // the solver's mailboxes
+    for (int k = (int)I * 256 + tid; k < pa.nmb; k += gridDim.x * 256) pa.mb[k] = MB_EMPTY;  // the solver's exchange buffers
     bool any = false;
     if (nsf > 0) any = __syncthreads_or(pa.rowf[I * NB + (tid & 63)] >= 0);
     if (!any) {  // uniform over the workgroup
@@ -5788,7 +6182,7 @@ struct DeviceEngine {
     unsigned long long* cg_mb = nullptr;  // all-reduce mailboxes of the persistent PCG
     int* cg_iters = nullptr;
     PcgArgs cg{};                       // k_eeq_pcg
-    bool cg_res = false;                // its blocks stay in registers
+    bool cg_res = false, cg_one = false;  // k_eeq_pcg_res, k_eeq_pcg_one
     TermArgs terms{};                   // k_terms
     double *cg_w = nullptr, *cg_w1 = nullptr, *cg_all = nullptr;
     int* cg_smon = nullptr;
@@ -6024,6 +6418,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         const double tol = pcg_tol > 0.0 ? pcg_tol : (E->mixed ? PCG_TOL_MIXED : PCG_TOL_FP64);
         E->cg_tol2 = tol * tol;
     }
+    const bool default_tol = !(pcg_tol > 0.0);
     try {
         const int n = P.n;
         E->n = n;
@@ -6599,7 +6994,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             int dev = 0, ncu = 0, per_cu = 0;
             if (hipGetDevice(&dev) != hipSuccess ||
                 hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eeq_pcg<false, true>, PCG_THREADS, 0) !=
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eeq_pcg<true>, PCG_THREADS, 0) !=
                     hipSuccess) {
                 status = kErrDevice;
                 msg = "PCG occupancy query failed";
@@ -6630,13 +7025,28 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             if (!E->use_cg && !E->mixed) E->lu_src = E->alloc<double>(E->mat_size);
         }
         if (E->use_cg) {
-            E->cg_z = E->alloc<double>(E->np);
-            E->cg_p = E->alloc<double>(2 * (size_t)E->np);
-            E->cg_part = E->alloc<double>((size_t)(E->np / NB) * E->np);
-            E->cg_mb = E->alloc<unsigned long long>(MB_WORDS);
+            const int nbk0 = E->np / NB;
+            E->cg_one = nbk0 <= NBK_ONE;
+            E->cg_res = !E->cg_one && (long)nbk0 * (nbk0 + 1) / 2 <= (long)PCG_WAVES * E->cg_groups &&
+                        E->cg_groups >= nbk0;
+            const size_t pw = (size_t)nbk0 * E->np;
+            if (E->cg_res) {
+                // mailboxes and four buffers each of y, s_f parts and partials, cleared together
+                const size_t words = MB_WORDS + 4 * ((size_t)E->np + 2 * nbk0 + pw);
+                E->cg_mb = E->alloc<unsigned long long>(words);
+                E->cg.nmb = (int)words;
+                E->cg_z = (double*)(E->cg_mb + MB_WORDS);
+                E->cg.sp = E->cg_z + 4 * (size_t)E->np;
+                E->cg_part = E->cg.sp + 8 * (size_t)nbk0;
+            } else if (!E->cg_one) {
+                E->cg_z = E->alloc<double>(E->np);
+                E->cg_p = E->alloc<double>(2 * (size_t)E->np);
+                E->cg_part = E->alloc<double>(pw);
+                E->cg_mb = E->alloc<unsigned long long>(MB_WORDS);
+                E->cg.nmb = MB_WORDS;
+            }
             E->cg_iters = E->alloc<int>(1);
             const int nbk = E->np / NB;
-            E->cg_res = (long)nbk * (nbk + 1) / 2 <= (long)PCG_WAVES * E->cg_groups;
             // split fragments: more than 64 variables, so never inside one block
             std::vector<int> rowf(E->np, -1), poff(1, 0), pidx;
             int nsf = 0;
@@ -6672,7 +7082,13 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             a.part = E->cg_part;
             a.mb = E->cg_mb;
             a.iters = E->cg_iters;
-            a.nsf = (nsf <= SM_MAXF && nbk <= SM_MAXB) ? nsf : 0;
+            a.nsf = (nsf <= SM_MAXF && nbk <= SM_MAXB && !E->cg_one) ? nsf : 0;
+            // long fragments converge by a factor of 4 in three or four iterations
+            // and are worse conditioned: there the mixed path's default stops a
+            // little later, so that its charges stay as close to the exact ones as
+            // those of the plain block-Jacobi iteration (19,360 atoms: gradient off
+            // by 1e-11 instead of 8e-11)
+            if (a.nsf > 0 && E->mixed && default_tol) a.tol2 = E->cg_tol2 * 0.09;
             if (a.nsf > 0) {
                 a.rowf = E->upload(rowf);
                 a.poff = E->upload(poff);
@@ -6681,7 +7097,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
                 a.w1 = E->cg_w1 = E->alloc<double>(2 * (size_t)nbk);
                 a.all = E->cg_all = E->alloc<double>(nsf);
                 a.smon = E->cg_smon = E->alloc<int>(nbk);
-                a.sp = E->alloc<double>(2 * (size_t)nbk);
+                if (!E->cg_res) a.sp = E->alloc<double>(2 * (size_t)nbk);
             }
         } else if (E->mixed && E->nmol > 1 && E->batch_fp32 && E->batch_solver != 2 && E->batch_solver < 4) {
             E->Ared32 = E->alloc<float>(E->mat_size);  // FP32 copies of the molecules' matrices and factors
@@ -7280,14 +7696,20 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
     } else if (E->use_cg) {
         // the persistent PCG (block-Jacobi factors and mailboxes were set up on the side stream)
         const dim3 grid(E->cg_groups), block(PCG_THREADS);
-        if (E->cg_res && E->cg.nsf)
-            LAUNCH(KC_PCG, (k_eeq_pcg<true, true>), grid, block, s, E->cg);
+        if (E->cg_one) {
+            switch (nbk) {
+                case 1: LAUNCH(KC_PCG, k_eeq_pcg_one<1>, dim3(1), block, s, E->cg); break;
+                case 2: LAUNCH(KC_PCG, k_eeq_pcg_one<2>, dim3(1), block, s, E->cg); break;
+                default: LAUNCH(KC_PCG, k_eeq_pcg_one<3>, dim3(1), block, s, E->cg); break;
+            }
+        } else if (E->cg_res && E->cg.nsf)
+            LAUNCH(KC_PCG, k_eeq_pcg_res<true>, grid, block, s, E->cg);
         else if (E->cg_res)
-            LAUNCH(KC_PCG, (k_eeq_pcg<true, false>), grid, block, s, E->cg);
+            LAUNCH(KC_PCG, k_eeq_pcg_res<false>, grid, block, s, E->cg);
         else if (E->cg.nsf)
-            LAUNCH(KC_PCG, (k_eeq_pcg<false, true>), grid, block, s, E->cg);
+            LAUNCH(KC_PCG, k_eeq_pcg<true>, grid, block, s, E->cg);
         else
-            LAUNCH(KC_PCG, (k_eeq_pcg<false, false>), grid, block, s, E->cg);
+            LAUNCH(KC_PCG, k_eeq_pcg<false>, grid, block, s, E->cg);
     } else if (!E->mixed) {
         if (E->lu_src)
             LAUNCH(KC_CHOL_DIAG, k_copy, dim3(cdiv((long)E->mat_size, 256)), dim3(256), s, (int)E->mat_size, E->Ared,

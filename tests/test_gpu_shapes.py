@@ -45,7 +45,7 @@ def check(m, Z, xyz, ref, precision):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("kind,size", [("water", 1), ("alkane", 1), ("water", 21), ("alkane", 20), ("alkane", 21),
                                        ("alkane", 42), ("alkane", 43), ("peptide", 9), ("peptide", 18), ("peptide", 27),
-                                       ("alkane", 85), ("water", 96), ("water", 97), ("peptide", 41), ("bundle", 3)])
+                                       ("alkane", 64), ("alkane", 85), ("water", 32), ("water", 33), ("water", 96), ("water", 97), ("peptide", 41), ("bundle", 3)])
 def test_single_molecule_sizes(kind, size, precision, oracle):
     Z, xyz = molecule(kind, size)
     m = GFNFFMethod(precision=precision)
@@ -86,6 +86,19 @@ def test_split_fragment_not_positive_definite(oracle):
     Z = np.ones(n, dtype=np.int32)
     m = GFNFFMethod()
     assert m.setMolecule(Mol(Z, xyz, bonds=[(i, i + 1) for i in range(n - 1)])), m.getErrorMessage()
+    m.calculateEnergy(True)
+    assert not m.hasError(), m.getErrorMessage()
+    check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), "fp64")
+
+
+@pytest.mark.parametrize("groups", [1, 5, 40])
+def test_pcg_groups_do_not_change_the_solve(groups, oracle):
+    """Bounded workgroup counts: too few for one block per wavefront stream the
+    blocks, more keep them resident (a 901-variable molecule, 120 blocks)."""
+    Z, xyz = molecule("alkane", 300)
+    m = GFNFFMethod()
+    m.setParameters({"pcg_groups": groups})
+    assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
     m.calculateEnergy(True)
     assert not m.hasError(), m.getErrorMessage()
     check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), "fp64")
