@@ -811,6 +811,147 @@ struct MfmaT<float> {
     }
 };
 
+__device__ __forceinline__ double readlane_d(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Cholesky factor and inverse factor of one 64 x 64 SPD block by a single
+// wavefront, in FP64 MFMA tiles.  With U = L^T the 16 x 16 tiles of
+// A = U^T U stay in the accumulator layout (lane (li, lk) holds elements
+// (4 v + lk, li), v < 4), in which a tile X read as the A operand of
+// v_mfma_f64_16x16x4f64 is X^T and read as the B operand is X: every product
+// of the algorithm, U_ki^T U_kj, U_kk^-T A_kj, U_kj^T V_ki and W_jj^T S
+// (V = L^-1, W_jj = U_jj^-1), has the form X^T Y and needs no data movement.
+// Only the 16 x 16 diagonal tiles are worked on element by element: lane li
+// takes column li (through LDS), pivots and rows are broadcast by readlane.
+// The four-columns-a-step form (chol_diag_block, a workgroup of 256 with two
+// barriers a step) was bound by that barrier chain, 27 us a block and 250 us
+// for 4096 of them at three workgroups per compute unit; this one has no
+// barrier, so the wavefronts of a SIMD fill each other's waits: 30 -> 16 us a
+// block alone, evaluation 166 -> 157 us (122 atoms), 4096 molecules 6.49 -> 6.16
+// ms mixed and 7.51 -> 7.13 ms FP64.
+// A: lower triangle, row-major, leading dimension ld; L is written back when
+// write_L; Linv: 64 x 64 row-major, zero above the diagonal.  buf: 16 x 17
+// doubles of LDS of the wavefront.  Returns whether every pivot was positive.
+__device__ __forceinline__ void xty(const dbl4& x, const dbl4& y, dbl4& c) {  // c += X^T Y
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c = MfmaT<double>::op(x[v], y[v], c);
+}
+// W = U^-1 of an upper 16 x 16 factor D = U^T U: on return d holds U and w W,
+// vt V = W^T, all in accumulator layout
+__device__ __forceinline__ bool chol16(dbl4& d, dbl4& w, dbl4& vt, double* buf) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    constexpr int S = 17;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) buf[(4 * v + lk) * S + li] = d[v];
+    __builtin_amdgcn_wave_barrier();
+    double a[16], iv = 0.0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = buf[r * S + li];
+    __builtin_amdgcn_wave_barrier();
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        double piv = readlane_d(a[k], k);
+        if (!(piv > 0.0)) {
+            ok = false;
+            piv = 1.0;
+        }
+        const double inv = rsqrt_nr(piv);
+        if (li == k) iv = inv;
+        a[k] = li >= k ? a[k] * inv : 0.0;  // U(k, li)
+#pragma unroll
+        for (int r = k + 1; r < 16; ++r) a[r] -= readlane_d(a[k], r) * a[k];
+    }
+    double x[16];  // column li of W
+#pragma unroll
+    for (int r = 15; r >= 0; --r) {
+        double s = li == r ? 1.0 : 0.0;
+#pragma unroll
+        for (int m = r + 1; m < 16; ++m) s -= readlane_d(a[r], m) * x[m];
+        x[r] = s * readlane_d(iv, r);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        d[v] = lk == 0 ? a[4 * v] : lk == 1 ? a[4 * v + 1] : lk == 2 ? a[4 * v + 2] : a[4 * v + 3];
+        w[v] = lk == 0 ? x[4 * v] : lk == 1 ? x[4 * v + 1] : lk == 2 ? x[4 * v + 2] : x[4 * v + 3];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) buf[(4 * v + lk) * S + li] = w[v];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) vt[v] = buf[li * S + 4 * v + lk];
+    __builtin_amdgcn_wave_barrier();
+    return ok;
+}
+__device__ __forceinline__ bool chol64_wave(double* A, int ld, double* Linv, bool write_L, double* buf) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    dbl4 U[4][4], W[4], V[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = i; j < 4; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = 16 * i + 4 * v + lk, c = 16 * j + li;
+                U[i][j][v] = A[(size_t)max(r, c) * ld + min(r, c)];
+            }
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        dbl4 vt;
+        ok = chol16(U[k][k], W[k], vt, buf) && ok;
+        V[k] = vt;
+#pragma unroll
+        for (int j = k + 1; j < 4; ++j) {
+            dbl4 t = {0.0, 0.0, 0.0, 0.0};
+            xty(W[k], U[k][j], t);
+            U[k][j] = t;
+        }
+#pragma unroll
+        for (int i = k + 1; i < 4; ++i) {
+            const dbl4 m = {-U[k][i][0], -U[k][i][1], -U[k][i][2], -U[k][i][3]};
+#pragma unroll
+            for (int j = i; j < 4; ++j) xty(m, U[k][j], U[i][j]);
+        }
+    }
+    if (write_L) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = i; j < 4; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int r = 16 * i + 4 * v + lk, c = 16 * j + li;
+                    if (r <= c) A[(size_t)c * ld + r] = U[i][j][v];
+                }
+    }
+    // V = L^-1 by block columns: V_ji = -W_jj^T sum_k U_kj^T V_ki
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        dbl4 col[4];
+        col[i] = V[i];
+#pragma unroll
+        for (int j = i + 1; j < 4; ++j) {
+            dbl4 sum = {0.0, 0.0, 0.0, 0.0}, t = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = i; k < j; ++k) xty(U[k][j], col[k], sum);
+            const dbl4 m = {-sum[0], -sum[1], -sum[2], -sum[3]};
+            xty(W[j], m, t);
+            col[j] = t;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Linv[(16 * j + 4 * v + lk) * NB + 16 * i + li] = j < i ? 0.0 : col[j][v];
+    }
+    return ok;
+}
+
 __device__ inline int xcd_tile(int b, int nb) {
     const int x = b & 7, l = b >> 3, per = nb >> 3, rem = nb & 7;
     return x * per + min(x, rem) + l;
@@ -4485,6 +4626,17 @@ __global__ __launch_bounds__(256, 3) void k_bstep_diag(const int* __restrict__ m
     chol_diag_block<T>(mnp[m], k * NB, A + mo[m], Linv + (size_t)vo[m] * NB, flags, S0, col, rdiag);
 }
 
+// the same in FP64, one wavefront per block
+__global__ __launch_bounds__(64, 2) void k_bstep_diag64(const int* __restrict__ mols, int k, const int* __restrict__ mnp,
+                                                        const long long* __restrict__ mo, const int* __restrict__ vo,
+                                                        double* __restrict__ A, double* __restrict__ Linv,
+                                                        int* __restrict__ flags) {
+    __shared__ double buf[16 * 17];
+    const int m = mols[blockIdx.x], np = mnp[m], k0 = k * NB;
+    const bool ok = chol64_wave(A + mo[m] + (size_t)k0 * np + k0, np, Linv + ((size_t)vo[m] + k0) * NB, true, buf);
+    if (!ok && threadIdx.x == 0) atomicOr(flags, FLAG_CHOL);
+}
+
 // FP64 panel tile over the whole 64-row tile in one product (the column
 // panel of the inverse read once per tile instead of once per half):
 // A(ri.., rj..) = P(ri.., 0..63) Q(0..63, 0..63)^T, P the tile itself (leading
@@ -4589,12 +4741,6 @@ __global__ __launch_bounds__(BSOLVE_T) void k_bsolve_subst(const int* __restrict
 // 2 g + 1 of the eight, MFMA step s takes column 2 g + s: a permutation of
 // the columns that both operands share), the next eight columns in flight
 // while the current ones are multiplied.
-__device__ __forceinline__ double readlane_d(double v, int l) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 
 // C = -(R - L(r0:r0+16XX, 0:K) L(j, 0:K)^T) over 16 XX rows from r0: element v
 // of block (xx, y) at row r0 + 16 xx + 4 v + lk, column 64 j + 16 y + li, read
@@ -5844,16 +5990,14 @@ __global__ __launch_bounds__(256) void k_solv_red_add(int nr, int np, const int*
 // and 1_f . w for its pieces.  A need not be positive definite where R is: a
 // block whose D fails is factored as it stands in R and takes no part in the
 // rank-one terms (smon 0).
-__global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ Rp, double* __restrict__ Lj,
+__global__ __launch_bounds__(256, 2) void k_bjacobi_setup(double* __restrict__ Rp, double* __restrict__ Lj,
                                                        int* __restrict__ flags, int nsf, PcgArgs pa,
                                                        const int* __restrict__ ra, const int* __restrict__ rl,
                                                        const double* __restrict__ x, const double* __restrict__ alp,
                                                        const double* __restrict__ diag, int solv, SolvArgs sv,
                                                        double* __restrict__ w, double* __restrict__ w1,
                                                        double* __restrict__ all, int* __restrict__ smon) {
-    __shared__ double sL[NB][NB + 1];
-    __shared__ double col[2][NB];
-    __shared__ double rdiag[NB];
+    __shared__ double buf[16 * 17], v0[2 * NB];
     __shared__ int bad;
     const size_t I = blockIdx.x;
     double* const Rb = Rp + (I * (I + 1) / 2 + I) * NB * NB;
@@ -5864,11 +6008,11 @@ __global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ R
     if (nsf > 0) any = __syncthreads_or(pa.rowf[I * NB + (tid & 63)] >= 0);
     if (!any) {  // uniform over the workgroup
         if (nsf > 0 && tid == 0) smon[I] = 0;
-        chol_diag_block<double>(NB, 0, Rb, Li, flags, sL, col, rdiag, false);
+        if (tid < 64 && !chol64_wave(Rb, NB, Li, false, buf) && tid == 0) atomicOr(flags, FLAG_CHOL);
         return;
     }
     if (tid == 0) bad = 0;
-    // D into Li, which chol_diag_block reads before it writes the inverse there
+    // D into Li, which chol64_wave reads before it writes the inverse there
     for (int e = tid; e < NB * NB; e += 256) {
         const int r = e >> 6, c = e & 63, fr = pa.rowf[I * NB + r], fc = pa.rowf[I * NB + c];
         double v;
@@ -5891,15 +6035,14 @@ __global__ __launch_bounds__(256, 3) void k_bjacobi_setup(double* __restrict__ R
         }
     }
     __syncthreads();
-    chol_diag_block<double>(NB, 0, Li, Li, &bad, sL, col, rdiag, false);
+    if (tid < 64 && !chol64_wave(Li, NB, Li, false, buf) && tid == 0) bad = 1;
     __syncthreads();
     const bool on = bad == 0;
-    if (!on) chol_diag_block<double>(NB, 0, Rb, Li, flags, sL, col, rdiag, false);
+    if (!on && tid < 64 && !chol64_wave(Rb, NB, Li, false, buf) && tid == 0) atomicOr(flags, FLAG_CHOL);
     __syncthreads();
     if (tid == 0) smon[I] = on;
     // w = L^-T (L^-1 1_f) per piece, the pieces of a block being disjoint: one
     // pass with both indicators, thread (t, q) a quarter of row t's products
-    double* const v0 = &sL[0][0];  // LDS of the factor, no longer read
     const int t = tid >> 2, q = tid & 3;
     double p0 = 0.0, p1 = 0.0;
     for (int u = 0; u < NB / 4; ++u) {
@@ -7419,6 +7562,14 @@ static void queue_solve(DeviceEngine* E, hipStream_t s, const T* A, const T* Lin
     LAUNCH(KC_TRSV, k_trsv_bwd_sweep<T>, dim3(nbk), dim3(256), s, np, A, Linv, y, x, E->ready, E->flags);
 }
 
+static void queue_diag(DeviceEngine* E, hipStream_t s, const int* mols, int nd, int k, double* A, double* Linv) {
+    LAUNCH(KC_BATCH_SOLVE, k_bstep_diag64, dim3(nd), dim3(64), s, mols, k, E->mnp, E->mmo, E->mvo, A, Linv, E->flags);
+}
+static void queue_diag(DeviceEngine* E, hipStream_t s, const int* mols, int nd, int k, float* A, float* Linv) {
+    LAUNCH(KC_BATCH_SOLVE, k_bstep_diag<float>, dim3(nd), dim3(256), s, mols, k, E->mnp, E->mmo, E->mvo, A, Linv,
+           E->flags);
+}
+
 // batch_solver 3: the per-molecule factorisations advanced one column block at
 // a time over the whole batch (three launches per step), then the
 // substitutions (and, for FP32 factors, the FP64 refinement) in one launch.
@@ -7429,8 +7580,7 @@ static void queue_batch_steps(DeviceEngine* E, hipStream_t s, T* A, T* Linv) {
         const int nd = E->bs_doff[k + 1] - E->bs_doff[k];
         const int npn = E->bs_poff[k + 1] - E->bs_poff[k];
         const int nu = E->bs_uoff[k + 1] - E->bs_uoff[k];
-        LAUNCH(KC_BATCH_SOLVE, k_bstep_diag<T>, dim3(nd), dim3(256), s, E->bs_dmols + E->bs_doff[k], k, E->mnp, E->mmo,
-               E->mvo, A, Linv, E->flags);
+        queue_diag(E, s, E->bs_dmols + E->bs_doff[k], nd, k, A, Linv);
         if (npn)
             LAUNCH(KC_BATCH_SOLVE, (k_bstep_tiles<T, false>), dim3(cdiv(npn, 4)), dim3(256), s,
                    E->bs_ptiles + E->bs_poff[k], npn, k, E->mnp, E->mmo, E->mvo, A, Linv);
@@ -7464,7 +7614,7 @@ static void queue_batch_factor(DeviceEngine* E, hipStream_t s) {
                            E->h2_ltiles[h] + E->h2_loff[h][j], nt, j, E->mnr, E->mnp, E->mmo, E->mvo, E->red_atom,
                            E->red_last, E->x, E->alp, E->diag, E->ured, E->Ared);
                 if (nd)
-                    LAUNCH(KC_BATCH_SOLVE, k_bstep_diag<double>, dim3(nd), dim3(256), st,
+                    LAUNCH(KC_BATCH_SOLVE, k_bstep_diag64, dim3(nd), dim3(64), st,
                            E->h2_dmols[h] + E->h2_doff[h][j], j, E->mnp, E->mmo, E->mvo, E->Ared, E->Linv, E->flags);
                 if (npn)
                     LAUNCH(KC_BATCH_SOLVE, (k_bstep_tiles<double, false>), dim3(cdiv(npn, 4)), dim3(256), st,
@@ -7482,7 +7632,7 @@ static void queue_batch_factor(DeviceEngine* E, hipStream_t s) {
             const int npn = E->bs_poff[j + 1] - E->bs_poff[j];
             LAUNCH(KC_BATCH_SOLVE, k_lstep_tiles, dim3(cdiv(nt, 4)), dim3(256), s, E->ls_tiles + E->ls_off[j], nt, j,
                    E->mnr, E->mnp, E->mmo, E->mvo, E->red_atom, E->red_last, E->x, E->alp, E->diag, E->ured, E->Ared);
-            LAUNCH(KC_BATCH_SOLVE, k_bstep_diag<double>, dim3(nd), dim3(256), s, E->bs_dmols + E->bs_doff[j], j,
+            LAUNCH(KC_BATCH_SOLVE, k_bstep_diag64, dim3(nd), dim3(64), s, E->bs_dmols + E->bs_doff[j], j,
                    E->mnp, E->mmo, E->mvo, E->Ared, E->Linv, E->flags);
             if (npn)
                 LAUNCH(KC_BATCH_SOLVE, (k_bstep_tiles<double, false>), dim3(cdiv(npn, 4)), dim3(256), s,
@@ -7499,7 +7649,7 @@ static void queue_batch_factor(DeviceEngine* E, hipStream_t s) {
             LAUNCH(KC_BATCH_SOLVE, k_lstep_tiles, dim3(cdiv(ndt, 4)), dim3(256), s, E->l6d_tiles + E->l6d_off[j], ndt,
                    j, E->mnr, E->mnp, E->mmo, E->mvo, E->red_atom, E->red_last, E->x, E->alp, E->diag, E->ured,
                    E->Ared);
-            LAUNCH(KC_BATCH_SOLVE, k_bstep_diag<double>, dim3(nd), dim3(256), s, E->bs_dmols + E->bs_doff[j], j,
+            LAUNCH(KC_BATCH_SOLVE, k_bstep_diag64, dim3(nd), dim3(64), s, E->bs_dmols + E->bs_doff[j], j,
                    E->mnp, E->mmo, E->mvo, E->Ared, E->Linv, E->flags);
             if (not_)
                 LAUNCH(KC_BATCH_SOLVE, k_lpanel_tiles, dim3(cdiv(not_, 4)), dim3(256), s,
