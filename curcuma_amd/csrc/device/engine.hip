@@ -3086,10 +3086,20 @@ __global__ __launch_bounds__(256) void k_atom_tail(int n, AtomTailArgs a) {
     dcn_total_atom(i, a.dEdcn[i], a);
 }
 
+// f(0) + .. + f(W - 1) in groups of four
+template <int W, class F>
+__device__ __forceinline__ double ordered_sum(F f) {
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < W; u += 4) s += (f(u) + f(u + 1)) + (f(u + 2) + f(u + 3));
+    return s;
+}
+
 // Per atom a = A 64 + l: the row-side partials of tiles (A, C), C = 0 .. A,
 // then the column-side partials of tiles (R, A), R = A .. nb - 1, in that
-// order; one wavefront per block per quarter of the tiles, the four quarters
-// added in order.
+// order, dealt to W wavefronts whose sums are added in order: W = 16 where the
+// tiles are split (few blocks, many partial sets: 512 H2O, 200 sets a block, 26
+// us with four wavefronts; evaluation 256 -> 242 us), 4 otherwise.
 // Batches (blocks != nullptr): one workgroup per 64-atom block {a0, n, A, base}
 // of a molecule (atoms a0 .. a0 + n - 1, its tiles numbered from base).
 // part2 (nullable): a second set of tile partials (the split pair terms),
@@ -3097,11 +3107,12 @@ __global__ __launch_bounds__(256) void k_atom_tail(int n, AtomTailArgs a) {
 // The atom's tail follows in the same launch, its neighbours dealt to the
 // four wavefronts (by one thread per atom in a launch of its own it took 15
 // us at any size: a chain of square roots and exponentials per neighbour).
-__global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const double* __restrict__ part,
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_pairs_sym_reduce(int n, int nb, const double* __restrict__ part,
                                                           const double* __restrict__ part2,
                                                           double* __restrict__ e_coul, double* __restrict__ e_disp,
                                                           const int4* __restrict__ blocks, int split, AtomTailArgs at) {
-    __shared__ double qs[4][PART_K][PS_B], fs[4][4][PS_B];
+    __shared__ double qs[W][PART_K][PS_B], fs[W][4][PS_B];
     int A = blockIdx.x, a0 = 0, base = 0;
     if (blocks) {
         const int4 bb = blocks[blockIdx.x];
@@ -3115,7 +3126,7 @@ __global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const d
     const int nset = (nb + 1) * split;  // A + 1 row-side tiles and nb - A column-side tiles, split sets each
     double s[PART_K] = {0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 2
-    for (int v = w; v < nset; v += 4) {
+    for (int v = w; v < nset; v += W) {
         const int u = v / split, sub = v % split;
         const bool rowside = u <= A;
         const int Rr = u - 1;  // column side: tile (R, A), R = u - 1 = A .. nb - 1
@@ -3134,7 +3145,7 @@ __global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const d
     {
         double o[4] = {0, 0, 0, 0};
         if (A * PS_B + l < n)
-            nbrep_fix_part(a0 + A * PS_B + l, w, 4, at.x, at.Z, at.metal, at.anb, at.repz, at.toff, at.tidx, at.tdist, o);
+            nbrep_fix_part(a0 + A * PS_B + l, w, W, at.x, at.Z, at.metal, at.anb, at.repz, at.toff, at.tidx, at.tdist, o);
 #pragma unroll
         for (int k = 0; k < 4; ++k) fs[w][k][l] = o[k];
     }
@@ -3143,10 +3154,10 @@ __global__ __launch_bounds__(256) void k_pairs_sym_reduce(int n, int nb, const d
     const int i = a0 + A * PS_B + threadIdx.x;
     double v[PART_K];
 #pragma unroll
-    for (int k = 0; k < PART_K; ++k) v[k] = (qs[0][k][l] + qs[1][k][l]) + (qs[2][k][l] + qs[3][k][l]);
+    for (int k = 0; k < PART_K; ++k) v[k] = ordered_sum<W>([&](int u) { return qs[u][k][l]; });
     double c[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) c[k] = (fs[0][k][l] + fs[1][k][l]) + (fs[2][k][l] + fs[3][k][l]);
+    for (int k = 0; k < 4; ++k) c[k] = ordered_sum<W>([&](int u) { return fs[u][k][l]; });
     at.g[3 * i] = v[0] + c[0];
     at.g[3 * i + 1] = v[1] + c[1];
     at.g[3 * i + 2] = v[2] + c[2];
@@ -6376,7 +6387,7 @@ struct DeviceEngine {
     double* qp;
     int *bond_ij, *bond_H, *bond_hboff, *bond_hbB, *bond_slot;
     int *bsel_hb, *bsel_plain, nb_hb, nb_plain;  // bond indices with / without HB coordination
-    int fin_lpa, hbg_lpa;                          // lanes per atom of k_finish and k_hb_gather
+    int fin_lpa, hbg_lpa, slot_lpa;                // lanes per atom of k_finish, k_hb_gather and k_slot_gather
     double* bond_par;
     int *ang_ijk, *ang_slot;
     double* ang_par;
@@ -7116,6 +7127,13 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->slot_off = E->upload(soff);
         E->fin_lpa = ((long long)soff[n] < 192LL * n) ? 16 : 64;  // lanes per atom of k_finish
         if (opt.gather_lanes) E->fin_lpa = opt.gather_lanes;
+        // the gather of the slots (and a single molecule's hydrogen bonds): a
+        // wavefront per atom also for short lists while that is at most four per
+        // SIMD, where the lists' length and not their number sets the time
+        // (216 H2O: 18 us with 16 lanes per atom; dynamics with this and the
+        // wider pair reduction 256 -> 247 us per step)
+        E->slot_lpa = E->nmol == 1 && E->nhb ? std::max(E->fin_lpa, E->hbg_lpa) : E->fin_lpa;
+        if (n <= 4096 && !opt.gather_lanes) E->slot_lpa = 64;
         E->slot_idx = E->upload(sidx);
         std::vector<int> doff(n + 1, 0), didx(2 * E->nbond);
         for (int b = 0; b < E->nbond; ++b) {
@@ -7792,7 +7810,7 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
             LAUNCH(KC_CHAIN, k_slot_gather<16>, dim3(cdiv(n, 16)), dim3(256), s, n, E->slot_off, E->slot_idx, E->slots,
                    h, E->gslot);
     };
-    if (E->nmol > 1) slot_gather(HBGather{}, E->fin_lpa);
+    if (E->nmol > 1) slot_gather(HBGather{}, E->slot_lpa);
     // pair_split: the charge-independent pair terms (dispersion, repulsion)
     // last before the solve, beside the factorisation's smaller column blocks
     if (E->pair_split) queue_pairs_sym(E, s, pa, E->ps_part2, PT_DISP | PT_REP);
@@ -7829,7 +7847,7 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
                    E->hb_ahbc, E->hb_s0, ha, E->x, E->hb_xslots, E->e_hb2);
     }
     if (E->nmol == 1)
-        slot_gather(hg, E->nhb ? std::max(E->fin_lpa, E->hbg_lpa) : E->fin_lpa);
+        slot_gather(hg, E->slot_lpa);
     else if (E->nhb) {
         if (E->hbg_lpa == 64)
             LAUNCH(KC_HB, k_hb_gather<64>, dim3(cdiv(n, 4)), dim3(256), hs, n, hg, E->ghb);
@@ -7907,9 +7925,13 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
                             E->dcn_slot, E->dEdcn, E->qtmp, E->vchain};
     if (E->ps_ntiles > 0) {  // each unordered pair once (single molecules; batches unless batch_pairs = 1)
         queue_pairs_sym(E, s, pa, E->ps_part, E->pair_split ? PT_COUL : PT_ALL);
-        LAUNCH(KC_PAIRS_AUX, k_pairs_sym_reduce, dim3(E->ps_nblocks), dim3(256), s, n, E->ps_nb, E->ps_part,
-               E->pair_split ? (const double*)E->ps_part2 : nullptr, E->e_coul, E->e_disp, E->ps_blocks, E->ps_split,
-               tail);
+        const double* part2 = E->pair_split ? E->ps_part2 : nullptr;
+        if (E->ps_split > 1)
+            LAUNCH(KC_PAIRS_AUX, k_pairs_sym_reduce<16>, dim3(E->ps_nblocks), dim3(1024), s, n, E->ps_nb, E->ps_part,
+                   part2, E->e_coul, E->e_disp, E->ps_blocks, E->ps_split, tail);
+        else
+            LAUNCH(KC_PAIRS_AUX, k_pairs_sym_reduce<4>, dim3(E->ps_nblocks), dim3(256), s, n, E->ps_nb, E->ps_part,
+                   part2, E->e_coul, E->e_disp, E->ps_blocks, E->ps_split, tail);
     } else {
         const dim3 grid(cdiv(n, TILE), E->pair_nchunk);
         if (!E->mixed) {
