@@ -5203,9 +5203,9 @@ __global__ __launch_bounds__(256) void k_adj_u(int n, const double* __restrict__
 // derivatives of the repulsion pair term e = ab exp(-al r^1.5) / r:
 //   dE'/d ln ab = E',  dE'/d al = -0.5 sqrt(r) e + 1.5 al r^2 e
 __device__ inline void rep_adj(double ab, double al, double r, double& dp_lnab, double& dp_al) {
-    const double sr = sqrt(r);
-    const double e = ab * exp(-al * r * sr) / r;
-    dp_lnab = -e / r - 1.5 * al * sr * e;
+    const double sr = sqrt(r), rinv = rcp_c(r);
+    const double e = ab * exp(-al * r * sr) * rinv;
+    dp_lnab = -e * rinv - 1.5 * al * sr * e;
     dp_al = -0.5 * sr * e + 1.5 * al * r * r * e;
 }
 
@@ -5213,12 +5213,14 @@ __device__ inline void rep_adj(double ab, double al, double r, double& dp_lnab, 
 // atom's dE/dCN share -dci sum zeta (ff_workspace_gfnff.cpp:715-767):
 __device__ inline void d4_adj(double c6, double dci, double zc, double q, double r2, double r, double& dEp_dq,
                               double& ddcn_dq) {
-    const double r0 = 0.58 * sqrt(q) + 4.80;
-    const double dr0 = 0.29 / sqrt(q);
+    const double rq = rsqrt_c(q);
+    const double r0 = 0.58 * (q * rq) + 4.80;
+    const double dr0 = 0.29 * rq;
     const double r0s = r0 * r0;
     const double r6 = r2 * r2 * r2, r06 = r0s * r0s * r0s;
-    const double t6 = 1.0 / (r6 + r06), t8 = 1.0 / (r6 * r2 + r06 * r0s);
-    const double dt6 = -t6 * t6 * 6.0 * r06 / r0 * dr0;        // d t6 / dq
+    const double p6 = r6 + r06, p8 = r6 * r2 + r06 * r0s, pi = rcp_c(p6 * p8);
+    const double t6 = p8 * pi, t8 = p6 * pi;  // 1 / p6, 1 / p8
+    const double dt6 = -t6 * t6 * 6.0 * (r0s * r0s * r0) * dr0;  // d t6 / dq
     const double dt8 = -t8 * t8 * 8.0 * r06 * r0 * dr0;        // d t8 / dq
     const double d8 = -8.0 * r2 * r2 * r2 * t8 * t8;
     const double dd6 = -6.0 * r2 * r2 * 2.0 * t6 * dt6;
@@ -5227,13 +5229,16 @@ __device__ inline void d4_adj(double c6, double dci, double zc, double q, double
     ddcn_dq = -dci * zc * (dt6 + 2.0 * t8 + 2.0 * q * dt8);
 }
 
-// Pair adjoint over full rows in j chunks (the pair kernel's decomposition).
+// Pair adjoint over full rows, the partners (all atoms, or the molecules of
+// the workgroup's rows) cut into gridDim.y chunks so that the launch has at
+// least 1024 workgroups (adj_chunks): 256 conformers, 33,700 atoms, 132 row
+// blocks, ran 432 us in one chunk on half of the chip's compute units; one
+// fitting step with this and the reduction below 2.39 -> 1.65 ms.
 // Row i collects sum_j (w_i . r_hat_ij) dE'_ij/dln(theta) + u_i d(dEdcn_i)/dln(theta)
 // for its own element and the partner's; part[chunk][k * n + i], k = p * ne + e.
 template <int NE>
 __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __restrict__ w,
-                                                    const double* __restrict__ u, int cj,
-                                                    double* __restrict__ part) {
+                                                    const double* __restrict__ u, double* __restrict__ part) {
     __shared__ double sx[TILE], sy[TILE], sz[TILE], ssz[TILE], san[TILE], srz[TILE], szt[TILE];
     __shared__ double sgw[TILE * 7];
     __shared__ int sZ[TILE], sel[TILE], smt[TILE];
@@ -5241,7 +5246,15 @@ __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __
     const int i = blockIdx.x * TILE + threadIdx.x;
     const bool act = i < n;
     int j0, j1;
-    pair_range(a, cj, j0, j1);
+    if (a.mol_of)
+        pair_range(a, a.n, j0, j1);
+    else
+        j0 = 0, j1 = n;
+    {
+        const int len = (j1 - j0 + gridDim.y - 1) / gridDim.y;
+        j0 += blockIdx.y * len;
+        j1 = min(j1, j0 + len);
+    }
     const int mlo = (a.mol_of && act) ? a.mol_off[a.mol_of[i]] : 0;
     const int mhi = (a.mol_of && act) ? a.mol_off[a.mol_of[i] + 1] : n;
     const double3 xi = act ? ld3(a.x, i) : make_double3(0, 0, 0);
@@ -5286,9 +5299,9 @@ __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __
             const double dx = xi.x - sx[jj], dy = xi.y - sy[jj], dz = xi.z - sz[jj];
             const double r2 = dx * dx + dy * dy + dz * dz;
             if (r2 > 2500.0) continue;  // beyond the D4 and repulsion cut-offs
-            const double r = sqrt(r2);
-            if (r < 1e-10) continue;
-            const double sw = (wi.x * dx + wi.y * dy + wi.z * dz) / r;
+            const double rinv = rsqrt_c(r2), r = r2 * rinv;
+            if (!(r >= 1e-10)) continue;
+            const double sw = (wi.x * dx + wi.y * dy + wi.z * dz) * rinv;
             const int ej = sel[jj];
             double dd4 = 0.0, dz_ = 0.0, da_ = 0.0;
             {   // D4 (r <= 50)
@@ -5427,19 +5440,26 @@ __global__ __launch_bounds__(256) void k_adj_brep(int nb, const int* __restrict_
     }
 }
 
-// Fixed-order reduction of the adjoint partials: one wavefront per output
-// component k; lanes stride the rows, then a fixed butterfly.
-__global__ __launch_bounds__(64) void k_adj_reduce(int n, int nchunk, const double* __restrict__ part, int nb,
-                                                   const double* __restrict__ bpart, int nk,
-                                                   double* __restrict__ out) {
-    const int k = blockIdx.x, lane = threadIdx.x;
+// Fixed-order reduction of the adjoint partials in two launches: workgroup
+// (k, b) adds share b of the rows of output component k (by one wavefront per
+// component it took 390 us for 33,700 atoms), then one wavefront per
+// component adds the shares.
+constexpr int ADJ_RB = 64;
+__global__ __launch_bounds__(256) void k_adj_reduce(int n, int nchunk, const double* __restrict__ part, int nb,
+                                                    const double* __restrict__ bpart, int nk,
+                                                    double* __restrict__ share) {
+    __shared__ double red[4];
+    const int k = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     double acc = 0.0;
     for (int c = 0; c < nchunk; ++c)
-        for (int i = lane; i < n; i += 64) acc += part[((size_t)c * nk + k) * n + i];
-    for (int b = lane; b < nb; b += 64) acc += bpart[(size_t)k * nb + b];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-    if (lane == 0) out[k] = acc;
+        for (int i = b * 256 + tid; i < n; i += ADJ_RB * 256) acc += part[((size_t)c * nk + k) * n + i];
+    for (int i = b * 256 + tid; i < nb; i += ADJ_RB * 256) acc += bpart[(size_t)k * nb + i];
+    acc = wg_sum256(acc, red);
+    if (tid == 0) share[k * ADJ_RB + b] = acc;
+}
+__global__ __launch_bounds__(64) void k_adj_final(const double* __restrict__ share, double* __restrict__ out) {
+    const double v = wave_sum(share[blockIdx.x * ADJ_RB + threadIdx.x]);
+    if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -6373,7 +6393,7 @@ struct DeviceEngine {
     int4 *l6d_tiles = nullptr, *l6o_tiles = nullptr;
     double* ured = nullptr;             // u of every reduced row (k_red_u)
     double* e_mol = nullptr;
-    double *adj_w = nullptr, *adj_u = nullptr, *adj_part = nullptr, *adj_bpart = nullptr, *adj_out = nullptr;
+    double *adj_w = nullptr, *adj_u = nullptr, *adj_part = nullptr, *adj_bpart = nullptr, *adj_share = nullptr, *adj_out = nullptr;
     float *Ared32 = nullptr, *Linv32 = nullptr, *b32 = nullptr, *y32 = nullptr, *d32 = nullptr;
     double *rvec = nullptr, *symv = nullptr;
     bool charged = false;
@@ -8221,19 +8241,26 @@ int device_update_params(DeviceEngine* E, const ParamSet& P, std::string& msg) {
     return kOk;
 }
 
+// partner chunks of the pair adjoint: at most 16, of at least 64 partners of
+// one large molecule
+static int adj_chunks(int n) {
+    const int rows = cdiv(n, TILE);
+    return std::max(1, std::min({16, cdiv(1024, rows), cdiv(n, 64)}));
+}
+
 template <int NE>
 static void queue_adjoint(DeviceEngine* E, hipStream_t s, const PairArgs& pa, double* part, double* bpart) {
     const int n = E->n;
-    const dim3 grid(cdiv(n, TILE), E->pair_nchunk);
-    hipLaunchKernelGGL(k_adj_pairs<NE>, grid, dim3(TILE), 0, s, pa, E->adj_w, E->adj_u, E->pair_cj, part);
+    const int nc = adj_chunks(n);
+    hipLaunchKernelGGL(k_adj_pairs<NE>, dim3(cdiv(n, TILE), nc), dim3(TILE), 0, s, pa, E->adj_w, E->adj_u, part);
     hipLaunchKernelGGL(k_adj_nbrep_fix<NE>, dim3(cdiv(n, 256)), dim3(256), 0, s, n, E->x, E->Z, E->metal, E->elem,
-                       E->anb, E->repz, E->toff, E->tidx, E->tdist, E->adj_w,
-                       part + (size_t)E->pair_nchunk * ADJ_P * NE * n);
+                       E->anb, E->repz, E->toff, E->tidx, E->tdist, E->adj_w, part + (size_t)nc * ADJ_P * NE * n);
     if (E->nbrep)
         hipLaunchKernelGGL(k_adj_brep<NE>, dim3(cdiv(E->nbrep, 256)), dim3(256), 0, s, E->nbrep, E->brep_ij,
                            E->brep_par, E->elem, E->x, E->adj_w, bpart);
-    hipLaunchKernelGGL(k_adj_reduce, dim3(ADJ_P * NE), dim3(64), 0, s, n, E->pair_nchunk + 1, part, E->nbrep, bpart,
-                       ADJ_P * NE, E->adj_out);
+    hipLaunchKernelGGL(k_adj_reduce, dim3(ADJ_P * NE, ADJ_RB), dim3(256), 0, s, n, nc + 1, part, E->nbrep, bpart,
+                       ADJ_P * NE, E->adj_share);
+    hipLaunchKernelGGL(k_adj_final, dim3(ADJ_P * NE), dim3(64), 0, s, E->adj_share, E->adj_out);
 }
 
 // dLoss/dln(theta) = sum_i w_i . dg_i/dln(theta) at the state of the last
@@ -8250,7 +8277,8 @@ int device_param_adjoint(DeviceEngine* E, const double* w, double* out, std::str
         try {
             E->adj_w = E->alloc<double>(3 * (size_t)n);
             E->adj_u = E->alloc<double>(n);
-            E->adj_part = E->alloc<double>((size_t)(E->pair_nchunk + 1) * ADJ_P * ne * n);
+            E->adj_part = E->alloc<double>((size_t)(adj_chunks(n) + 1) * ADJ_P * ne * n);
+            E->adj_share = E->alloc<double>(ADJ_P * ne * ADJ_RB);
             E->adj_bpart = E->alloc<double>((size_t)ADJ_P * ne * std::max(E->nbrep, 1));
             E->adj_out = E->alloc<double>(ADJ_P * ne);
         } catch (const std::bad_alloc&) {
