@@ -5815,8 +5815,8 @@ __device__ inline double born_b(const SolvArgs& a, int i, int j) {
 }
 
 // Born radii: one wavefront per atom over all partners within lrcut
-__global__ __launch_bounds__(256) void k_solv_born(SolvArgs a) {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+__device__ void solv_born(const SolvArgs& a, int blk) {
+    const int i = blk * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
     if (i >= a.n) return;  // wavefront-uniform
     const double3 xi = ld3(a.x, i);
     const double rvi = a.vdwr[i];
@@ -5847,7 +5847,17 @@ __global__ __launch_bounds__(256) void k_solv_born(SolvArgs a) {
 // compacted into LDS in ascending order; one thread per grid point forms
 // the switched product; one thread per neighbour then sums its derivative
 // over the grid points (no atomics).
-__global__ __launch_bounds__(256) void k_solv_sasa(SolvArgs a) {
+__device__ void solv_shape(const SolvArgs& a);
+// Geometry parts of one evaluation in one launch: the surface areas (a
+// workgroup per atom), then the shape descriptor, then the Born radii.
+__global__ __launch_bounds__(256) void k_solv_geom(SolvArgs a) {
+    if ((int)blockIdx.x >= a.n) {
+        if ((int)blockIdx.x == a.n)
+            solv_shape(a);
+        else
+            solv_born(a, blockIdx.x - a.n - 1);
+        return;
+    }
     __shared__ double3 nx[SOLV_NB];
     __shared__ double nlo[SOLV_NB], nhi[SOLV_NB], nsa[SOLV_NB];
     __shared__ int nj[SOLV_NB];
@@ -5946,7 +5956,7 @@ __global__ __launch_bounds__(256) void k_solv_sasa(SolvArgs a) {
 // Shape descriptor (one workgroup): the inertia tensor of spheres with the
 // van der Waals radii about their volume-weighted centre, and
 // adet = sqrt(det^(1/3) / (2/5 sum r^3)).
-__global__ __launch_bounds__(256) void k_solv_shape(SolvArgs a) {
+__device__ void solv_shape(const SolvArgs& a) {
     __shared__ double red[4];
     const int tid = threadIdx.x;
     double tr = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
@@ -5990,7 +6000,9 @@ __global__ __launch_bounds__(256) void k_solv_shape(SolvArgs a) {
 
 // Reduced Born matrix added to the reduced EEQ matrix, in the storage of
 // k_eeq_reduced (full == 0: lower triangle of the row-major matrix, 1: also
-// the upper triangle, 2: packed tiles with full diagonal tiles)
+// the upper triangle, 2: packed tiles with full diagonal tiles); gridDim.y
+// workgroups share a tile (16 entries per thread in a row took 30 us at any
+// size)
 __global__ __launch_bounds__(256) void k_solv_red_add(int nr, int np, const int* __restrict__ ra,
                                                       const int* __restrict__ rl, SolvArgs a, double* __restrict__ A,
                                                       int full) {
@@ -5999,7 +6011,7 @@ __global__ __launch_bounds__(256) void k_solv_red_add(int nr, int np, const int*
     while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
     while (bi * (bi + 1) / 2 > t) --bi;
     const int bj = t - bi * (bi + 1) / 2;
-    for (int e = threadIdx.x; e < NB * NB; e += 256) {
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < NB * NB; e += gridDim.y * 256) {
         const int rr = e >> 6, cc = e & 63, r = bi * NB + rr, c = bj * NB + cc;
         if (c > r || r >= nr || c >= nr) continue;
         const int ia = ra[r], la = rl[r], ib = ra[c], lb = rl[c];
@@ -7750,23 +7762,21 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
     // side stream while this stream computes CN, the EEQ right-hand side and
     // every term that does not depend on the EEQ charges; the solve waits
     // for both (and runs alone, as the persistent solver requires).
-    if (E->solv) {
-        // Born radii, surface areas and the shape descriptor: geometry only,
-        // ahead of the fork so that the reduced matrix can take the Born part
-        LAUNCH(KC_SOLV, k_solv_born, dim3(cdiv(n, 4)), dim3(256), s, E->sa);
-        LAUNCH(KC_SOLV, k_solv_sasa, dim3(n), dim3(256), s, E->sa);
-        LAUNCH(KC_SOLV, k_solv_shape, dim3(1), dim3(256), s, E->sa);
-    }
+    // Born radii, surface areas and shape: geometry only, and the matrix needs
+    // the radii and the hydrogen-bond weights of the surfaces, so on the side
+    // stream; a charged molecule's right-hand side needs the radii on this one
+    if (E->solv && E->charged) LAUNCH(KC_SOLV, k_solv_geom, dim3(n + 1 + cdiv(n, 4)), dim3(256), s, E->sa);
     HIP_OK(hipEventRecord(E->ev_fork, s));
     HIP_OK(hipStreamWaitEvent(E->side, E->ev_fork, 0));
     // EEQ
     const int np = E->np, nbk = np / NB;
     if (E->nmol == 1) {
+        if (E->solv && !E->charged) LAUNCH(KC_SOLV, k_solv_geom, dim3(n + 1 + cdiv(n, 4)), dim3(256), E->side, E->sa);
         LAUNCH(KC_EEQ_BUILD, k_eeq_reduced, dim3(nbk * (nbk + 1) / 2), dim3(RED_T), E->side, E->nr, np,
                E->red_atom, E->red_last, E->red_lidx, E->red_ul, E->red_nul, E->x, E->alp, E->diag, E->Ared,
                E->use_cg ? 2 : 0);
         if (E->solv)
-            LAUNCH(KC_SOLV, k_solv_red_add, dim3(nbk * (nbk + 1) / 2), dim3(256), E->side, E->nr, np, E->red_atom,
+            LAUNCH(KC_SOLV, k_solv_red_add, dim3(nbk * (nbk + 1) / 2, 8), dim3(256), E->side, E->nr, np, E->red_atom,
                    E->red_last, E->sa, E->Ared, E->use_cg ? 2 : 0);
         if (E->use_cg) {
             // block-Jacobi factors of R's diagonal blocks and the solver's
@@ -7941,6 +7951,16 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
                             E->chi_base, E->cnf, E->gam, E->alp, E->cn, E->q, E->eself, E->qtmp};
         LAUNCH(KC_CHARGES, k_charges, dim3(natb + cdiv(E->nfrag, 4)), dim3(256), s, ca);
     }
+    if (E->solv) {
+        // the solvation terms need the charges and what the side stream holds:
+        // there, beside the pair terms, joined before k_finish
+        HIP_OK(hipEventRecord(E->ev_fork, s));
+        HIP_OK(hipStreamWaitEvent(E->side, E->ev_fork, 0));
+        LAUNCH(KC_SOLV, k_solv_pairs, dim3(cdiv(n, 4)), dim3(256), E->side, E->sa, E->q);
+        LAUNCH(KC_SOLV, k_solv_energy, dim3(1), dim3(256), E->side, E->sa, E->q);
+        LAUNCH(KC_SOLV, k_solv_grad, dim3(cdiv(n, 4)), dim3(256), E->side, E->sa);
+        HIP_OK(hipEventRecord(E->ev_join, E->side));
+    }
     // pair terms
     const AtomTailArgs tail{E->x,    E->Z,       E->metal,   E->anb,      E->repz,  E->toff,
                             E->tidx, E->tdist,   E->gpair,   E->e_rep,    E->dcn_off, E->dcn_idx,
@@ -7977,12 +7997,7 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
                E->dEdcn, E->e_coul, E->e_disp, E->e_rep);
         LAUNCH(KC_CHAIN, k_atom_tail, dim3(cdiv(n, 256)), dim3(256), s, n, tail);
     }
-    if (split) HIP_OK(hipStreamWaitEvent(s, E->ev_join, 0));
-    if (E->solv) {
-        LAUNCH(KC_SOLV, k_solv_pairs, dim3(cdiv(n, 4)), dim3(256), s, E->sa, E->q);
-        LAUNCH(KC_SOLV, k_solv_energy, dim3(1), dim3(256), s, E->sa, E->q);
-        LAUNCH(KC_SOLV, k_solv_grad, dim3(cdiv(n, 4)), dim3(256), s, E->sa);
-    }
+    if (split || E->solv) HIP_OK(hipStreamWaitEvent(s, E->ev_join, 0));
     FinishArgs fa{};
     fa.n = n;
     fa.x = E->x;
