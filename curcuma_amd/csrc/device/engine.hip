@@ -1278,6 +1278,9 @@ __global__ __launch_bounds__(256) void k_trsv_bwd_sweep(int np, const T* __restr
 // ---------------------------------------------------------------------------
 constexpr int PCG_THREADS = 512;
 constexpr int PCG_WAVES = PCG_THREADS / 64;
+constexpr int PCGS_THREADS = 256;  // the streaming form, k_eeq_pcg
+constexpr int PCGS_WAVES = PCGS_THREADS / 64;
+constexpr int PCGS_PP = 8;  // from this many blocks per wavefront on, two register buffers stream in turn
 
 // Sum over the 64 lanes of a wavefront (fixed butterfly; every lane gets it).
 __device__ inline double wave_sum(double v) {
@@ -1337,35 +1340,39 @@ constexpr unsigned long long MB_EMPTY = 0x7ff0deadbeef0001ull;
 constexpr int MB_LINE = 16;                  // 64-bit words per 128-byte line
 constexpr int MB_WORDS = 4 * 256 * MB_LINE;  // lines (g, k), k < 4, at (4 g + k) MB_LINE
 
-// red: 4 PCG_WAVES doubles of LDS, used in halves by the barrier's parity, so
+// between: issued behind the publication and ahead of the polls (loads whose
+// latency the barrier covers; ahead of the publication they would delay it).
+// red: 4 PCGS_WAVES doubles of LDS, used in halves by the barrier's parity, so
 // that a barrier writes the half that was last read before the barrier ahead
 // of it.
-__device__ bool grid_allreduce2(double v0, double v1, double* sums, unsigned long long* mb, int j, int* flags,
-                                double* red) {
+template <class F>
+__device__ __forceinline__ bool grid_allreduce2(double v0, double v1, double* sums, unsigned long long* mb, int j,
+                                                int* flags, double* red, F between) {
     const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, k = j & 3;
-    double* const rd = red + (j & 1) * 2 * PCG_WAVES;
+    double* const rd = red + (j & 1) * 2 * PCGS_WAVES;
     v0 = wave_sum(v0);
     v1 = wave_sum(v1);
     if ((tid & 63) == 0) {
         rd[tid >> 6] = v0;
-        rd[PCG_WAVES + (tid >> 6)] = v1;
+        rd[PCGS_WAVES + (tid >> 6)] = v1;
     }
     wait_vm();
     __syncthreads();
     if (tid == 0) {
         unsigned long long* const own = mb + (4 * g + k) * MB_LINE;
         unsigned long long* const old = mb + (4 * g + ((k + 2) & 3)) * MB_LINE;
-        double s0 = rd[0], s1 = rd[PCG_WAVES];
+        double s0 = rd[0], s1 = rd[PCGS_WAVES];
 #pragma unroll
-        for (int w = 1; w < PCG_WAVES; ++w) {
+        for (int w = 1; w < PCGS_WAVES; ++w) {
             s0 += rd[w];
-            s1 += rd[PCG_WAVES + w];
+            s1 += rd[PCGS_WAVES + w];
         }
         st_cu(own, __double_as_longlong(s0));
         st_cu(own + 1, __double_as_longlong(s1));
         st_cu(old, MB_EMPTY);
         st_cu(old + 1, MB_EMPTY);
     }
+    between();
     double u0 = 0.0, u1 = 0.0;
     int bad = 0;
     if (tid < G) {
@@ -1392,12 +1399,12 @@ __device__ bool grid_allreduce2(double v0, double v1, double* sums, unsigned lon
         u1 = wave_sum(u1);
         if ((tid & 63) == 0) {
             rd[tid >> 6] = u0;
-            rd[PCG_WAVES + (tid >> 6)] = u1;
+            rd[PCGS_WAVES + (tid >> 6)] = u1;
         }
     }
     const bool ok = __syncthreads_or(bad) == 0;
     sums[0] = (rd[0] + rd[1]) + (rd[2] + rd[3]);
-    sums[1] = (rd[PCG_WAVES] + rd[PCG_WAVES + 1]) + (rd[PCG_WAVES + 2] + rd[PCG_WAVES + 3]);
+    sums[1] = (rd[PCGS_WAVES] + rd[PCGS_WAVES + 1]) + (rd[PCGS_WAVES + 2] + rd[PCGS_WAVES + 3]);
     return ok;
 }
 
@@ -1573,8 +1580,15 @@ __global__ __launch_bounds__(LU_T) void k_eeq_lu_fallback(int np, int nr, const 
 // rows of x and r, and the Linv of a single owned block, in LDS for the
 // whole solve and writes x at the end.
 //
-// The matrix streams through once per iteration; eight wavefronts per
-// workgroup (two per SIMD) let one load while the other multiplies.
+// Streaming (np > 4032): one wavefront per SIMD with the whole register file.
+// Up to PCGS_PP blocks per wavefront its first block stays in registers for
+// the whole solve (water_3000, 4.4 blocks each: a quarter of the matrix), and
+// the next one is loaded behind the publication of the barrier ahead of it,
+// which hides its latency; with more, two register buffers take the blocks in
+// turn.  water_3000 1324 -> 1259 us against eight wavefronts with one buffer
+// (mixed 1019 -> 970); in turn from two blocks on 1282 and 987.  80 chains of
+// C80H162 run at 0.34 ms an iteration either way: 1.49 GB of blocks and 0.09
+// GB of partials at 4.6 TB/s, where a device copy moves 5.2.
 //
 // Preconditioner.  M = D, the diagonal blocks of R, cuts a fragment of more
 // than 64 variables into pieces, and every variable of the fragment carries
@@ -1697,10 +1711,11 @@ __device__ inline void packed_block(int t, int& I, int& J) {
 // sigma_f s_f of every split fragment into sfs, from the published parts;
 // returns sum_f sigma_f s_f^2 (the same in every workgroup).  sig: sigma_f.
 // pbuf: the parts, in LDS.
+template <int NT>
 __device__ double sm_sums(const PcgArgs& a, double* sfs, const double* sig, const double* pbuf, double* red) {
     const int tid = threadIdx.x, l8 = tid & 7;
     double e = 0.0;
-    for (int f0 = 0; f0 < a.nsf; f0 += PCG_THREADS / 8) {
+    for (int f0 = 0; f0 < a.nsf; f0 += NT / 8) {
         const int f = f0 + (tid >> 3);
         double s = 0.0;
         if (f < a.nsf)
@@ -1718,31 +1733,32 @@ __device__ double sm_sums(const PcgArgs& a, double* sfs, const double* sig, cons
     __syncthreads();
     double t = red[0];
 #pragma unroll
-    for (int w = 1; w < PCG_WAVES; ++w) t += red[w];
+    for (int w = 1; w < NT / 64; ++w) t += red[w];
     return t;
 }
 
+template <int NT>
 __device__ double sm_gather(const PcgArgs& a, int npc, double* sfs, const double* sig, double* pbuf, double* red) {
-    for (int k = threadIdx.x; k < npc; k += PCG_THREADS) pbuf[k] = ld_c(a.sp + a.pidx[k]);
+    for (int k = threadIdx.x; k < npc; k += NT) pbuf[k] = ld_c(a.sp + a.pidx[k]);
     __syncthreads();
-    return sm_sums(a, sfs, sig, pbuf, red);
+    return sm_sums<NT>(a, sfs, sig, pbuf, red);
 }
 
-template <bool SM>
-__global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
-    __shared__ double red[4 * PCG_WAVES], red2[2][PCG_WAVES];
+template <bool SM, bool PP>
+__global__ __launch_bounds__(PCGS_THREADS, 1) void k_eeq_pcg(PcgArgs a) {
+    __shared__ double red[4 * PCGS_WAVES], red2[2][PCGS_WAVES];
     __shared__ double pown[PCG_MAXB][NB];
-    __shared__ double qs[PCG_WAVES][NB];
+    __shared__ double qs[PCGS_WAVES][NB];
     __shared__ double rb[NB], wb[NB], zb[NB];
     __shared__ double xo[PCG_MAXB][NB], ro[PCG_MAXB][NB];  // owned rows of x and r, resident for the solve
     __shared__ double Lc[NB * LDC];                         // Linv of the owned block when there is one
-    __shared__ __align__(16) double pw[PCG_WAVES][2][NB];    // per wavefront: p of the block's rows and columns
+    __shared__ __align__(16) double pw[PCGS_WAVES][2][NB];    // per wavefront: p of the block's rows and columns
     __shared__ double sfs[SM ? SM_MAXF : 1], sig[SM ? SM_MAXF : 1], pbuf[SM ? SM_MAXP : 1];
     // a diagonal block that is not positive definite (FLAG_CHOL, set before
     // this launch and not cleared in it, so every workgroup reads the same
     // value) leaves the solve to the dense fallback
     if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & FLAG_CHOL) {
-        if (blockIdx.x == 0 && a.lu_w && eeq_lu<PCG_THREADS>(a.np, a.nr, 0, a.Rp, a.b, a.lu_w, a.x) && threadIdx.x == 0)
+        if (blockIdx.x == 0 && a.lu_w && eeq_lu<PCGS_THREADS>(a.np, a.nr, 0, a.Rp, a.b, a.lu_w, a.x) && threadIdx.x == 0)
             atomicOr(a.flags, FLAG_LU);
         return;
     }
@@ -1750,20 +1766,28 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
     const int nown = (nbk - g + G - 1) / G;
     // this wavefront's blocks of the packed order: [t0, t1)
-    const long T = (long)nbk * (nbk + 1) / 2, W = (long)PCG_WAVES * G, gw = (long)PCG_WAVES * g + wv;
+    const long T = (long)nbk * (nbk + 1) / 2, W = (long)PCGS_WAVES * G, gw = (long)PCGS_WAVES * g + wv;
     const int t0 = (int)(T * gw / W), t1 = (int)(T * (gw + 1) / W);
     int I0, J0;
     packed_block(t0, I0, J0);
     // lane (rg, cg) holds rows 8 rg + i (i < 8) and columns 2 cg + (k & 1) + 16 (k >> 1) (k < 8) of a
     // block: every 16-byte load instruction reads whole 128-byte row segments
     const int rg = l >> 3, cg = l & 7;
-    double rv[8][8];
+    // PP: rv and ra take the blocks of the range in turn, the next one in
+    // flight; otherwise ra keeps the first for the whole solve
+    double ra[8][8], rv[8][8];
+    constexpr int S0 = PP ? 0 : 1;  // first streamed block
+    if (!PP && t0 < t1) load_block(ra, a.Rp + (size_t)t0 * NB * NB, l);
+    auto first_stream = [&]() {
+        if (t0 + S0 < t1) load_block(rv, a.Rp + (size_t)(t0 + S0) * NB * NB, l);
+    };
+    auto nothing = []() {};
     const bool lcache = nown == 1;
     if (lcache)
-        for (int e = tid; e < NB * NB; e += PCG_THREADS) Lc[(e >> 6) * LDC + (e & 63)] = a.Lj[(size_t)g * NB * NB + e];
+        for (int e = tid; e < NB * NB; e += PCGS_THREADS) Lc[(e >> 6) * LDC + (e & 63)] = a.Lj[(size_t)g * NB * NB + e];
     const int npc = SM ? a.poff[a.nsf] : 0;
     if (SM)
-        for (int f = tid; f < a.nsf; f += PCG_THREADS) {
+        for (int f = tid; f < a.nsf; f += PCGS_THREADS) {
             double s = 1.0 / a.all[f];
             for (int k = a.poff[f]; k < a.poff[f + 1]; ++k) s += a.w1[a.pidx[k]];
             sig[f] = 1.0 / s;
@@ -1807,10 +1831,10 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
     }
     int nbar = 0;  // barriers passed
     double sums[2];
-    if (!grid_allreduce2(lrz, lbb, sums, a.mb, nbar++, a.flags, red)) return;
+    if (!grid_allreduce2(lrz, lbb, sums, a.mb, nbar++, a.flags, red, first_stream)) return;
     double rz = sums[0];
     const double bb = sums[1];
-    if (SM) rz -= sm_gather(a, npc, sfs, sig, pbuf, red2[0]);
+    if (SM) rz -= sm_gather<PCGS_THREADS>(a, npc, sfs, sig, pbuf, red2[0]);
     double beta = 0.0;
     int it = 0;
     bool done = !(bb > 0.0);
@@ -1829,30 +1853,82 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
         }
         double lpq = 0.0;
         int I = I0, J = J0;
-        for (int t = t0; t < t1; ++t) {
-            load_block(rv, a.Rp + (size_t)t * NB * NB, l);
+        // what a block's product needs of z and p (y, p, w and fragment of its
+        // columns and rows), loaded ahead of the next block's loads: loads
+        // return in order
+        struct Raw {
+            double zj, pj, zi, pi, wj, wi;
+            int fj, fi;
+        };
+        auto fetch = [&](int I, int J) {
+            Raw r;
+            const int cj = J * NB + l, ci = I * NB + l;
+            r.zj = ld_c(a.z + cj);
+            r.zi = ld_c(a.z + ci);
+            r.pj = it == 0 ? 0.0 : ld_c(pprev + cj);
+            r.pi = it == 0 ? 0.0 : ld_c(pprev + ci);
+            r.fj = SM ? a.rowf[cj] : -1;
+            r.fi = SM ? a.rowf[ci] : -1;
+            r.wj = SM && r.fj >= 0 ? a.w[cj] : 0.0;
+            r.wi = SM && r.fi >= 0 ? a.w[ci] : 0.0;
+            return r;
+        };
+        auto next = [&](int& I, int& J) {
+            if (++J > I) {
+                ++I;
+                J = 0;
+            }
+        };
+        auto product = [&](const double (&blk)[8][8], const Raw& r) {
             // p of row I * 64 + l and column J * 64 + l
-            const double pcj = (it == 0) ? 0.0 : ld_c(pprev + J * NB + l);
-            const double pjl = zrow(J * NB + l) + beta * pcj;
-            const double pci = (it == 0) ? 0.0 : ld_c(pprev + I * NB + l);
-            const double pil = zrow(I * NB + l) + beta * pci;
+            double zj = r.zj, zi = r.zi;
+            if (SM) {
+                if (r.fj >= 0) zj -= sfs[r.fj >> 1] * r.wj;
+                if (r.fi >= 0) zi -= sfs[r.fi >> 1] * r.wi;
+            }
+            const double pjl = zj + beta * r.pj, pil = zi + beta * r.pi;
             pw[wv][0][l] = pil;
             pw[wv][1][l] = pjl;
             __builtin_amdgcn_wave_barrier();
             double rs, cs, pjc;
-            block_products(rv, pw[wv], l, I != J, rs, cs, pjc);
+            block_products(blk, pw[wv], l, I != J, rs, cs, pjc);
             st_c(a.part + ((size_t)I * nbk + J) * NB + l, rs);
             lpq += pil * rs;
             if (I != J) {
                 st_c(a.part + ((size_t)J * nbk + I) * NB + 2 * cg + (rg & 1) + 16 * (rg >> 1), cs);
                 lpq += pjc * cs;
             }
-            if (++J > I) {
-                ++I;
-                J = 0;
+            next(I, J);
+        };
+        if (!PP) {
+            if (t0 < t1) product(ra, fetch(I, J));
+            for (int t = t0 + 1; t < t1; ++t) {
+                if (t > t0 + 1) load_block(rv, a.Rp + (size_t)t * NB * NB, l);  // the first: behind the last barrier
+                product(rv, fetch(I, J));
+            }
+        } else if (t0 < t1) {
+            Raw r0 = fetch(I, J);
+            for (int t = t0; t < t1; t += 2) {
+                int I1 = I, J1 = J;
+                next(I1, J1);
+                Raw r1{};
+                if (t + 1 < t1) {
+                    r1 = fetch(I1, J1);
+                    load_block(ra, a.Rp + (size_t)(t + 1) * NB * NB, l);
+                }
+                product(rv, r0);
+                if (t + 1 >= t1) break;
+                I1 = I;
+                J1 = J;
+                next(I1, J1);
+                if (t + 2 < t1) {
+                    r0 = fetch(I1, J1);
+                    load_block(rv, a.Rp + (size_t)(t + 2) * NB * NB, l);
+                }
+                product(ra, r1);
             }
         }
-        if (!grid_allreduce2(lpq, 0.0, sums, a.mb, nbar++, a.flags, red)) return;
+        if (!grid_allreduce2(lpq, 0.0, sums, a.mb, nbar++, a.flags, red, nothing)) return;
         const double pq = sums[0];
         const double alpha = rz / pq;
         // (2) owners: q rows from the partials (Y order), x, r, z and the
@@ -1861,15 +1937,15 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
         for (int o = 0; o < nown; ++o) {
             const int kb = g + o * G;
             {
-                // thread (row l, part wv) adds Y = wv, wv + PCG_WAVES, ... in batches of 16 loads
+                // thread (row l, part wv) adds Y = wv, wv + PCGS_WAVES, ... in batches of 16 loads
                 const double* pr = a.part + (size_t)kb * nbk * NB + l;
                 double acc = 0.0;
-                for (int y0 = wv; y0 < nbk; y0 += 16 * PCG_WAVES) {
+                for (int y0 = wv; y0 < nbk; y0 += 16 * PCGS_WAVES) {
                     double t16[16];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) t16[u] = ld_c(pr + (size_t)min(y0 + PCG_WAVES * u, nbk - 1) * NB);
+                    for (int u = 0; u < 16; ++u) t16[u] = ld_c(pr + (size_t)min(y0 + PCGS_WAVES * u, nbk - 1) * NB);
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) acc += (y0 + PCG_WAVES * u < nbk) ? t16[u] : 0.0;
+                    for (int u = 0; u < 16; ++u) acc += (y0 + PCGS_WAVES * u < nbk) ? t16[u] : 0.0;
                 }
                 qs[wv][l] = acc;
             }
@@ -1877,7 +1953,7 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
             if (tid < NB) {
                 double qv = qs[0][tid];
 #pragma unroll
-                for (int w = 1; w < PCG_WAVES; ++w) qv += qs[w][tid];
+                for (int w = 1; w < PCGS_WAVES; ++w) qv += qs[w][tid];
                 xo[o][tid] += alpha * pown[o][tid];
                 const double rn = ro[o][tid] - alpha * qv;
                 ro[o][tid] = rn;
@@ -1886,11 +1962,11 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg(PcgArgs a) {
             __syncthreads();
             publish(kb, lrz2, lrr);
         }
-        if (!grid_allreduce2(lrz2, lrr, sums, a.mb, nbar++, a.flags, red)) return;
+        if (!grid_allreduce2(lrz2, lrr, sums, a.mb, nbar++, a.flags, red, first_stream)) return;
         const double rr = sums[1];
         double rz2 = sums[0];
         done = rr <= a.tol2 * bb;
-        if (SM && !done) rz2 -= sm_gather(a, npc, sfs, sig, pbuf, red2[it & 1]);
+        if (SM && !done) rz2 -= sm_gather<PCGS_THREADS>(a, npc, sfs, sig, pbuf, red2[it & 1]);
         beta = rz2 / rz;
         rz = rz2;
     }
@@ -2073,7 +2149,7 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg_res(PcgArgs a) {
         }
         if (done || it >= a.maxit) break;
         if (SM) {
-            rz -= sm_sums(a, sfs, sig, pbuf, red2);
+            rz -= sm_sums<PCG_THREADS>(a, sfs, sig, pbuf, red2);
             if (fI >= 0) yI -= sfs[fI >> 1] * wI;
             if (fJ >= 0) yJ -= sfs[fJ >> 1] * wJ;
         }
@@ -6657,7 +6733,17 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         for (int i = 0; i < n; ++i) fa[P.frag[i]].push_back(i);
         std::vector<int> red_atom, red_last, red_of(n, -1), foff(P.nfrag + 1, 0), fatoms;
         std::vector<double> qp(n, 0.0);
-        if (E->use_cg) reduced_order(P, fa);
+        // On the mixed path the pair terms take the charges rounded to FP32, so that
+        // two solves that agree to the tolerance can round a charge to
+        // neighbouring values; one such step moves the gradient by up to 1.6e-7 of
+        // its RMS where charges reach 0.5 e (a peptide), by 4e-9 where they stay
+        // below 0.1 e (hydrocarbons).  There the order and the preconditioner of
+        // long fragments apply on both paths, for polar molecules on the FP64 path
+        // only, whose charges converge to rounding.
+        double qmax = 0.0;
+        for (double v : P.qa) qmax = std::max(qmax, std::fabs(v));
+        const bool long_frag = E->use_cg && (!E->mixed || qmax <= 0.1);
+        if (long_frag) reduced_order(P, fa);
         for (int f = 0; f < P.nfrag; ++f) {
             int m = (int)fa[f].size();
             int last = fa[f].back();
@@ -7199,7 +7285,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             int dev = 0, ncu = 0, per_cu = 0;
             if (hipGetDevice(&dev) != hipSuccess ||
                 hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eeq_pcg<true>, PCG_THREADS, 0) !=
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eeq_pcg<true, true>, PCGS_THREADS, 0) !=
                     hipSuccess) {
                 status = kErrDevice;
                 msg = "PCG occupancy query failed";
@@ -7258,7 +7344,7 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
             for (int r0 = 0; r0 < E->nr;) {
                 int r1 = r0 + 1;
                 while (r1 < E->nr && red_last[r1] == red_last[r0]) ++r1;
-                if (r1 - r0 > NB) {
+                if (r1 - r0 > NB && long_frag) {
                     for (int r = r0; r < r1; ++r) {
                         const int bk = r / NB;
                         // second piece of its block when another split fragment, which then
@@ -7916,10 +8002,18 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
             LAUNCH(KC_PCG, k_eeq_pcg_res<true>, grid, block, s, E->cg);
         else if (E->cg_res)
             LAUNCH(KC_PCG, k_eeq_pcg_res<false>, grid, block, s, E->cg);
-        else if (E->cg.nsf)
-            LAUNCH(KC_PCG, k_eeq_pcg<true>, grid, block, s, E->cg);
-        else
-            LAUNCH(KC_PCG, k_eeq_pcg<false>, grid, block, s, E->cg);
+        else {
+            const dim3 sb(PCGS_THREADS);
+            const bool pp = (long)nbk * (nbk + 1) / 2 >= (long)PCGS_PP * PCGS_WAVES * E->cg_groups;
+            if (E->cg.nsf && pp)
+                LAUNCH(KC_PCG, (k_eeq_pcg<true, true>), grid, sb, s, E->cg);
+            else if (E->cg.nsf)
+                LAUNCH(KC_PCG, (k_eeq_pcg<true, false>), grid, sb, s, E->cg);
+            else if (pp)
+                LAUNCH(KC_PCG, (k_eeq_pcg<false, true>), grid, sb, s, E->cg);
+            else
+                LAUNCH(KC_PCG, (k_eeq_pcg<false, false>), grid, sb, s, E->cg);
+        }
     } else if (!E->mixed) {
         if (E->lu_src)
             LAUNCH(KC_CHOL_DIAG, k_copy, dim3(cdiv((long)E->mat_size, 256)), dim3(256), s, (int)E->mat_size, E->Ared,
