@@ -2,24 +2,24 @@
 // single molecules and batches of independent molecules.
 //
 // One evaluation is a fixed sequence of kernels on two streams (launch_eval):
-//   second stream: the reduced EEQ matrix (k_eeq_reduced / k_eeq_reduced_batch)
-//     and, for batches, the per-molecule factorisation (k_lstep_tiles,
-//     k_bstep_diag, k_bstep_tiles or the per-molecule forms), then the
-//     hydrogen-bond kernels of batches;
+//   second stream: the reduced EEQ matrix (k_eeq_reduced / k_eeq_reduced_batch),
+//     for single molecules the solver's preconditioner (k_bjacobi_setup), for
+//     batches the per-molecule factorisation (k_lstep_tiles, k_bstep_diag64,
+//     k_bstep_tiles or the per-molecule forms); solvation (k_solv_*); of a
+//     batch also the hydrogen bonds, behind the factorisation;
 //   evaluation stream:
+//   k_start             coordinates, flags, bounding boxes
 //   k_cn / k_cn_mol     CN (6 Bohr), log cap, dlogdcn, D4 weights, EEQ rhs, CN neighbour lists
-//   k_d4_half           per-atom D4 half contraction of C6 and dC6/dCN
-//   k_bonds .. k_batm   bonded term lists writing per-atom gradient slots
-//   k_slot_gather       per-atom sum of the slots
-//   k_hb_*              hydrogen bonds (single molecules on this stream)
+//   k_terms             bonded term lists (per-atom gradient slots), D4 half contraction, reduced rhs
+//   k_hb_roles/k_hb_full  hydrogen bonds
+//   k_slot_gather       per-atom sum of the slots (and of a molecule's hydrogen bonds)
 //   -- join --
-//   EEQ solve           k_eeq_pcg / k_chol_* + k_trsv_* (single), k_bsolve_subst (batches)
+//   EEQ solve           k_eeq_pcg_one / _res / k_eeq_pcg or k_chol_* + k_trsv_* (single), k_bsolve_subst (batches)
 //   k_charges           charges from the reduced solution, self energy, qtmp
 //   k_pairs_sym         Coulomb + D4 dispersion + repulsion, each pair once (64 x 64 tiles)
-//   k_pairs_sym_reduce  fixed-order sum of the tile partials (no atomics)
-//   k_atom_tail         bonded / 1,3 / 1,4 H-H corrections of the repulsion pair sum, dE/dCN totals
-//   k_finish            CN chain rule + gradient assembly
-//   k_reduce1/_final    fixed-order energy reductions
+//   k_pairs_sym_reduce  fixed-order sum of the tile partials (no atomics), corrections of the
+//                       repulsion over the topological neighbourhood, dE/dCN totals
+//   k_finish            CN chain rule + gradient assembly, fixed-order energy reductions
 // Reference semantics: see oracle/gfnff_oracle.c (same formulas, same cut-offs).
 #include <hip/hip_runtime.h>
 
@@ -2501,7 +2501,7 @@ struct PairArgs {
     const int* nref;
     const int* metal;
     const double* c6ref;
-    const double* h;  // [n][nelem][7] D4 half contraction (k_d4_half)
+    const double* h;  // [n][nelem][7] D4 half contraction (k_terms)
     const double* dh;
     const int* mol_of;   // batches: molecule of each atom (nullptr: one molecule)
     const int* mol_off;  // batches: atom offsets of the molecules
@@ -5087,7 +5087,7 @@ __global__ __launch_bounds__(BSOLVE_T, MINB) void k_eeq_batch_fused(
 // ---- left-looking factorisation by column blocks over the whole batch (batch_solver 5)
 // Column block j is three launches over every molecule with more than j
 // column blocks: the tiles (i, j), i >= j, formed by fused_tile (one
-// wavefront per tile, any molecule), the diagonal blocks (k_bstep_diag) and
+// wavefront per tile, any molecule), the diagonal blocks (k_bstep_diag64) and
 // the panel tiles L(i, j) = C(i, j) L(j, j)^-T (k_bstep_tiles<double,
 // false>).  The per-molecule form's parallelism (four wavefronts) becomes
 // thousands of independent tiles per launch, and the entries of R are still

@@ -102,3 +102,34 @@ def test_pcg_groups_do_not_change_the_solve(groups, oracle):
     m.calculateEnergy(True)
     assert not m.hasError(), m.getErrorMessage()
     check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), "fp64")
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_batch_past_the_pinned_buffers(precision, oracle):
+    """133 566 atoms: past the size up to which host buffers go through pinned
+    memory.  Copies of six molecules against the oracle, and every copy against
+    the first."""
+    mols = [molecule(*k) for k in (("alkane", 1), ("water", 2), ("peptide", 9), ("alkane", 42), ("peptide", 27),
+                                   ("alkane", 64))]
+    per = sum(len(z) for z, _ in mols)
+    copies = 131072 // per + 5
+    off = np.cumsum([0] + [len(z) for z, _ in mols] * copies)
+    Z = np.concatenate([z for z, _ in mols] * copies)
+    xyz = np.vstack([x for _, x in mols] * copies)
+    b = GFNFFBatch(precision=precision)
+    assert b.setBatch(off, Z, xyz), b.getErrorMessage()
+    b.calculateEnergy(True)
+    assert not b.hasError(), b.getErrorMessage()
+    e = b.getEnergies().reshape(copies, len(mols))
+    g = b.getGradient().reshape(copies, per, 3)
+    q = b.getCharges().reshape(copies, per)
+    # sums of at most 1e4 terms of order 1 in FP64; FP32 pair terms may round a charge the other way
+    tol = 1e-11 if precision == "fp64" else 1e-6
+    assert np.abs(e - e[0]).max() < tol and np.abs(g - g[0]).max() < tol and np.abs(q - q[0]).max() < 1e-11
+    for k, (z, x) in enumerate(mols):
+        m = GFNFFMethod()
+        assert m.setMolecule(Mol(z, x))
+        ref = oracle.eval(m.params_view(), x * (1.0 / BOHR))
+        m._energy, m._grad = e[0, k], g[0, off[k]:off[k + 1]]
+        m.getCharges = lambda: q[0, off[k]:off[k + 1]]
+        check(m, z, x, ref, precision)
