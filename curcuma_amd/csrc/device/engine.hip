@@ -3880,9 +3880,12 @@ __device__ __forceinline__ void xb_entry(int b, int nx, const int* __restrict__ 
 // is the reference arithmetic; T = float (mixed path) forms the coordinate
 // differences in FP64 and evaluates the term in FP32 with hardware rsqrt,
 // rcp and exp.
-__device__ inline double hb_sqrt(double v) { return sqrt(v); }
+// The FP64 cores are bound by instruction issue: a divide or square-root
+// sequence is 10 to 15 of their FP64 instructions, the refined estimates
+// (about 1 ulp) are 4 and 5.
+__device__ inline double hb_sqrt(double v) { return v * rsqrt_c(fmax(v, 1e-300)); }
 __device__ inline float hb_sqrt(float v) { return __builtin_sqrtf(v); }
-__device__ inline double hb_rcp(double v) { return 1.0 / v; }
+__device__ inline double hb_rcp(double v) { return rcp_c(v); }
 __device__ inline float hb_rcp(float v) { return __builtin_amdgcn_rcpf(v); }
 __device__ inline double hb_exp(double v) { return exp(v); }
 __device__ inline float hb_exp(float v) { return __expf(v); }
@@ -4151,10 +4154,14 @@ __global__ __launch_bounds__(256) void k_hb_roles(HBRoles r, HBArgs a, const dou
 // Hydrogen bonds of cases 2-4, one thread each: energy, and the gradient in
 // the triplet's slots s0 (A), s0 + 1 (H), s0 + 2 (B), s0 + 3 + k (k-th
 // neighbour of B), then the carbonyl's D atoms.  MODE 0: every entry by the
-// FP64 core; MODE 1: case-2 entries only, by hb_core2<T> (the mixed path's
-// FP32 terms); MODE 2: entries of cases 3 and 4 only, FP64.  ord (MODE 1
+// general FP64 core; MODE 1: case-2 entries only, by hb_core2<T> (FP32 terms
+// on the mixed path); MODE 2: entries of cases 3 and 4 only, FP64.  ord (MODE 1
 // and 2): the entries of the mode, case 2 first, so that no lane idles on
 // an entry of the other mode; nh counts the mode's entries.
+// Bound by FP64 instruction issue.  The general core holds 256 VGPRs (two
+// wavefronts per SIMD) and divides throughout; the lean one 152.  With it and
+// the estimates of hb_rcp in the case-1 roles an FP64 evaluation of 9000
+// atoms of water goes 1258 -> 1236 us, of 4096 molecules 7.14 -> 7.10 ms.
 template <typename T, int MODE>
 __global__ __launch_bounds__(256, 2) void k_hb_full(int nh, const int* __restrict__ ord, const int4* __restrict__ ahbc,
                                                  const int* __restrict__ slot0, HBArgs a, const double* __restrict__ x,
@@ -7951,16 +7958,24 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
             else
                 LAUNCH(KC_HB, k_hb_roles<double>, dim3(nrole), dim3(256), hs, hr, ha, E->x, E->hb_gout, E->e_hb);
         }
-        // cases 2-4: on the mixed path the case-2 entries by the lean FP32
-        // kernel and those of cases 3 and 4 by the FP64 one
+        // cases 2-4: the case-2 entries by the lean core (FP32 terms on the
+        // mixed path), those of cases 3 and 4 by the general FP64 one; a short
+        // FP64 list that holds both by the general core in one launch (38
+        // atoms, host buffers: 134 us against 143 with two; 61 conformers and 256
+        // molecules within their noise)
         const int n34 = E->nhb2 - E->nhb2_c2;
-        if (E->nhb2 && !E->mixed)
+        constexpr int HB_ONE_MAX = 16384;
+        const bool one = !E->mixed && n34 > 0 && E->nhb2 <= HB_ONE_MAX;
+        if (one)
             LAUNCH(KC_HB, (k_hb_full<double, 0>), dim3(cdiv(E->nhb2, 256)), dim3(256), hs, E->nhb2, E->hb_ord,
+                   E->hb_ahbc, E->hb_s0, ha, E->x, E->hb_xslots, E->e_hb2);
+        if (!one && E->nhb2_c2 && !E->mixed)
+            LAUNCH(KC_HB, (k_hb_full<double, 1>), dim3(cdiv(E->nhb2_c2, 256)), dim3(256), hs, E->nhb2_c2, E->hb_ord,
                    E->hb_ahbc, E->hb_s0, ha, E->x, E->hb_xslots, E->e_hb2);
         if (E->mixed && E->nhb2_c2)
             LAUNCH(KC_HB, (k_hb_full<float, 1>), dim3(cdiv(E->nhb2_c2, 256)), dim3(256), hs, E->nhb2_c2, E->hb_ord,
                    E->hb_ahbc, E->hb_s0, ha, E->x, E->hb_xslots, E->e_hb2);
-        if (E->mixed && n34 > 0)
+        if (!one && n34 > 0)
             LAUNCH(KC_HB, (k_hb_full<double, 2>), dim3(cdiv(n34, 256)), dim3(256), hs, n34, E->hb_ord + E->nhb2_c2,
                    E->hb_ahbc, E->hb_s0, ha, E->x, E->hb_xslots, E->e_hb2);
     }
