@@ -2677,7 +2677,7 @@ __global__ __launch_bounds__(TILE) void k_pairs_part(PairArgs a, int cj, double*
             }
             // non-bonded repulsion (generic pair factor; bonded / 1,3 / 1,4
             // corrections follow in k_atom_tail)
-            if (r <= 20.0 && r >= 1e-8) {
+            if (r2 <= 400.0 && r >= 1e-8) {
                 double ff = rep_ff(zi, sZ[jj], mi, smt[jj]);
                 double al = sqrt(ani * san[jj]) * ff;
                 double ab = rzi * srz[jj] * 0.4270;
@@ -2964,10 +2964,10 @@ __global__ __launch_bounds__(PS_B) void k_pairs_sym(PairArgs a, double* __restri
         T dEdr = 0, hec = 0, hed = 0, her = 0, dci = 0, dcj = 0;
         const T r2 = (T)r2d;
         const T rinv = ps_rsqrt(r2), r = r2 * rinv;
-        const bool coul = (terms & PT_COUL) && ((sizeof(T) == 4) ? (r2d >= 1e-20) : (r <= T(100) && r >= T(1e-10)));
-        const bool disp = (terms & PT_DISP) &&
-                          ((sizeof(T) == 4) ? (r2d <= 2500.0 && r2d >= 1e-20) : (r <= T(50) && r >= T(1e-10)));
-        const bool rep = (terms & PT_REP) && ((sizeof(T) == 4) ? (r2d <= 400.0 && r2d >= 1e-16) : (r <= T(20) && r >= T(1e-8)));
+        // cut-offs on the squares: r is within rounding of the root, not the rounded root
+        const bool coul = (terms & PT_COUL) && r2d >= 1e-20;
+        const bool disp = (terms & PT_DISP) && r2d <= 2500.0 && r2d >= 1e-20;
+        const bool rep = (terms & PT_REP) && r2d <= 400.0 && r2d >= 1e-16;
         if (coul) {
             const T gij = ps_rsqrt(ali + cal[jj]);
             const T gr = gij * r;
@@ -3889,6 +3889,9 @@ __device__ inline double hb_rcp(double v) { return rcp_c(v); }
 __device__ inline float hb_rcp(float v) { return __builtin_amdgcn_rcpf(v); }
 __device__ inline double hb_exp(double v) { return exp(v); }
 __device__ inline float hb_exp(float v) { return __expf(v); }
+// r_AB <= 50 Bohr; FP64 on the square, as r is within rounding of the root, not the rounded root
+__device__ inline bool hb_near(double rab2, double) { return rab2 <= 2500.0; }
+__device__ inline bool hb_near(float, float rAB) { return rAB <= 50.0f; }
 template <typename T>
 struct V3 {
     T x, y, z;
@@ -3941,7 +3944,7 @@ __device__ double hb_core1(int A, int H, int B, const HBArgs& a, const double* _
     const T rbh2 = drbh.x * drbh.x + drbh.y * drbh.y + drbh.z * drbh.z;
     const T rab2 = drab.x * drab.x + drab.y * drab.y + drab.z * drab.z;
     const T rAH = hb_sqrt(rah2), rHB = hb_sqrt(rbh2), rAB = hb_sqrt(rab2);
-    if (!(rAB <= T(50))) return 0.0;
+    if (!hb_near(rab2, rAB)) return 0.0;
     T basA, basB, aciA, aciB, QH, QA, QB, radab;
     hb_params<T>(A, H, B, a, basA, basB, aciA, aciB, QH, QA, QB, radab);
     const T rAH4 = rah2 * rah2, rHB4 = rbh2 * rbh2;
@@ -4009,7 +4012,7 @@ __device__ double hb_core2(int A, int H, int B, const HBArgs& a, const double* _
     const T rAH = hb_sqrt(rah2), rHB = hb_sqrt(rbh2), rAB = hb_sqrt(rab2);
     double E = 0.0;
     bool written = false;
-    if (rAB <= T(50)) {
+    if (hb_near(rab2, rAB)) {
         T basA, basB, aciA, aciB, QH, QA, QB, radab;
         hb_params<T>(A, H, B, a, basA, basB, aciA, aciB, QH, QA, QB, radab);
         const T irab2 = hb_rcp(rab2), irAB = hb_rcp(rAB), irHB = hb_rcp(rHB), irbh2 = irHB * irHB;
@@ -5383,7 +5386,7 @@ __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __
             const double r2 = dx * dx + dy * dy + dz * dz;
             if (r2 > 2500.0) continue;  // beyond the D4 and repulsion cut-offs
             const double rinv = rsqrt_c(r2), r = r2 * rinv;
-            if (!(r >= 1e-10)) continue;
+            if (!(r2 >= 1e-20)) continue;
             const double sw = (wi.x * dx + wi.y * dy + wi.z * dz) * rinv;
             const int ej = sel[jj];
             double dd4 = 0.0, dz_ = 0.0, da_ = 0.0;
@@ -5404,7 +5407,7 @@ __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __
                 d4_adj(c6, dci, zti * szt[jj], q, r2, r, dEp_dq, ddcn_dq);
                 dd4 = (sw * dEp_dq + ui * ddcn_dq) * q;  // d / d ln(theta) of one factor of q
             }
-            if (r <= 20.0 && r >= 1e-8) {   // non-bonded repulsion, generic pair factor
+            if (r2 <= 400.0 && r2 >= 1e-16) {   // non-bonded repulsion, generic pair factor
                 const double ff = rep_ff(zi, sZ[jj], mi, smt[jj]);
                 const double al = sqrt(ani * san[jj]) * ff;
                 const double ab = rzi * srz[jj] * 0.4270;
