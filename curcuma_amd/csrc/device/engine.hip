@@ -5596,6 +5596,7 @@ constexpr int RED_BLOCKS = 64;
 constexpr int NPARTS = 16;  // energy segments reduced per evaluation
 struct FinishArgs {
     int n, nred, nmolb;  // workgroups per energy segment, and of the molecules' energies
+    int first;           // workgroups ahead of this launch's (0; the energies', where their class is timed)
     const double *x, *rcov, *dlog, *v;
     const int *nbn, *nbl;
     const double *gslot, *gpair, *ghb, *gsolv;
@@ -5686,7 +5687,7 @@ __device__ void reduce_segment(const FinishArgs& a, int sg, int b) {
 
 template <int LPA>
 __global__ __launch_bounds__(256) void k_finish(FinishArgs a) {
-    int blk = blockIdx.x;
+    int blk = blockIdx.x + a.first;
     if (blk < NPARTS * a.nred) {
         reduce_segment(a, blk / a.nred, blk % a.nred);
         return;
@@ -7910,7 +7911,11 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
     {
         TermArgs ta = E->terms;
         ta.rhs = rsrc;
-        if (ta.end[11] <= TERMS_FUSED_MAX) {
+        // a launch per list also where one of these classes is timed
+        const int tc = E->timer.cls;
+        const bool timed = tc == KC_EEQ_BUILD || tc == KC_PAIRS_AUX || tc == KC_BONDS || tc == KC_ANGLES ||
+                           tc == KC_TORS || tc == KC_HB || tc == KC_BREP || tc == KC_ATM || tc == KC_BATM;
+        if (ta.end[11] <= TERMS_FUSED_MAX && !timed) {
             LAUNCH(KC_BONDS, k_terms<-1>, dim3(ta.end[11]), dim3(256), s, ta);
         } else {
             auto wgs = [&](int k) { return dim3(ta.end[k] - (k ? ta.end[k - 1] : 0)); };
@@ -8158,10 +8163,16 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
         fa.nmolb = cdiv(E->nmol, 4);
     }
     const int head = NPARTS * fa.nred + fa.nmolb;
+    int left = head + cdiv(n, E->fin_lpa == 64 ? 4 : 16);
+    if (E->timer.cls == KC_REDUCE || E->timer.cls == KC_CHAIN) {  // the energies in a launch of their own
+        LAUNCH(KC_REDUCE, k_finish<64>, dim3(head), dim3(256), s, fa);
+        fa.first = head;
+        left -= head;
+    }
     if (E->fin_lpa == 64)
-        LAUNCH(KC_CHAIN, k_finish<64>, dim3(head + cdiv(n, 4)), dim3(256), s, fa);
+        LAUNCH(KC_CHAIN, k_finish<64>, dim3(left), dim3(256), s, fa);
     else
-        LAUNCH(KC_CHAIN, k_finish<16>, dim3(head + cdiv(n, 16)), dim3(256), s, fa);
+        LAUNCH(KC_CHAIN, k_finish<16>, dim3(left), dim3(256), s, fa);
     if (hipGetLastError() != hipSuccess) {
         msg = "kernel launch failed";
         return kErrDevice;

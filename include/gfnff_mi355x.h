@@ -270,11 +270,16 @@ int gfnff_param_adjoint(gfnff_handle* h, const double* w, double* dtheta, int32_
 int gfnff_cn_neighbours(gfnff_handle* h, int32_t* counts, int32_t* idx, int32_t maxnb);
 
 /* Engine extension (no counterpart in the reference): HIP-event timing of one
- * kernel class on the evaluation stream, for roofline measurement.  Classes:
+ * kernel class, for roofline measurement.  Classes:
  * cn eeq_build chol_diag chol_panel chol_update trsv charges pairs pairs_aux nbrep
- * refine bonds angles torsions brep hb atm batm chain reduce; NULL or "" switches timing
- * off.  Every launch of the class in later evaluations is bracketed by a
- * start/stop event pair. */
+ * refine bonds angles torsions brep hb atm batm chain reduce pcg batch_solve solvation;
+ * NULL or "" switches timing off.  Every launch of the class in later
+ * evaluations is bracketed by a start/stop event pair on its stream.  A class
+ * whose work an evaluation merges with others' (the term lists of small
+ * systems, the energy reduction with the chain rule) runs in launches of its
+ * own while it, or a class merged with it, is selected.  nbrep, the corrections
+ * of the non-bonded repulsion, is timed with pairs_aux and has no launch; a
+ * single molecule's gather of hydrogen-bond gradients is timed with chain. */
 int gfnff_profile_kernel(gfnff_handle* h, const char* name);
 
 /* Waits for the recorded events and returns the summed launch time (ms) and
