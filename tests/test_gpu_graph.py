@@ -8,7 +8,8 @@ this hardware; the evaluation records none).  The kernels sum in a fixed
 order, so replay and eager results are bitwise equal.  Covered: a batch of
 molecules on the mixed path and a single molecule on the PCG path (the
 persistent solver under graph launch), coordinates changed between
-replays, and a capture dropped when the engine is rebuilt."""
+replays, a capture dropped when the engine is rebuilt, and solvated
+molecules, whose second fork and join of the streams lie behind the charges."""
 import ctypes as C
 
 import numpy as np
@@ -18,6 +19,7 @@ from conftest import BOHR, HipRuntime, gpu_available
 from curcuma_amd import GFNFFBatch, GFNFFMethod, Mol
 from curcuma_amd._lib import NTERMS
 from curcuma_amd.workloads import mixed_batch, water_cluster
+from test_alpb import ammonium
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +77,12 @@ def test_graph_replay_single_pcg_and_rebuild():
     m.setParameters({"gather_lanes": 64})
     with pytest.raises(RuntimeError):
         m.launchGraph(None)
+
+
+@pytest.mark.parametrize("case", ["cluster", "cation"])
+def test_graph_replay_solvated(case):
+    """A neutral cluster (the surfaces on the second stream) and a cation (on the first, ahead of the fork)."""
+    Z, xyz = water_cluster(80, seed=5) if case == "cluster" else ammonium()
+    m = GFNFFMethod({"solvent": "water"})
+    assert m.setMolecule(Mol(np.asarray(Z), np.asarray(xyz), 0 if case == "cluster" else 1)), m.getErrorMessage()
+    run_case(m, HipRuntime(), np.asarray(xyz) * (1.0 / BOHR))

@@ -7,6 +7,8 @@ launch.  FP64: the oracle's arithmetic in another order, so energies agree to
 1e-9 Eh and gradients and charges to 1e-9 (the repository's parity bound);
 mixed: 1e-6 Eh per atom and 1e-5 Eh/Bohr RMS.
 """
+import math
+
 import numpy as np
 import pytest
 
@@ -76,32 +78,117 @@ def test_small_batch_sizes(precision, oracle):
         check(m, z, x, ref, precision)
 
 
-def test_split_fragment_not_positive_definite(oracle):
-    """70 hydrogens 0.74 A apart, bonded into one chain: A and the reduced matrix
+@pytest.mark.parametrize("n,groups", [(70, 0), (300, 0), (300, 2)])
+def test_split_fragment_not_positive_definite(n, groups, oracle):
+    """Hydrogens 0.74 A apart, bonded into one chain: A and the reduced matrix
     are indefinite (lowest eigenvalue -0.05), so the preconditioner's blocks fail
-    and the dense fallback gives the charges, as in the oracle."""
-    n = 70
+    and the dense fallback gives the charges, as in the oracle.  70 atoms: the
+    one-workgroup solver; 300: the resident one, and with two workgroups the
+    streaming one, whose other workgroups leave the solve to the first."""
     xyz = np.zeros((n, 3))
     xyz[:, 0] = 0.74 * np.arange(n)
     Z = np.ones(n, dtype=np.int32)
     m = GFNFFMethod()
+    m.setParameters({"pcg_groups": groups})
     assert m.setMolecule(Mol(Z, xyz, bonds=[(i, i + 1) for i in range(n - 1)])), m.getErrorMessage()
     m.calculateEnergy(True)
     assert not m.hasError(), m.getErrorMessage()
     check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), "fp64")
 
 
-@pytest.mark.parametrize("groups", [1, 5, 40])
-def test_pcg_groups_do_not_change_the_solve(groups, oracle):
-    """Bounded workgroup counts: too few for one block per wavefront stream the
-    blocks, more keep them resident (a 901-variable molecule, 120 blocks)."""
-    Z, xyz = molecule("alkane", 300)
+def eeq_matrices(m, xyz):
+    """A of a single fragment and its reduced matrix (last atom eliminated), from the parameter set."""
+    n = len(xyz)
+    v = m.params_view()
+    gam, alp = (np.ctypeslib.as_array(p, shape=(n,)) for p in (v.gam_eff, v.alpeeq))
+    A = np.diag(gam + np.sqrt(2.0 / np.pi) / np.sqrt(alp))
+    for i in range(n):
+        for j in range(i):
+            r = np.linalg.norm(xyz[i] - xyz[j]) / BOHR
+            A[i, j] = A[j, i] = math.erf(r / math.sqrt(alp[i] + alp[j])) / r
+    k = n - 1
+    return A, A[:k, :k] - A[:k, k:] - A[k:, :k] + A[k, k]
+
+
+@pytest.mark.parametrize("groups", [0, 2])
+def test_block_of_a_not_positive_definite_where_r_is(groups, oracle):
+    """260 hydrogens in a chain whose first three are 0.6695 A apart: A of the
+    first 64 variables has an eigenvalue of -1e-5, the reduced matrix's block is
+    positive definite and so is the whole, so that block takes no part in the
+    rank-one terms (resident and streaming solver).  With a lowest eigenvalue of 4e-5
+    and charges of 20 e the rounding of A alone moves charges, forces and the
+    residual past the parity bounds; the energy is stationary in the charges."""
+    n = 260
+    d = np.full(n - 1, 1.1)
+    d[:2] = 0.6695
+    xyz = np.zeros((n, 3))
+    xyz[1:, 0] = np.cumsum(d)
     m = GFNFFMethod()
+    m.setParameters({"pcg_groups": groups})
+    Z = np.ones(n, dtype=np.int32)
+    assert m.setMolecule(Mol(Z, xyz, bonds=[(i, i + 1) for i in range(n - 1)])), m.getErrorMessage()
+    A, R = eeq_matrices(m, xyz)
+    assert np.linalg.eigvalsh(A[:64, :64])[0] < -1e-6
+    assert np.linalg.eigvalsh(R)[0] > 1e-6 and np.linalg.eigvalsh(R[:64, :64])[0] > 1e-6
+    e = m.calculateEnergy(True)
+    assert not m.hasError(), m.getErrorMessage()
+    assert m.solverIterations() > 0
+    assert abs(e - oracle.eval(m.params_view(), xyz * (1.0 / BOHR))["E"]) < 1e-9 * n / 100
+
+
+@pytest.mark.parametrize("kind,size,groups,precision", [
+    ("alkane", 300, 2, "fp64"), ("alkane", 300, 5, "fp64"), ("alkane", 300, 20, "fp64"), ("alkane", 300, 0, "fp64"),
+    ("water", 256, 1, "fp64"), ("water", 256, 4, "fp64"), ("water", 256, 0, "fp64"), ("peptide", 70, 1, "mixed"),
+    ("peptide", 70, 4, "mixed")])
+def test_pcg_groups_do_not_change_the_solve(kind, size, groups, precision, oracle):
+    """Bounded workgroup counts: too few for one block per wavefront stream the
+    blocks, from eight per wavefront on through two buffers in turn (alkane 2,
+    water 1, peptide 1), below with the first one resident (alkane 5, water 4,
+    peptide 4); more keep every block resident.  901 variables in 120 blocks with
+    a split fragment, 512 and 492 in 36 without."""
+    Z, xyz = molecule(kind, size)
+    m = GFNFFMethod(precision=precision)
     m.setParameters({"pcg_groups": groups})
     assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
     m.calculateEnergy(True)
     assert not m.hasError(), m.getErrorMessage()
+    assert m.solverIterations() > 0
+    check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), precision)
+
+
+def test_too_few_pcg_groups_take_the_cholesky(oracle):
+    """15 row blocks on one workgroup are more than it can own."""
+    Z, xyz = molecule("alkane", 300)
+    m = GFNFFMethod()
+    m.setParameters({"pcg_groups": 1})
+    assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
+    m.calculateEnergy(True)
+    assert not m.hasError() and m.solverIterations() == 0
     check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), "fp64")
+
+
+@pytest.mark.parametrize("groups", [0, 2])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("order", ["long short long", "short long short"])
+def test_long_fragment_beside_short_ones(order, precision, groups, oracle):
+    """C60H122 chains (181 variables) and methanes (4): a 64-variable block that
+    holds the end of one split fragment, short fragments and the start of the
+    next, and one that starts with short fragments."""
+    parts, y = [], 0.0
+    for k in order.split():
+        for size in ([60] if k == "long" else [1, 1]):
+            z, x = alkane(size, sigma=0.02, seed=len(parts))
+            parts.append((z, x + [0.0, y, 0.0]))
+            y += 6.0
+    Z, xyz = np.concatenate([z for z, _ in parts]), np.vstack([x for _, x in parts])
+    m = GFNFFMethod(precision=precision)
+    m.setParameters({"pcg_groups": groups})
+    assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
+    assert m.params_view().nfrag == len(parts)
+    m.calculateEnergy(True)
+    assert not m.hasError(), m.getErrorMessage()
+    assert m.solverIterations() > 0
+    check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), precision)
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
