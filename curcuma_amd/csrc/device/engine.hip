@@ -8188,7 +8188,8 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
 // atoms 209 -> 135 us, 61 conformers 388 -> 333 us).  Larger systems keep the copies, whose
 // bandwidth counts there and whose staging belongs to the runtime.
 constexpr int HOST_PINNED_MAX = 131072;
-// results of one evaluation: [0, 16) energies, [16] flags, then gradient, charges, CN
+// results of one evaluation: [0, 16) energies, [16] flags, then charges, CN
+// and, unless grad is nullptr, the gradient
 __global__ __launch_bounds__(256) void k_host_out(int n, const double* __restrict__ out, const int* __restrict__ flags,
                                                   const double* __restrict__ grad, const double* __restrict__ q,
                                                   const double* __restrict__ cn, double* __restrict__ dst) {
@@ -8196,12 +8197,12 @@ __global__ __launch_bounds__(256) void k_host_out(int n, const double* __restric
     if (e < GFNFF_NTERMS + 1) dst[e] = out[e];
     if (e == GFNFF_NTERMS + 1) dst[e] = (double)flags[0];
     double* const r = dst + GFNFF_NTERMS + 2;
-    if (e < 3 * n)
-        r[e] = grad[e];
-    else if (e < 4 * n)
-        r[e] = q[e - 3 * n];
-    else if (e < 5 * n)
-        r[e] = cn[e - 4 * n];
+    if (e < n)
+        r[e] = q[e];
+    else if (e < 2 * n)
+        r[e] = cn[e - n];
+    else if (grad && e < 5 * n)
+        r[e] = grad[e - 2 * n];
 }
 
 int device_eval_host(DeviceEngine* E, const double* xyz_bohr, bool want_grad, double* e_terms, double* grad,
@@ -8220,16 +8221,17 @@ int device_eval_host(DeviceEngine* E, const double* xyz_bohr, bool want_grad, do
         std::memcpy(E->hpin, xyz_bohr, sizeof(double) * 3 * n);
         const int st = launch_eval(E, E->hpin, nullptr, nullptr, E->own, msg);
         if (st) return st;
-        hipLaunchKernelGGL(k_host_out, dim3(cdiv(std::max(5 * n, GFNFF_NTERMS + 2), 256)), dim3(256), 0, E->own, n,
-                           E->out, E->flags, E->grad, E->q, E->cn, o);
+        const double* const g = want_grad && grad ? E->grad : nullptr;
+        hipLaunchKernelGGL(k_host_out, dim3(cdiv(std::max((g ? 5 : 2) * n, GFNFF_NTERMS + 2), 256)), dim3(256), 0,
+                           E->own, n, E->out, E->flags, g, E->q, E->cn, o);
         HIP_OK(hipGetLastError());
         HIP_OK(hipStreamSynchronize(E->own));
         const double* const r = o + GFNFF_NTERMS + 2;
         std::memcpy(e_terms, o, sizeof(double) * (GFNFF_NTERMS + 1));
         flags = (int)o[GFNFF_NTERMS + 1];
-        if (want_grad && grad) std::memcpy(grad, r, sizeof(double) * 3 * n);
-        if (q) std::memcpy(q, r + 3 * (size_t)n, sizeof(double) * n);
-        if (cn) std::memcpy(cn, r + 4 * (size_t)n, sizeof(double) * n);
+        if (q) std::memcpy(q, r, sizeof(double) * n);
+        if (cn) std::memcpy(cn, r + n, sizeof(double) * n);
+        if (g) std::memcpy(grad, r + 2 * (size_t)n, sizeof(double) * 3 * n);
     } else {
         HIP_OK(hipMemcpyAsync(E->gpair, xyz_bohr, 3 * sizeof(double) * n, hipMemcpyHostToDevice, E->own));
         // gpair is overwritten by the pair reduction after the head of the evaluation has consumed it

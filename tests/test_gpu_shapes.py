@@ -137,7 +137,8 @@ def test_block_of_a_not_positive_definite_where_r_is(groups, oracle):
 
 
 @pytest.mark.parametrize("kind,size,groups,precision", [
-    ("alkane", 300, 2, "fp64"), ("alkane", 300, 5, "fp64"), ("alkane", 300, 20, "fp64"), ("alkane", 300, 0, "fp64"),
+    ("alkane", 300, 2, "fp64"), ("alkane", 300, 5, "fp64"), ("alkane", 300, 20, "fp64"), ("alkane", 300, 40, "fp64"),
+    ("alkane", 300, 0, "fp64"),
     ("water", 256, 1, "fp64"), ("water", 256, 4, "fp64"), ("water", 256, 0, "fp64"), ("peptide", 70, 1, "mixed"),
     ("peptide", 70, 4, "mixed")])
 def test_pcg_groups_do_not_change_the_solve(kind, size, groups, precision, oracle):
@@ -189,6 +190,23 @@ def test_long_fragment_beside_short_ones(order, precision, groups, oracle):
     assert not m.hasError(), m.getErrorMessage()
     assert m.solverIterations() > 0
     check(m, Z, xyz, oracle.eval(m.params_view(), xyz * (1.0 / BOHR)), precision)
+
+
+def test_energy_only_call_between_gradients():
+    """A call without the gradient leaves it out of the results' buffer: energy and
+    charges are those of a full call, before and after one."""
+    Z, xyz = molecule("peptide", 9)
+    m = GFNFFMethod()
+    assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
+    e0 = m.calculateEnergy(False)
+    q0, cn0 = m.getCharges(), m.getCN()
+    assert np.all(m.getGradient() == 0.0)
+    e1 = m.calculateEnergy(True)
+    g1 = m.getGradient()
+    assert m.calculateEnergy(False) == e0 == e1 and np.any(g1 != 0.0)
+    assert np.array_equal(m.getCharges(), q0) and np.array_equal(m.getCN(), cn0)
+    m.calculateEnergy(True)
+    assert np.array_equal(m.getGradient(), g1)
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
