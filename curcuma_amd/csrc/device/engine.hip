@@ -358,7 +358,9 @@ __device__ inline double rsqrt_nr2(double v) {
 // 2^-23) by one step of third order, which leaves e^3: with h = 1 - v y^2,
 // 1/sqrt(v) = y (1 + h / 2 + 3 h^2 / 8 + ..), and with h = 1 - v y,
 // 1/v = y (1 + h + h^2 + ..).  Five and three operations behind the estimate,
-// against about 14 of a division and 20 of a square root.
+// against about 14 of a division and 20 of a square root.  Within about one
+// unit in the last place; v has to be finite, normal and, with its reciprocal,
+// in range: 0 and infinity give NaN.
 __device__ inline double rsqrt_c(double v) {
     const double y = __builtin_amdgcn_rsq(v);
     const double h = fma(-v * y, y, 1.0);
@@ -1586,9 +1588,11 @@ __global__ __launch_bounds__(LU_T) void k_eeq_lu_fallback(int np, int nr, const 
 // the next one is loaded behind the publication of the barrier ahead of it,
 // which hides its latency; with more, two register buffers take the blocks in
 // turn.  water_3000 1324 -> 1259 us against eight wavefronts with one buffer
-// (mixed 1019 -> 970); in turn from two blocks on 1282 and 987.  80 chains of
-// C80H162 run at 0.34 ms an iteration either way: 1.49 GB of blocks and 0.09
-// GB of partials at 4.6 TB/s, where a device copy moves 5.2.
+// (mixed 1019 -> 970); in turn from two blocks on 1282 and 987.  The first form
+// takes 30 us an iteration on water_3000 (113 MB of blocks through the memory,
+// 120 MB read and 5 MB written with partials and vectors: 4.1 TB/s between two
+// barriers); 80 chains of C80H162 run at 0.34 ms either way: 1.49 GB of blocks
+// and 0.09 GB of partials at 4.6 TB/s, where a device copy moves 5.2.
 //
 // Preconditioner.  M = D, the diagonal blocks of R, cuts a fragment of more
 // than 64 variables into pieces, and every variable of the fragment carries
@@ -1602,8 +1606,8 @@ __global__ __launch_bounds__(LU_T) void k_eeq_lu_fallback(int np, int nr, const 
 // Owners publish y and their pieces' parts of s_f; after the barrier every
 // workgroup forms the same sigma_f s_f, and z on the fly.  Together with the
 // order of the variables along the bond graph (reduced_order): 80 chains of
-// C80H162 (mixed) 467 -> 76 iterations and 159 -> 27 ms, C300H602 148 -> 38,
-// H-(Gly)200-OH 97 -> 39, C40H82 39 -> 15.
+// C80H162 (mixed) 467 -> 76 to 80 iterations by the geometry and 159 -> 27 ms,
+// C300H602 148 -> 38, H-(Gly)200-OH 97 -> 39, C40H82 39 -> 15.
 constexpr int PCG_MAXB = 8;
 constexpr double PCG_TOL_FP64 = 1e-13;   // default |r| / |b| of the FP64 path
 constexpr double PCG_TOL_MIXED = 1e-10;  // default of the mixed path (EEQ energy is variational in q)
@@ -1994,7 +1998,9 @@ __global__ __launch_bounds__(PCGS_THREADS, 1) void k_eeq_pcg(PcgArgs a) {
 // reads before it polls for the one after, so no reader sees a word of four
 // iterations ago.  Measured, evaluation, against blocks resident behind full
 // barriers: 216 H2O 261 -> 240 us, H-(Gly)200-OH 726 -> 637, C300H602 650 ->
-// 590; two exchanges of about 4 us each bound an iteration.
+// 590; two exchanges of about 4 us each bound an iteration.  A block is half of
+// a lane's 256 registers; 17 others are spilled without split fragments (80
+// bytes of scratch per lane) and 36 with them (128 bytes).
 __device__ __forceinline__ double poll_c(const double* p, int& bad, const int* flags) {
     const unsigned long long* u = reinterpret_cast<const unsigned long long*>(p);
     unsigned long long v = ld_cu(u);
@@ -2230,9 +2236,9 @@ __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg_res(PcgArgs a) {
 
 // And with everything in one workgroup (np <= 64 NBK_ONE): the blocks in the
 // registers of one wavefront each, vectors and factors in LDS, a barrier of
-// the workgroup where the others cross the chip.  122 atoms: 15 iterations
-// 154 -> 30 us, evaluation 297 -> 169 us.  Three row blocks fill the registers
-// and LDS of a compute unit.
+// the workgroup where the others cross the chip.  122 atoms: evaluation 297 ->
+// 169 us; an iteration takes 4.3 us there (15: 64 us) and 5.7 with three row
+// blocks, which fill the registers and LDS of a compute unit.
 constexpr int NBK_ONE = 3;
 template <int NBK>
 __global__ __launch_bounds__(PCG_THREADS) void k_eeq_pcg_one(PcgArgs a) {
@@ -2876,9 +2882,11 @@ __device__ inline double ps_exp(double v) { return exp(v); }
 //
 // split: the 64 steps of a tile are dealt in equal runs to split wavefronts
 // (blocks t * split .. t * split + split - 1), each with partials of its own.
-// A step is a chain of erf, exp, square roots and divisions, about 1.5 us when
-// one wavefront has its SIMD to itself, so a launch of few tiles is bound by
-// that chain and not by throughput (ps_split).
+// A step is a chain of reciprocal square roots, the D4 contraction of every
+// element among the step's columns and, near by, erf and exp: about 1.1 us when
+// one wavefront has its SIMD to itself (122 atoms, both types: 80 us of 64 steps,
+// 18 of 8), so a launch of few tiles is bound by that chain and not by
+// throughput (ps_split).
 constexpr int PT_COUL = 1, PT_DISP = 2, PT_REP = 4, PT_ALL = 7;
 template <typename T, int NE>
 __global__ __launch_bounds__(PS_B) void k_pairs_sym(PairArgs a, double* __restrict__ part,
@@ -3180,9 +3188,10 @@ __device__ __forceinline__ double ordered_sum(F f) {
 // of a molecule (atoms a0 .. a0 + n - 1, its tiles numbered from base).
 // part2 (nullable): a second set of tile partials (the split pair terms),
 // added tile by tile after the first.
-// The atom's tail follows in the same launch, its neighbours dealt to the
-// four wavefronts (by one thread per atom in a launch of its own it took 15
-// us at any size: a chain of square roots and exponentials per neighbour).
+// The atom's tail follows in the same launch, its neighbours dealt to the W
+// wavefronts (by one thread per atom in a launch of its own it took 15 us at
+// any size: a chain of square roots and exponentials per neighbour).  W = 16
+// leaves a lane 128 registers, 12 of them spilled.
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_pairs_sym_reduce(int n, int nb, const double* __restrict__ part,
                                                           const double* __restrict__ part2,
@@ -3881,8 +3890,8 @@ __device__ __forceinline__ void xb_entry(int b, int nx, const int* __restrict__ 
 // differences in FP64 and evaluates the term in FP32 with hardware rsqrt,
 // rcp and exp.
 // The FP64 cores are bound by instruction issue: a divide or square-root
-// sequence is 10 to 15 of their FP64 instructions, the refined estimates
-// (about 1 ulp) are 4 and 5.
+// sequence is 14 and 20 of their FP64 instructions, the refined estimates
+// (about 1 ulp) 4 for the reciprocal and 8 for the square root.
 __device__ inline double hb_sqrt(double v) { return v * rsqrt_c(fmax(v, 1e-300)); }
 __device__ inline float hb_sqrt(float v) { return __builtin_sqrtf(v); }
 __device__ inline double hb_rcp(double v) { return rcp_c(v); }
@@ -4091,7 +4100,7 @@ __device__ double hb_core2(int A, int H, int B, const HBArgs& a, const double* _
 // Case-1 hydrogen bonds by role: the case-1 triplets are kept three times,
 // grouped by the atom in role A, H or B (entries: the other two atoms), each
 // group cut into chunks of at most HB_CHUNK triplets.  One wavefront per
-// chunk, one kernel per role, evaluates every triplet of its chunk (lanes
+// chunk evaluates every triplet of its chunk (lanes
 // stride the chunk; a triplet is evaluated once per role, which costs less
 // than storing and gathering per-triplet gradients), adds the gradient on its
 // own atom (and, for role A, the energy) with a fixed butterfly and writes
@@ -5316,8 +5325,8 @@ __device__ inline void d4_adj(double c6, double dci, double zc, double q, double
 }
 
 // Pair adjoint over full rows, the partners (all atoms, or the molecules of
-// the workgroup's rows) cut into gridDim.y chunks so that the launch has at
-// least 1024 workgroups (adj_chunks): 256 conformers, 33,700 atoms, 132 row
+// the workgroup's rows) cut into up to 16 chunks (gridDim.y, adj_chunks), until
+// the launch has 1024 workgroups: 256 conformers, 33,700 atoms, 132 row
 // blocks, ran 432 us in one chunk on half of the chip's compute units; one
 // fitting step with this and the reduction below 2.39 -> 1.65 ms.
 // Row i collects sum_j (w_i . r_hat_ij) dE'_ij/dln(theta) + u_i d(dEdcn_i)/dln(theta)
@@ -6500,7 +6509,7 @@ struct DeviceEngine {
     double* hpin = nullptr;  // pinned: coordinates and results of a host-buffer evaluation
     std::vector<void*> bufs;
     // parameters (device)
-    int *Z, *elem, *nref, *metal, *frag, *toff, *tidx, *tdist;
+    int *Z, *elem, *nref, *metal, *toff, *tidx, *tdist;
     double *chi_base, *gam, *alp, *cnf, *rcov_cn, *rcov_d3, *hb_rad, *hb_lpd, *qa, *zeta, *szr, *anb, *repz, *refcn, *c6ref;
     int *red_atom, *red_last, *red_of, *frag_off, *frag_atoms;
     int *red_lidx, *red_ul, *red_nul;  // distinct last atoms per 64-block of reduced variables
@@ -6719,7 +6728,6 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         E->elem = E->upload(P.elem);
         E->nref = E->upload(P.nref);
         E->metal = E->upload(P.metal);
-        E->frag = E->upload(P.frag);
         E->toff = E->upload(P.topo_off);
         E->tidx = E->upload(P.topo_idx);
         E->tdist = E->upload(P.topo_dist);
@@ -6750,7 +6758,8 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         // its RMS where charges reach 0.5 e (a peptide), by 4e-9 where they stay
         // below 0.1 e (hydrocarbons).  There the order and the preconditioner of
         // long fragments apply on both paths, for polar molecules on the FP64 path
-        // only, whose charges converge to rounding.
+        // only, whose charges converge to rounding: a long polar molecule keeps its
+        // results and its iterations on the mixed path (H-(Gly)200-OH 97, FP64 39).
         double qmax = 0.0;
         for (double v : P.qa) qmax = std::max(qmax, std::fabs(v));
         const bool long_frag = E->use_cg && (!E->mixed || qmax <= 0.1);
@@ -7261,8 +7270,9 @@ DeviceEngine* device_create(const ParamSet& P, int precision, const Options& opt
         // the gather of the slots (and a single molecule's hydrogen bonds): a
         // wavefront per atom also for short lists while that is at most four per
         // SIMD, where the lists' length and not their number sets the time
-        // (216 H2O: 18 us with 16 lanes per atom; dynamics with this and the
-        // wider pair reduction 256 -> 247 us per step)
+        // (evaluation with 16 lanes and with 64: 216 H2O 220.2 and 217.7 us, 512
+        // 289.5 and 283.5; 64 and 1000 to 3000 H2O, alkanes of 122 to 1802 atoms and
+        // batches of 828 to 20,777 the same within 0.4 %)
         E->slot_lpa = E->nmol == 1 && E->nhb ? std::max(E->fin_lpa, E->hbg_lpa) : E->fin_lpa;
         if (n <= 4096 && !opt.gather_lanes) E->slot_lpa = 64;
         E->slot_idx = E->upload(sidx);
@@ -7968,9 +7978,10 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
         }
         // cases 2-4: the case-2 entries by the lean core (FP32 terms on the
         // mixed path), those of cases 3 and 4 by the general FP64 one; a short
-        // FP64 list that holds both by the general core in one launch (38
-        // atoms, host buffers: 134 us against 143 with two; 61 conformers and 256
-        // molecules within their noise)
+        // FP64 list that holds both by the general core in one launch, which
+        // saves a launch of the chain (peptides of 38 atoms, 40 entries: 96 us
+        // against 99.7 with two; 143 atoms 208.7 against 211.0; 283 to 1403 atoms
+        // and batches of 56 to 57,000 entries the same within 0.3 %)
         const int n34 = E->nhb2 - E->nhb2_c2;
         constexpr int HB_ONE_MAX = 16384;
         const bool one = !E->mixed && n34 > 0 && E->nhb2 <= HB_ONE_MAX;
@@ -8184,9 +8195,12 @@ static int launch_eval(DeviceEngine* E, const double* xin, double* energy_out, d
 // memory that the device reads and writes itself: the head of the evaluation
 // reads the coordinates there and one launch at its end writes every result,
 // side by side, so that a call is one queue of launches and one wait.  By
-// pageable copies it was five transfers with a wait in the runtime each (38
-// atoms 209 -> 135 us, 61 conformers 388 -> 333 us).  Larger systems keep the copies, whose
-// bandwidth counts there and whose staging belongs to the runtime.
+// pageable copies it was five transfers with a wait in the runtime each.  By
+// copies and by pinned memory: 38 atoms 209 and 135 us, 648 345 and 256, 3,000
+// 589 and 430, batches of 3,415 877 and 751 us, 53,797 1.44 and 1.38 ms, 124,193
+// 2.22 and 2.19, 204,392 3.15 and 3.07, 409,164 5.70 and 5.73, 819,770 11.2 and
+// 11.5 ms.  Larger systems keep the copies, whose bandwidth counts there and
+// whose staging belongs to the runtime.
 constexpr int HOST_PINNED_MAX = 131072;
 // results of one evaluation: [0, 16) energies, [16] flags, then charges, CN
 // and, unless grad is nullptr, the gradient

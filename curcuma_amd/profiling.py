@@ -134,7 +134,8 @@ def work_per_eval(cls: str, info: dict, rc: dict) -> tuple[float, str]:
     if cls == "trsv":
         npd = info["np_pad"]
         return 2.0 * 8.0 * npd * npd / 2, "byte"  # the factor is read once per sweep
-    if cls == "pcg":  # the packed symmetric FP64 matrix (64x64 lower blocks) is streamed once per CG iteration
+    if cls == "pcg":  # the packed symmetric FP64 matrix (64x64 lower blocks) once per CG iteration, also where
+        # some of it stays in registers (the counters' traffic is what moves)
         nbk = info["np_pad"] // NB
         return info.get("pcg_iters", 0) * 8.0 * (nbk * (nbk + 1) // 2) * NB * NB, "byte"
     if cls == "eeq_build":

@@ -186,9 +186,12 @@ int gfnff_cn(gfnff_handle* h, double* cn);
  * solve, the default); "batch_pairs" 0 = pair terms of batches with each
  * pair once in 64 x 64 tiles per molecule (default), 1 = one thread per row
  * atom over its molecule; "gather_lanes" 0 (by mean list length), 16 or 64
- * lanes per atom in the slot and hydrogen-bond gathers; "pcg_groups" 0 (all
- * workgroups that fit, at most 256) or an upper bound on the persistent
- * PCG's workgroups. */
+ * lanes per atom in the slot and hydrogen-bond gathers; "pcg_groups" 0 (as many
+ * workgroups of the iterative solve as give every wavefront at most one matrix
+ * block and every 64-variable row block two workgroups, at most those that fit
+ * and at most 256; up to 192 variables one workgroup whatever the key says) or
+ * an upper bound: a lower count may stream the blocks instead of keeping them
+ * on chip, and one below an eighth of the row blocks means the Cholesky solve. */
 int gfnff_set_param(gfnff_handle* h, const char* key, double value);
 
 /* GFNFF_PREC_FP64 (default, the reference's arithmetic) or GFNFF_PREC_MIXED:
