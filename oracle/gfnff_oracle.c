@@ -1,6 +1,6 @@
 /*
  * gfnff_oracle.c -- CPU FP64 restatement of the reference's GFN-FF
- * per-evaluation path.  TEST INFRASTRUCTURE ONLY: it is the checker that the
+ * per-evaluation path.  TEST INFRASTRUCTURE ONLY: it is what the
  * HIP engine is compared against (tests/, __graft_entry__.smoke() and the
  * bench.py cpu_baseline leg).  Nothing in the shipped engine links or calls it.
  *

@@ -5,7 +5,7 @@ energies.  FP64 kernels on both precision paths.
 Bars: energy and every term |dE| <= 1e-9 Eh, charges 1e-9 e, gradient
 components 1e-9 Eh/Bohr against the oracle (FP64 path); the xtb fixture's
 own 1e-7 Eh.  The mixed path's pair terms are FP32, so its bar is the
-north star's (1e-6 Eh/atom, gradient RMS 1e-5 Eh/Bohr)."""
+mixed path's own (1e-6 Eh/atom, gradient RMS 1e-5 Eh/Bohr)."""
 import json
 
 import numpy as np

@@ -3,7 +3,7 @@ same Bohr coordinates).  Every call goes through the C-ABI.
 
 Tolerances: energies are FP64 on both sides and agree to rounding; the bar
 asserted is |dE| <= 1e-9 Eh absolute or 1e-12 relative per term, charges
-1e-9 e, gradient components 1e-9 Eh/Bohr (the north-star bar for the FP64
+1e-9 e, gradient components 1e-9 Eh/Bohr (the parity bar for the FP64
 path is |dE| <= 1e-6 Eh/atom and gradient RMS <= 1e-5 Eh/Bohr).
 """
 import numpy as np
