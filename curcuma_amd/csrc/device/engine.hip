@@ -5535,11 +5535,15 @@ __global__ __launch_bounds__(256) void k_adj_brep(int nb, const int* __restrict_
     }
 }
 
-// Fixed-order reduction of the adjoint partials in two launches: workgroup
-// (k, b) adds share b of the rows of output component k (by one wavefront per
-// component it took 390 us for 33,700 atoms), then one wavefront per
-// component adds the shares.
+// Fixed-order reduction of the adjoint partials: workgroup (k, b) adds share b
+// of the rows of output component k (by one wavefront per component it took
+// 390 us for 33,700 atoms), then one wavefront per component adds the shares.
+// Up to ADJ_ONE_MAX rows of all chunks one share is the sum, which saves the
+// second launch and the idle workgroups of the first (whole call, one and 64
+// shares: 6 atoms 46 and 73 us, 195 atoms 95 and 116, 900 atoms, 15,000 rows,
+// 137 and 144, 1500 atoms, 26,500 rows, 174 and 173).
 constexpr int ADJ_RB = 64;
+constexpr int ADJ_ONE_MAX = 16384;
 __global__ __launch_bounds__(256) void k_adj_reduce(int n, int nchunk, const double* __restrict__ part, int nb,
                                                     const double* __restrict__ bpart, int nk,
                                                     double* __restrict__ share) {
@@ -5547,10 +5551,10 @@ __global__ __launch_bounds__(256) void k_adj_reduce(int n, int nchunk, const dou
     const int k = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     double acc = 0.0;
     for (int c = 0; c < nchunk; ++c)
-        for (int i = b * 256 + tid; i < n; i += ADJ_RB * 256) acc += part[((size_t)c * nk + k) * n + i];
-    for (int i = b * 256 + tid; i < nb; i += ADJ_RB * 256) acc += bpart[(size_t)k * nb + i];
+        for (int i = b * 256 + tid; i < n; i += gridDim.y * 256) acc += part[((size_t)c * nk + k) * n + i];
+    for (int i = b * 256 + tid; i < nb; i += gridDim.y * 256) acc += bpart[(size_t)k * nb + i];
     acc = wg_sum256(acc, red);
-    if (tid == 0) share[k * ADJ_RB + b] = acc;
+    if (tid == 0) share[k * gridDim.y + b] = acc;
 }
 __global__ __launch_bounds__(64) void k_adj_final(const double* __restrict__ share, double* __restrict__ out) {
     const double v = wave_sum(share[blockIdx.x * ADJ_RB + threadIdx.x]);
@@ -8463,9 +8467,10 @@ static void queue_adjoint(DeviceEngine* E, hipStream_t s, const PairArgs& pa, do
     if (E->nbrep)
         hipLaunchKernelGGL(k_adj_brep<NE>, dim3(cdiv(E->nbrep, 256)), dim3(256), 0, s, E->nbrep, E->brep_ij,
                            E->brep_par, E->elem, E->x, E->adj_w, bpart);
-    hipLaunchKernelGGL(k_adj_reduce, dim3(ADJ_P * NE, ADJ_RB), dim3(256), 0, s, n, nc + 1, part, E->nbrep, bpart,
-                       ADJ_P * NE, E->adj_share);
-    hipLaunchKernelGGL(k_adj_final, dim3(ADJ_P * NE), dim3(64), 0, s, E->adj_share, E->adj_out);
+    const bool one = (long)(nc + 1) * n + E->nbrep <= ADJ_ONE_MAX;
+    hipLaunchKernelGGL(k_adj_reduce, dim3(ADJ_P * NE, one ? 1 : ADJ_RB), dim3(256), 0, s, n, nc + 1, part, E->nbrep,
+                       bpart, ADJ_P * NE, one ? E->adj_out : E->adj_share);
+    if (!one) hipLaunchKernelGGL(k_adj_final, dim3(ADJ_P * NE), dim3(64), 0, s, E->adj_share, E->adj_out);
 }
 
 // dLoss/dln(theta) = sum_i w_i . dg_i/dln(theta) at the state of the last

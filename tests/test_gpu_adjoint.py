@@ -25,10 +25,11 @@ def grad_at(m, theta):
     return m.getGradient().copy()
 
 
-@pytest.mark.parametrize("case", ["alkane30", "water27", "complex"])
+@pytest.mark.parametrize("case", ["alkane30", "water27", "complex", "water1", "water300", "water330"])
 def test_adjoint_matches_finite_differences(case):
     """complex (H, C, N, O; 231 atoms) holds case-4 hydrogen bonds, whose
-    lone-pair distance must not follow the fitted repz scales."""
+    lone-pair distance must not follow the fitted repz scales; water 1, 300 and
+    330 lie at the small end and on both sides of the one-launch reduction."""
     if case == "alkane30":
         Z, xyz = alkane(30, sigma=0.05, seed=5)
     elif case == "complex":
@@ -36,7 +37,7 @@ def test_adjoint_matches_finite_differences(case):
         fx = load_fixture("complex")
         Z, xyz = np.array(fx["Z"]), np.array(fx["xyz_bohr"]) * BOHR
     else:
-        Z, xyz = water_cluster(27, seed=7)
+        Z, xyz = water_cluster(int(case[5:]), seed=7)
     m = GFNFFMethod()
     assert m.setMolecule(Mol(Z, xyz)), m.getErrorMessage()
     npar = m.paramCount()
