@@ -5395,7 +5395,7 @@ __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __
             const double r2 = dx * dx + dy * dy + dz * dz;
             if (r2 > 2500.0) continue;  // beyond the D4 and repulsion cut-offs
             const double rinv = rsqrt_c(r2), r = r2 * rinv;
-            if (!(r2 >= 1e-20)) continue;
+            if (!(r >= 1e-10)) continue;
             const double sw = (wi.x * dx + wi.y * dy + wi.z * dz) * rinv;
             const int ej = sel[jj];
             double dd4 = 0.0, dz_ = 0.0, da_ = 0.0;
@@ -5416,7 +5416,7 @@ __global__ __launch_bounds__(TILE) void k_adj_pairs(PairArgs a, const double* __
                 d4_adj(c6, dci, zti * szt[jj], q, r2, r, dEp_dq, ddcn_dq);
                 dd4 = (sw * dEp_dq + ui * ddcn_dq) * q;  // d / d ln(theta) of one factor of q
             }
-            if (r2 <= 400.0 && r2 >= 1e-16) {   // non-bonded repulsion, generic pair factor
+            if (r2 <= 400.0 && r >= 1e-8) {   // non-bonded repulsion, generic pair factor
                 const double ff = rep_ff(zi, sZ[jj], mi, smt[jj]);
                 const double al = sqrt(ani * san[jj]) * ff;
                 const double ab = rzi * srz[jj] * 0.4270;
@@ -5540,10 +5540,11 @@ __global__ __launch_bounds__(256) void k_adj_brep(int nb, const int* __restrict_
 // 390 us for 33,700 atoms), then one wavefront per component adds the shares.
 // Up to ADJ_ONE_MAX rows of all chunks one share is the sum, which saves the
 // second launch and the idle workgroups of the first (whole call, one and 64
-// shares: 6 atoms 46 and 73 us, 195 atoms 95 and 116, 900 atoms, 15,000 rows,
-// 137 and 144, 1500 atoms, 26,500 rows, 174 and 173).
+// shares: 6 atoms 46 and 73 us, 195 atoms 90 and 111, 900 atoms, 15,000 rows,
+// 131 and 138; 1500 atoms, 26,500 rows, the same).
 constexpr int ADJ_RB = 64;
 constexpr int ADJ_ONE_MAX = 16384;
+template <int RB>  // shares, 1 or ADJ_RB
 __global__ __launch_bounds__(256) void k_adj_reduce(int n, int nchunk, const double* __restrict__ part, int nb,
                                                     const double* __restrict__ bpart, int nk,
                                                     double* __restrict__ share) {
@@ -5551,10 +5552,10 @@ __global__ __launch_bounds__(256) void k_adj_reduce(int n, int nchunk, const dou
     const int k = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     double acc = 0.0;
     for (int c = 0; c < nchunk; ++c)
-        for (int i = b * 256 + tid; i < n; i += gridDim.y * 256) acc += part[((size_t)c * nk + k) * n + i];
-    for (int i = b * 256 + tid; i < nb; i += gridDim.y * 256) acc += bpart[(size_t)k * nb + i];
+        for (int i = b * 256 + tid; i < n; i += RB * 256) acc += part[((size_t)c * nk + k) * n + i];
+    for (int i = b * 256 + tid; i < nb; i += RB * 256) acc += bpart[(size_t)k * nb + i];
     acc = wg_sum256(acc, red);
-    if (tid == 0) share[k * gridDim.y + b] = acc;
+    if (tid == 0) share[k * RB + b] = acc;
 }
 __global__ __launch_bounds__(64) void k_adj_final(const double* __restrict__ share, double* __restrict__ out) {
     const double v = wave_sum(share[blockIdx.x * ADJ_RB + threadIdx.x]);
@@ -8467,10 +8468,14 @@ static void queue_adjoint(DeviceEngine* E, hipStream_t s, const PairArgs& pa, do
     if (E->nbrep)
         hipLaunchKernelGGL(k_adj_brep<NE>, dim3(cdiv(E->nbrep, 256)), dim3(256), 0, s, E->nbrep, E->brep_ij,
                            E->brep_par, E->elem, E->x, E->adj_w, bpart);
-    const bool one = (long)(nc + 1) * n + E->nbrep <= ADJ_ONE_MAX;
-    hipLaunchKernelGGL(k_adj_reduce, dim3(ADJ_P * NE, one ? 1 : ADJ_RB), dim3(256), 0, s, n, nc + 1, part, E->nbrep,
-                       bpart, ADJ_P * NE, one ? E->adj_out : E->adj_share);
-    if (!one) hipLaunchKernelGGL(k_adj_final, dim3(ADJ_P * NE), dim3(64), 0, s, E->adj_share, E->adj_out);
+    if ((long)(nc + 1) * n + E->nbrep <= ADJ_ONE_MAX) {
+        hipLaunchKernelGGL(k_adj_reduce<1>, dim3(ADJ_P * NE), dim3(256), 0, s, n, nc + 1, part, E->nbrep, bpart,
+                           ADJ_P * NE, E->adj_out);
+        return;
+    }
+    hipLaunchKernelGGL(k_adj_reduce<ADJ_RB>, dim3(ADJ_P * NE, ADJ_RB), dim3(256), 0, s, n, nc + 1, part, E->nbrep,
+                       bpart, ADJ_P * NE, E->adj_share);
+    hipLaunchKernelGGL(k_adj_final, dim3(ADJ_P * NE), dim3(64), 0, s, E->adj_share, E->adj_out);
 }
 
 // dLoss/dln(theta) = sum_i w_i . dg_i/dln(theta) at the state of the last
